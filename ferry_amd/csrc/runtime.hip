@@ -1213,12 +1213,33 @@ struct SelArgs {
   uint32_t* sel;
   int l0, nl, max_n;
   int* err;
+  int cus;
 };
+
+// Wavefronts of a Quest selection workgroup (one row each).  A launch of no
+// more rows than CUs has one workgroup per CU whatever its size, so a row's
+// records are scored by 16 wavefronts: four leave 8 KiB in flight per CU and
+// the row's arithmetic on one wavefront per SIMD.  Up to two rows per CU, 8;
+// more rows fill the CUs with workgroups of 4, whose top-k phases overlap the
+// others' loads better.  bf16, 4 query heads per kv head, 8192 blocks, us per
+// launch with 4 / 8 / 16 wavefronts: 128 rows 293 / 169 / 131, 256 rows
+// 321 / 201 / 176, 512 rows 379 / 344 / 345, 1024 rows 668 / 667 / 674; 512
+// blocks: 256 rows 24 / 18 / 17, 512 rows 30 / 27 / 34, 1024 rows 47 / 50 / 65.
+int select_waves(unsigned rows, int cus) {
+  return rows <= (unsigned)cus ? 16 : rows <= 2u * (unsigned)cus ? 8 : 4;
+}
 
 template <int DT, int G, bool LAYER>
 void launch_sel(const dim3& grid, size_t lds, hipStream_t s, const SelArgs& a) {
-  hipLaunchKernelGGL((k_select_topk<DT, G, LAYER, 4>), grid, dim3(256), lds, s, a.g, a.q, a.ctx_blocks,
-                     a.sums, a.sum_scales, a.sum_mod, a.sel, a.l0, a.nl, a.max_n, a.err);
+#define FERRY_SEL_LAUNCH(W)                                                                         \
+  hipLaunchKernelGGL((k_select_topk<DT, G, LAYER, W>), grid, dim3(64 * W), lds, s, a.g, a.q,         \
+                     a.ctx_blocks, a.sums, a.sum_scales, a.sum_mod, a.sel, a.l0, a.nl, a.max_n, a.err)
+  switch (select_waves(grid.x, a.cus)) {
+    case 16: FERRY_SEL_LAUNCH(16); return;
+    case 8: FERRY_SEL_LAUNCH(8); return;
+    default: FERRY_SEL_LAUNCH(4); return;
+  }
+#undef FERRY_SEL_LAUNCH
 }
 template <int DT, bool LAYER>
 void launch_sel_g(int G, const dim3& grid, size_t lds, hipStream_t s, const SelArgs& a) {
@@ -1265,7 +1286,8 @@ int ferry_select_topk_layers(ferry_ctx* ctx, int32_t l0, int32_t nl, const float
   HIPC(hipSetDevice(ctx->device));
   const dim3 grid((unsigned)((size_t)g.n_req * nl * (layer ? 1 : g.Hkv)));
   const SelArgs a{g,   q,   ctx_blocks,    ctx->sums, ctx->sum_scales, ctx->sum_blocks,
-                  sel, l0,  nl,            g.max_blocks, ctx->err};
+                  sel, l0,  nl,            g.max_blocks, ctx->err,
+                  ctx->cus};
   if (layer)
     launch_sel_dt<true>(g.dtype, G, grid, lds, (hipStream_t)stream, a);
   else

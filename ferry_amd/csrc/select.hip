@@ -1014,10 +1014,14 @@ FERRY_SUMS_INST(FERRY_F16)
 FERRY_SUMS_INST(FERRY_BF16)
 FERRY_SUMS_INST(FERRY_FP8_E4M3)
 
-#define FERRY_SEL_INST(DT, G, LAYER)                                                           \
-  template __global__ void k_select_topk<DT, G, LAYER, 4>(Geo, const float*, const int32_t*,     \
+#define FERRY_SEL_INST_W(DT, G, LAYER, W)                                                      \
+  template __global__ void k_select_topk<DT, G, LAYER, W>(Geo, const float*, const int32_t*,     \
                                                           const uint8_t*, const float*, uint64_t,  \
                                                           uint32_t*, int, int, int, int*);
+#define FERRY_SEL_INST(DT, G, LAYER) \
+  FERRY_SEL_INST_W(DT, G, LAYER, 4)  \
+  FERRY_SEL_INST_W(DT, G, LAYER, 8)  \
+  FERRY_SEL_INST_W(DT, G, LAYER, 16)
 #define FERRY_SEL_INST_G(DT, LAYER) \
   FERRY_SEL_INST(DT, 1, LAYER)      \
   FERRY_SEL_INST(DT, 2, LAYER)      \

@@ -67,6 +67,33 @@ def test_select_topk_bit_exact(dtype, Hkv, Hq, host_blocks, mode):
     assert p.ex.stats()["device_error"] == 0
 
 
+@pytest.mark.parametrize("dtype,Hkv,Hq,mode,n_req", [
+    (F.BF16, 2, 8, F.TOPK_PER_HEAD, 100),
+    (F.FP8, 2, 16, F.TOPK_PER_HEAD, 100),
+    (F.F32, 2, 2, F.TOPK_PER_HEAD, 100),
+    (F.F16, 2, 4, F.TOPK_LAYER_MAX, 200),
+])
+def test_select_workgroup_sizes_bit_exact(dtype, Hkv, Hq, mode, n_req):
+    """A workgroup has 16, 8 or 4 wavefronts by the rows of the launch (up to
+    256, 512, more on 256 CUs): 200, 400 and 600 rows of one context set, with
+    context lengths around a wavefront's and a workgroup's span of blocks."""
+    L, k, mb = 3, 12, 270
+    p = Pair(n_req, L, Hkv, Hq, k, 16, mb, dtype, host_blocks=1031)
+    p.ex.summaries_build()
+    rng = np.random.default_rng(dtype + 3)
+    ctx = rng.choice([0, 12, 13, 15, 16, 17, 63, 64, 65, 255, 256, 257, 270], n_req).astype(np.int32)
+    q = rng.standard_normal((n_req, L, Hq, 128)).astype(np.float32)
+    dq, dctx = torch.from_numpy(q).cuda(), torch.from_numpy(ctx).cuda()
+    want = O.select_topk(p.g, q, ctx, mode)
+    for step in (1, 2, 3):  # layers per launch
+        sel = torch.full((n_req, L, Hkv, k), -7, dtype=torch.int32, device="cuda")
+        for l0 in range(0, L, step):
+            p.ex.select_topk(dq, dctx, sel, mode, layers=(l0, min(step, L - l0)))
+        torch.cuda.synchronize()
+        assert np.array_equal(sel.cpu().numpy().view(np.uint32), want), step
+    assert p.ex.stats()["device_error"] == 0
+
+
 def test_one_record_per_block_gives_the_same_selection():
     """A table with a record per (set, block) (3x the host tier here) repeats
     the host-tier records and selects exactly what the small table does."""
