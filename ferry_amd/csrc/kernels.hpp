@@ -240,11 +240,14 @@ __global__ void k_select_mass(Geo g, const float* q, const int32_t* ctx_blocks, 
 template <int DT, int G, int W, int U>
 __global__ void k_mass_units(Geo g, const float* q, const int32_t* ctx_blocks, const uint8_t* kt,
                              const float* kt_scales, uint64_t kt_mod, float* ws, float* mass,
-                             unsigned* counter, int l0, int nl, int max_n, int* err);
+                             unsigned* counter, int parts, int l0, int nl, int max_n, int* err);
 __global__ void k_mass_reset(unsigned* counter);
+template <int G>
+__global__ void k_mass_finish(Geo g, const int32_t* ctx_blocks, const float* lsum, const float* part_ms,
+                              int parts, float* score, int nl, int max_n);
 template <int W>
-__global__ void k_mass_topk(Geo g, const int32_t* ctx_blocks, const float* mass, uint32_t* sel, int l0,
-                            int nl, int max_n);
+__global__ void k_mass_topk(Geo g, const int32_t* ctx_blocks, const float* mass, int rows, uint32_t* sel,
+                            int l0, int nl, int max_n);
 // persistent workgroups of k_select_mass (fp32 K); each holds max_blocks * G * 2
 // floats of workspace
 constexpr int kMassWgs = 2048;
@@ -259,6 +262,7 @@ constexpr int kMassUnitWaves = 8;
 constexpr int kMassUnitInflight = 3;
 constexpr int kMassUnitWgs = 2048;
 constexpr int kMassTopkWaves = 4;
+constexpr int kMassTopkWideWaves = 16;
 
 // queue.hip: the ceiling of the ring's tickets (one shared 64-bit word)
 __global__ void k_ticket_probe(unsigned long long* word, int iters, int kind, int* failed);

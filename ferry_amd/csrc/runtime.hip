@@ -131,6 +131,7 @@ struct ferry_ctx {
   int attn_waves = 0;              // wavefronts per attention workgroup (FERRY_ATTN_WAVES), 0 = default
   int cus = 256;                   // compute units of the device
   int mass_resident = 0;           // k_mass_units workgroups resident at once (0: not yet asked)
+  int mass_split_slots = 0;        // ... with a unit's blocks split between workgroups (0: not yet asked)
   int mass_lds = -1;               // k_mass_units keeps block log-sums in LDS (-1: not yet decided)
   int group_waves_env = 0;         // prefix-group kernel wavefronts (FERRY_GROUP_WAVES=4|8), 0 = by launch
   int fetch_waves = 0;             // wavefronts per fetch workgroup (FERRY_FETCH_WAVES: 1, 2, 4; 0 = by rule)
@@ -1337,24 +1338,26 @@ uint64_t mass_slice_bytes(ferry_ctx* ctx) {
   return (uint64_t)g.max_blocks * (uint64_t)(g.Hq / g.Hkv) * 2 * sizeof(float);
 }
 
-// Workgroups of k_mass_units the device holds at once (occupancy x CUs),
-// computed once per context.
-int mass_units_resident(ferry_ctx* ctx) {
-  if (ctx->mass_resident > 0) return ctx->mass_resident;
+// The k_mass_units instance of the context's type and head group.
+const void* mass_units_fn(const ferry_ctx* ctx) {
   const Geo& g = ctx->g;
   const int G = g.Hq / g.Hkv;
-  const void* fn = nullptr;
-#define FERRY_MASS_FN(DT)                                                                           \
-  fn = G == 1   ? reinterpret_cast<const void*>(&k_mass_units<DT, 1, kMassUnitWaves, kMassUnitInflight>) \
-       : G == 2 ? reinterpret_cast<const void*>(&k_mass_units<DT, 2, kMassUnitWaves, kMassUnitInflight>) \
-       : G == 4 ? reinterpret_cast<const void*>(&k_mass_units<DT, 4, kMassUnitWaves, kMassUnitInflight>) \
-                : reinterpret_cast<const void*>(&k_mass_units<DT, 8, kMassUnitWaves, kMassUnitInflight>)
-  if (g.dtype == FERRY_F16) FERRY_MASS_FN(FERRY_F16);
-  else if (g.dtype == FERRY_BF16) FERRY_MASS_FN(FERRY_BF16);
-  else FERRY_MASS_FN(FERRY_FP8_E4M3);
+#define FERRY_MASS_FN(DT)                                                                              \
+  (G == 1   ? reinterpret_cast<const void*>(&k_mass_units<DT, 1, kMassUnitWaves, kMassUnitInflight>) \
+   : G == 2 ? reinterpret_cast<const void*>(&k_mass_units<DT, 2, kMassUnitWaves, kMassUnitInflight>) \
+   : G == 4 ? reinterpret_cast<const void*>(&k_mass_units<DT, 4, kMassUnitWaves, kMassUnitInflight>) \
+            : reinterpret_cast<const void*>(&k_mass_units<DT, 8, kMassUnitWaves, kMassUnitInflight>))
+  return g.dtype == FERRY_F16    ? FERRY_MASS_FN(FERRY_F16)
+         : g.dtype == FERRY_BF16 ? FERRY_MASS_FN(FERRY_BF16)
+                                 : FERRY_MASS_FN(FERRY_FP8_E4M3);
 #undef FERRY_MASS_FN
+}
+
+// Workgroups of k_mass_units the device holds at once with `lds` bytes each
+// (occupancy x CUs).
+int mass_resident_wgs(ferry_ctx* ctx, size_t lds) {
+  const void* fn = mass_units_fn(ctx);
   int per_cu = 0;
-  const size_t lds = mass_lds_bytes(ctx);
   const bool on_dev = hipSetDevice(ctx->device) == hipSuccess;
   if (on_dev && lds > 65536)
     (void)hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMassLdsWs);
@@ -1363,8 +1366,17 @@ int mass_units_resident(ferry_ctx* ctx) {
     (void)hipGetLastError();
     per_cu = 1;  // still correct: the workgroups take the units from the counter
   }
-  ctx->mass_resident = per_cu * ctx->cus;
+  return per_cu * ctx->cus;
+}
+// Computed once per context: a unit per workgroup pass, and split units, whose
+// log-sums go to HBM (no dynamic LDS).
+int mass_units_resident(ferry_ctx* ctx) {
+  if (ctx->mass_resident <= 0) ctx->mass_resident = mass_resident_wgs(ctx, mass_lds_bytes(ctx));
   return ctx->mass_resident;
+}
+int mass_split_resident(ferry_ctx* ctx) {
+  if (ctx->mass_split_slots <= 0) ctx->mass_split_slots = mass_resident_wgs(ctx, 0);
+  return ctx->mass_split_slots;
 }
 
 // Workgroups of a mass selection over nl layers, at most cap: (request,
@@ -1394,6 +1406,55 @@ uint64_t mass_ws_bytes(ferry_ctx* ctx, int nl, uint64_t wgs) {
   return mass_mass_offset(ctx, wgs) + (uint64_t)g.n_req * nl * g.Hkv * g.max_blocks * sizeof(float);
 }
 
+// Workgroups that share one unit's blocks in a 16-bit or fp8 mass selection
+// over nl layers: 1 (a unit per workgroup pass) where two units or more share
+// a workgroup slot (the workgroups the GPU holds at once: one per CU for bf16,
+// two for fp8).  Fewer units leave slots idle and every unit's records to one
+// workgroup's loads in flight, so each unit is split: about two parts per slot
+// while a part has 256 blocks (the second hides the first's start), at least
+// one part per slot while a part has 32.  us per one-layer launch, 8192 / 512
+// blocks: bf16 128 units whole 859 / 75, split in 4 696 / 61, in 2 719 / 57;
+// 32 units whole 788 / 67, in 8 190 / 26; 8 units whole 778 / 65, in 16
+// 75 / 21; 256 units whole 1314 / 100, in 2 1408 / 99; fp8 128 units whole
+// 805 / 70, in 8 427 / 55, in 4 430 / 46.
+int mass_parts(ferry_ctx* ctx, int nl) {
+  const Geo& g = ctx->g;
+  const uint64_t units = (uint64_t)g.n_req * nl * g.Hkv, mb = (uint64_t)g.max_blocks;
+  if (g.dtype == FERRY_F32) return 1;
+  const uint64_t slots = (uint64_t)mass_split_resident(ctx);
+  if (2 * units > slots) return 1;
+  const uint64_t large = std::min((2 * slots + units - 1) / units, mb / 256);
+  return (int)std::max<uint64_t>(1, std::max(large, std::min(slots / units, mb / 32)));
+}
+
+// Workspace of such a launch: the log-sums (a float per block and query head
+// of every unit), the parts' (max, sum) and a score per block of every item,
+// each 256-byte aligned.
+struct MassSplit {
+  uint64_t ms, score, bytes;  // offsets in bytes; the log-sums are at 0
+};
+MassSplit mass_split_layout(ferry_ctx* ctx, int nl, int parts) {
+  const Geo& g = ctx->g;
+  const uint64_t units = (uint64_t)g.n_req * nl * g.Hkv, G = (uint64_t)(g.Hq / g.Hkv);
+  auto up = [](uint64_t b) { return (b + 255) / 256 * 256; };
+  MassSplit m;
+  m.ms = up(units * g.max_blocks * G * sizeof(float));
+  m.score = m.ms + up(units * parts * G * 2 * sizeof(float));
+  m.bytes = m.score + (uint64_t)g.n_req * nl * g.max_blocks * sizeof(float);
+  return m;
+}
+
+// The context's workspace: what any layer range of a mass selection needs.
+uint64_t mass_ctx_bytes(ferry_ctx* ctx) {
+  const Geo& g = ctx->g;
+  uint64_t need = mass_ws_bytes(ctx, g.L, mass_wgs(ctx, g.L, ~0ull));
+  for (int nl = 1; nl <= g.L; ++nl) {
+    const int parts = mass_parts(ctx, nl);
+    if (parts > 1) need = std::max(need, mass_split_layout(ctx, nl, parts).bytes);
+  }
+  return need;
+}
+
 }  // namespace
 
 extern "C" {
@@ -1420,7 +1481,7 @@ int ferry_ktiles_build(ferry_ctx* ctx, uint64_t n_records, void* stream) {
     ctx->kt_records = S;
   }
   if (!ctx->mass_ws && (uint64_t)g.max_blocks * 4 <= kMassLds)
-    HIPC(hipMalloc(&ctx->mass_ws, mass_ws_bytes(ctx, g.L, mass_wgs(ctx, g.L, ~0ull))));
+    HIPC(hipMalloc(&ctx->mass_ws, mass_ctx_bytes(ctx)));
   ctx->kt_perm = g.dtype != FERRY_F32;
   const unsigned blocks = (unsigned)std::min<uint64_t>((g.host_blocks + 3) / 4, 16384);
   switch (KT / 1024) {
@@ -1454,10 +1515,11 @@ int ferry_ktiles_view(ferry_ctx* ctx, void** ktiles, float** scales, uint64_t* n
 namespace {
 
 // The mass selection of layers [l0, l0 + nl) with `wgs` workgroups
-// (mass_wgs) and workspace `ws` of mass_ws_bytes(ctx, nl, wgs).
+// (mass_wgs) and workspace `ws` of mass_ws_bytes(ctx, nl, wgs); a launch of few
+// units is split (mass_parts) where `ws`, of ws_bytes, holds what that takes.
 int launch_select_mass(ferry_ctx* ctx, int32_t l0, int32_t nl, const float* q,
                        const int32_t* ctx_blocks, uint32_t* sel, void* stream, float* ws,
-                       uint64_t wgs) {
+                       uint64_t wgs, uint64_t ws_bytes) {
   const Geo& g = ctx->g;
   HIPC(hipSetDevice(ctx->device));
   hipStream_t s = (hipStream_t)stream;
@@ -1479,16 +1541,27 @@ int launch_select_mass(ferry_ctx* ctx, int32_t l0, int32_t nl, const float* q,
     return FERRY_OK;
   }
   // matrix cores: the units' masses, then each item's sum over kv heads and top k
+  uint8_t* wsb = reinterpret_cast<uint8_t*>(ws);
   unsigned* counter = reinterpret_cast<unsigned*>(ws);
-  const size_t ulds = mass_lds_bytes(ctx);  // block log-sums in LDS, else HBM slices
-  float* slices = ulds ? nullptr : reinterpret_cast<float*>(reinterpret_cast<uint8_t*>(ws) + kMassCounterBytes);
-  float* mass = reinterpret_cast<float*>(reinterpret_cast<uint8_t*>(ws) + mass_mass_offset(ctx, wgs));
-  hipLaunchKernelGGL(k_mass_reset, dim3(1), dim3(64), 0, s, counter);
-  HIPC(hipGetLastError());
+  size_t ulds = mass_lds_bytes(ctx);  // block log-sums in LDS, else HBM slices
+  float* slices = ulds ? nullptr : reinterpret_cast<float*>(wsb + kMassCounterBytes);
+  float* mass = reinterpret_cast<float*>(wsb + mass_mass_offset(ctx, wgs));
+  int parts = mass_parts(ctx, nl);
+  const MassSplit split = mass_split_layout(ctx, nl, parts);
+  if (parts > 1 && split.bytes > ws_bytes) parts = 1;
+  if (parts > 1) {
+    wgs = (uint64_t)g.n_req * nl * g.Hkv * parts;
+    ulds = 0;
+    slices = ws;
+    mass = reinterpret_cast<float*>(wsb + split.ms);
+  } else {
+    hipLaunchKernelGGL(k_mass_reset, dim3(1), dim3(64), 0, s, counter);
+    HIPC(hipGetLastError());
+  }
 #define FERRY_MASS_UNITS(DT, GG)                                                                 \
   hipLaunchKernelGGL((k_mass_units<DT, GG, kMassUnitWaves, kMassUnitInflight>), dim3((unsigned)wgs), \
                      dim3(64 * kMassUnitWaves), ulds, s, g, q, ctx_blocks, ctx->ktab, ctx->ktab_scales, \
-                     ctx->kt_records, slices, mass, counter, l0, nl, g.max_blocks, ctx->err)
+                     ctx->kt_records, slices, mass, counter, parts, l0, nl, g.max_blocks, ctx->err)
 #define FERRY_MASS_UNITS_G(DT)                \
   switch (G) {                                \
     case 1: FERRY_MASS_UNITS(DT, 1); break;   \
@@ -1505,8 +1578,30 @@ int launch_select_mass(ferry_ctx* ctx, int32_t l0, int32_t nl, const float* q,
 #undef FERRY_MASS_UNITS
   HIPC(hipGetLastError());
   const unsigned items = (unsigned)std::min<uint64_t>((uint64_t)g.n_req * nl, kMassWgs);
-  hipLaunchKernelGGL((k_mass_topk<kMassTopkWaves>), dim3(items), dim3(64 * kMassTopkWaves), lds, s, g,
-                     ctx_blocks, mass, sel, l0, nl, g.max_blocks);
+  if (parts > 1) {  // fewer units than workgroup slots, so every item has a grid row
+    float* score = reinterpret_cast<float*>(wsb + split.score);
+    const dim3 fgrid((unsigned)((g.max_blocks + 255) / 256), (unsigned)(g.n_req * nl));
+    const size_t flds = (size_t)g.Hq * sizeof(float);
+#define FERRY_MASS_FINISH(GG)                                                                          \
+  hipLaunchKernelGGL(k_mass_finish<GG>, fgrid, dim3(256), flds, s, g, ctx_blocks, slices, mass, parts, \
+                     score, nl, g.max_blocks)
+    switch (G) {
+      case 1: FERRY_MASS_FINISH(1); break;
+      case 2: FERRY_MASS_FINISH(2); break;
+      case 4: FERRY_MASS_FINISH(4); break;
+      default: FERRY_MASS_FINISH(8); break;
+    }
+#undef FERRY_MASS_FINISH
+    HIPC(hipGetLastError());
+    mass = score;
+  }
+  const int rows = parts > 1 ? 1 : g.Hkv;  // mass rows of an item
+  if (items <= (unsigned)ctx->cus)
+    hipLaunchKernelGGL((k_mass_topk<kMassTopkWideWaves>), dim3(items), dim3(64 * kMassTopkWideWaves), lds,
+                       s, g, ctx_blocks, mass, rows, sel, l0, nl, g.max_blocks);
+  else
+    hipLaunchKernelGGL((k_mass_topk<kMassTopkWaves>), dim3(items), dim3(64 * kMassTopkWaves), lds, s, g,
+                       ctx_blocks, mass, rows, sel, l0, nl, g.max_blocks);
   HIPC(hipGetLastError());
   return FERRY_OK;
 }
@@ -1536,7 +1631,7 @@ int ferry_select_mass_layers(ferry_ctx* ctx, int32_t l0, int32_t nl, const float
   if (int rc = check_select_mass(ctx, l0, nl, q, ctx_blocks, sel)) return rc;
   if (!ctx->mass_ws) return fail(FERRY_EINVAL, "no mass-selection workspace (ferry_ktiles_build failed)");
   return launch_select_mass(ctx, l0, nl, q, ctx_blocks, sel, stream, ctx->mass_ws,
-                            mass_wgs(ctx, nl, ~0ull));
+                            mass_wgs(ctx, nl, ~0ull), mass_ctx_bytes(ctx));
 }
 
 int ferry_select_mass(ferry_ctx* ctx, const float* q, const int32_t* ctx_blocks, uint32_t* sel,
@@ -1570,7 +1665,7 @@ int ferry_select_mass_noalloc(ferry_ctx* ctx, const float* q, const int32_t* ctx
   for (int l0 = 0; l0 < g.L; l0 += nl) {
     const int n = std::min(nl, g.L - l0);
     if (int rc = launch_select_mass(ctx, l0, n, q, ctx_blocks, sel, stream, ctx->scratch_dev,
-                                    mass_wgs(ctx, n, wgs_cap(n))))
+                                    mass_wgs(ctx, n, wgs_cap(n)), kNoAllocScratchBytes))
       return rc;
   }
   return FERRY_OK;

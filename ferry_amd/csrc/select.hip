@@ -762,12 +762,19 @@ __global__ __launch_bounds__(W * 64) void k_select_mass(Geo g, const float* __re
 // 0.80-0.84 of HBM (by where the 137 GB table landed) against 0.79 for a
 // whole (request, layer) item per workgroup, whose kv heads stream one after
 // the other.
+//
+// parts > 1 (a launch of few units, mass_parts()): a unit's blocks are split
+// between `parts` workgroups, one part each (grid units * parts, no counter).
+// Every block's log-sums go to ws_all[unit][b][G] (G floats per 2-4 KiB
+// record), the part's (M, S) to mass[unit][part][G][2], and k_mass_finish
+// forms the masses once every part is done.  A unit per workgroup left half
+// the CUs idle at the long-context GQA shape's one-layer launch (128 units).
 template <int DT, int G, int W, int U>
 __global__ __launch_bounds__(W * 64) void k_mass_units(
     Geo g, const float* __restrict__ q, const int32_t* __restrict__ ctx_blocks,
     const uint8_t* __restrict__ kt, const float* __restrict__ kt_scales, uint64_t kt_mod,
-    float* __restrict__ ws_all, float* __restrict__ mass, unsigned* __restrict__ counter, int l0,
-    int nl, int max_n, int* __restrict__ err) {
+    float* __restrict__ ws_all, float* __restrict__ mass, unsigned* __restrict__ counter, int parts,
+    int l0, int nl, int max_n, int* __restrict__ err) {
   static_assert(G >= 1 && G <= 16, "the score tile holds up to 16 query heads");
   static_assert(DT == FERRY_F16 || DT == FERRY_BF16 || DT == FERRY_FP8_E4M3, "16/8-bit K");
   typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -786,17 +793,21 @@ __global__ __launch_bounds__(W * 64) void k_mass_units(
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int n = lane & 15, grp = lane >> 4;
   const bool head_lane = grp == 0 && n < G;
-  const bool in_lds = ws_all == nullptr;  // workgroup-uniform
-  float* ws = in_lds ? nullptr : ws_all + (size_t)blockIdx.x * max_n * G * 2;
+  const bool split = parts > 1;           // launch-uniform
+  const bool in_lds = ws_all == nullptr;  // launch-uniform
+  float* ws = in_lds || split ? nullptr : ws_all + (size_t)blockIdx.x * max_n * G * 2;
   const unsigned n_units = (unsigned)(g.n_req * nl * g.Hkv);
   const float qmul = 1.4426950408889634f / sqrtf((float)D);  // log2(e) / sqrt(D)
 
   for (;;) {
-    // the previous unit is done with the LDS and the workspace slice
-    if (tid == 0) next_unit = atomicAdd(counter, 1u);
-    __syncthreads();
-    const unsigned un = next_unit;
-    __syncthreads();  // every thread has read next_unit before it is rewritten
+    unsigned un = blockIdx.x / (unsigned)parts;
+    if (!split) {
+      // the previous unit is done with the LDS and the workspace slice
+      if (tid == 0) next_unit = atomicAdd(counter, 1u);
+      __syncthreads();
+      un = next_unit;
+      __syncthreads();  // every thread has read next_unit before it is rewritten
+    }
     if (un >= n_units) break;  // workgroup-uniform; every unit is taken once
     const int unit = (int)un;
     const int item = unit / g.Hkv, h = unit % g.Hkv;
@@ -808,7 +819,15 @@ __global__ __launch_bounds__(W * 64) void k_mass_units(
       if (tid == 0 && h == 0) set_error(err, FERRY_ERANGE);
       nb = 0;
     }
-    if (nb <= g.k) continue;  // workgroup-uniform: k_mass_topk lists every block
+    if (nb <= g.k) {  // workgroup-uniform: k_mass_topk lists every block
+      if (split) break;
+      continue;
+    }
+    // this workgroup's blocks [lo, hi) of the unit
+    const int part = split ? (int)(blockIdx.x % (unsigned)parts) : 0;
+    const int per = (nb + parts - 1) / parts;
+    const int lo = min(nb, part * per), hi = min(nb, lo + per);
+    if (split) ws = ws_all + (size_t)unit * max_n * G;
     const uint64_t set = (uint64_t)rl * g.Hkv + h;
     // ---- Q^T operand: k-step ks, this lane's 8 dims, head n (0 for pad heads)
     uint32_t qb[NQ][4][4];
@@ -840,13 +859,13 @@ __global__ __launch_bounds__(W * 64) void k_mass_units(
       }
     }
     float run_m = -INFINITY, run_s = 0.0f;
-    for (int b0 = wave; b0 < nb; b0 += W * U) {
+    for (int b0 = lo + wave; b0 < hi; b0 += W * U) {
       u32x4 kw[U][NKW];
       float ksc[U];
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         const int b = b0 + W * u;
-        if (b < nb) {  // wavefront-uniform
+        if (b < hi) {  // wavefront-uniform
           const uint64_t rec = host_index(set, (uint32_t)b, (uint64_t)g.max_blocks, kt_mod);
           // lane-transposed record: this lane's word w is word 64 w + lane
           const u32x4* base = reinterpret_cast<const u32x4*>(kt + rec * KT) + lane;
@@ -858,7 +877,7 @@ __global__ __launch_bounds__(W * 64) void k_mass_units(
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         const int b = b0 + W * u;
-        if (b >= nb) break;  // wavefront-uniform
+        if (b >= hi) break;  // wavefront-uniform
         f32x4 s = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) {
@@ -890,7 +909,9 @@ __global__ __launch_bounds__(W * 64) void k_mass_units(
         float e = (exp2f(x[0] - m) + exp2f(x[1] - m)) + (exp2f(x[2] - m) + exp2f(x[3] - m));
         e = sum_over_groups(e);
         if (head_lane) {
-          if (in_lds) {
+          if (split) {
+            ws[(size_t)b * G + n] = m + log2f(e);
+          } else if (in_lds) {
             lws[b * G + n] = m + log2f(e);  // the block's log2-sum-exp2
           } else {
             ws[((size_t)b * G + n) * 2] = m;
@@ -909,10 +930,16 @@ __global__ __launch_bounds__(W * 64) void k_mass_units(
     if (tid < G) {
       float mm = -INFINITY, ss = 0.0f;
       for (int w = 0; w < W; ++w) lse_merge(mm, ss, red_m[w][tid], red_s[w][tid]);
+      if (split) {  // k_mass_finish merges the parts' (M, S)
+        float* ms = mass + ((size_t)blockIdx.x * G + tid) * 2;
+        ms[0] = mm;
+        ms[1] = ss;
+      }
       lse_m[tid] = mm;
       lse_zi[tid] = 1.0f / ss;
       lse_l[tid] = mm + log2f(ss);  // the unit's log2-sum-exp2
     }
+    if (split) break;  // launch-uniform: one part per workgroup
     __syncthreads();
     float* mrow = mass + (size_t)unit * max_n;
     for (int b = tid; b < nb; b += NT) {
@@ -935,18 +962,58 @@ __global__ void k_mass_reset(unsigned* counter) {
   if (blockIdx.x == 0 && threadIdx.x == 0) *counter = 0u;
 }
 
+// k_mass_finish (after a k_mass_units launch with parts > 1): the score of
+// every block of every (request, layer) item, one thread per block.  A query
+// head's log2-sum-exp2 L is merged over its parts once per workgroup; the
+// block's score is exp2(l_b - L) summed over the query heads of a kv head, then
+// over the kv heads, in k_mass_topk's order.  Grid (blocks / 256, items);
+// dynamic LDS: a float per query head of the layer.
+template <int G>
+__global__ __launch_bounds__(256) void k_mass_finish(Geo g, const int32_t* __restrict__ ctx_blocks,
+                                                     const float* __restrict__ lsum,
+                                                     const float* __restrict__ part_ms, int parts,
+                                                     float* __restrict__ score, int nl, int max_n) {
+  extern __shared__ float lse[];  // [Hkv * G]
+  const int tid = threadIdx.x, item = blockIdx.y;
+  int nb = ctx_blocks[item / nl];
+  if (nb < 0 || nb > max_n || nb > g.max_blocks) nb = 0;  // k_mass_units latched the error
+  if (nb <= g.k || (int)blockIdx.x * 256 >= nb) return;    // workgroup-uniform
+  const size_t u0 = (size_t)item * g.Hkv;
+  for (int i = tid; i < g.Hkv * G; i += 256) {
+    const float* ms = part_ms + ((u0 + i / G) * parts * G + i % G) * 2;
+    float mm = -INFINITY, ss = 0.0f;
+    for (int p = 0; p < parts; ++p) lse_merge(mm, ss, ms[(size_t)p * G * 2], ms[(size_t)p * G * 2 + 1]);
+    lse[i] = mm + log2f(ss);
+  }
+  __syncthreads();
+  const int b = blockIdx.x * 256 + tid;
+  if (b >= nb) return;
+  float s = 0.0f;
+#pragma unroll 4
+  for (int hh = 0; hh < g.Hkv; ++hh) {
+    const float* l = lsum + ((u0 + hh) * max_n + b) * G;
+    float acc = 0.0f;
+#pragma unroll
+    for (int gq = 0; gq < G; ++gq) acc += exp2f(l[gq] - lse[hh * G + gq]);
+    s = hh == 0 ? acc : s + acc;
+  }
+  score[(size_t)item * max_n + b] = s;
+}
+
 // k_mass_topk: one (request, layer) item per workgroup pass.  A block's score
-// is its mass summed over the kv heads in head order (mass[unit][b] of the
-// item's Hkv units, written by k_mass_units in the same stream); the scores go
-// through the same radix top-k as the Quest method and the item's list is
-// written to every kv head's row.  A context of at most k blocks lists every
-// block in order.  Dynamic LDS: max_n keys.
+// is its mass summed over the item's `rows` mass rows in order: the kv heads'
+// (mass[unit][b], written by k_mass_units in the same stream), or one row of
+// finished scores (k_mass_finish).  The scores go through the same radix top-k
+// as the Quest method and the item's list is written to every kv head's row.
+// A context of at most k blocks lists every block in order.  A workgroup has
+// 16 wavefronts, which read an item's rows four blocks at a time, where a
+// launch has no more items than CUs, else 4.  Dynamic LDS: max_n keys.
 template <int W>
 __global__ __launch_bounds__(W * 64) void k_mass_topk(Geo g, const int32_t* __restrict__ ctx_blocks,
-                                                      const float* __restrict__ mass,
+                                                      const float* __restrict__ mass, int rows,
                                                       uint32_t* __restrict__ sel, int l0, int nl,
                                                       int max_n) {
-  constexpr int NT = W * 64;
+  constexpr int NT = W * 64, U = 4;
   extern __shared__ uint32_t lds[];
   __shared__ uint32_t hist[256];
   __shared__ uint32_t wtot[2 * W];
@@ -967,11 +1034,18 @@ __global__ __launch_bounds__(W * 64) void k_mass_topk(Geo g, const int32_t* __re
         for (int hh = 0; hh < g.Hkv; ++hh) out0[(size_t)hh * k + j] = j < kk ? (uint32_t)j : kNone;
       continue;
     }
-    const float* m0 = mass + (size_t)item * g.Hkv * max_n;
-    for (int b = tid; b < nb; b += NT) {
-      float s = m0[b];
-      for (int hh = 1; hh < g.Hkv; ++hh) s += m0[(size_t)hh * max_n + b];
-      lds[b] = fkey(s);
+    const float* m0 = mass + (size_t)item * rows * max_n;
+    for (int b0 = tid; b0 < nb; b0 += NT * U) {
+      float s[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) s[u] = b0 + u * NT < nb ? m0[b0 + u * NT] : 0.0f;
+      for (int hh = 1; hh < rows; ++hh)
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+          if (b0 + u * NT < nb) s[u] += m0[(size_t)hh * max_n + b0 + u * NT];
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (b0 + u * NT < nb) lds[b0 + u * NT] = fkey(s[u]);
     }
     __syncthreads();
     topk_ascending<W>(lds, nb, kk, hist, wtot, sh, out0, g.Hkv, (size_t)k);
@@ -987,7 +1061,7 @@ __global__ __launch_bounds__(W * 64) void k_mass_topk(Geo g, const int32_t* __re
 #define FERRY_MASS_UNITS_INST(DT, G)                                                          \
   template __global__ void k_mass_units<DT, G, kMassUnitWaves, kMassUnitInflight>(            \
       Geo, const float*, const int32_t*, const uint8_t*, const float*, uint64_t, float*, float*, \
-      unsigned*, int, int, int, int*);
+      unsigned*, int, int, int, int, int*);
 #define FERRY_MASS_UNITS_INST_G(DT) \
   FERRY_MASS_UNITS_INST(DT, 1)      \
   FERRY_MASS_UNITS_INST(DT, 2)      \
@@ -1000,8 +1074,18 @@ FERRY_MASS_INST(FERRY_F32, 8)
 FERRY_MASS_UNITS_INST_G(FERRY_F16)
 FERRY_MASS_UNITS_INST_G(FERRY_BF16)
 FERRY_MASS_UNITS_INST_G(FERRY_FP8_E4M3)
-template __global__ void k_mass_topk<kMassTopkWaves>(Geo, const int32_t*, const float*, uint32_t*, int,
-                                                     int, int);
+#define FERRY_MASS_TOPK_INST(W)                                                                 \
+  template __global__ void k_mass_topk<W>(Geo, const int32_t*, const float*, int, uint32_t*, int, \
+                                          int, int);
+FERRY_MASS_TOPK_INST(kMassTopkWaves)
+FERRY_MASS_TOPK_INST(kMassTopkWideWaves)
+#define FERRY_MASS_FINISH_INST(G)                                                                  \
+  template __global__ void k_mass_finish<G>(Geo, const int32_t*, const float*, const float*, int, \
+                                            float*, int, int);
+FERRY_MASS_FINISH_INST(1)
+FERRY_MASS_FINISH_INST(2)
+FERRY_MASS_FINISH_INST(4)
+FERRY_MASS_FINISH_INST(8)
 template __global__ void k_ktiles_build<2>(Geo, const uint8_t*, const float*, uint8_t*, float*, int);
 template __global__ void k_ktiles_build<4>(Geo, const uint8_t*, const float*, uint8_t*, float*, int);
 template __global__ void k_ktiles_build<8>(Geo, const uint8_t*, const float*, uint8_t*, float*, int);

@@ -34,11 +34,11 @@ def _run(p, q, ctx, layers=None):
     return sel.cpu().numpy().view(np.uint32)
 
 
-def _check_rows(p, got, q, ctx, rows=None):
+def _check_rows(p, got, q, ctx, rows=None, sc=None):
     """Compare got [B,L,Hkv,k] with the oracle under the near-tie bar; returns
     the fraction of rows that match exactly."""
     g = p.g
-    sc = O.mass_scores(g, q, ctx)
+    sc = O.mass_scores(g, q, ctx) if sc is None else sc
     exact = total = 0
     for r in range(g.n_req):
         for l in range(g.n_layers) if rows is None else rows:
@@ -141,6 +141,34 @@ def test_select_mass_hbm_workspace_parity(dtype, Hkv, Hq, monkeypatch):
     frac = _check_rows(p, _run(p, q, ctx), q, ctx)
     print("[mass] exact rows", frac, flush=True)
     assert frac >= 0.9
+    assert p.ex.stats()["device_error"] == 0
+
+
+@pytest.mark.parametrize("dtype,Hkv,Hq,ws", [
+    (F.BF16, 8, 16, ""), (F.F16, 8, 8, ""), (F.FP8, 8, 16, ""), (F.BF16, 8, 8, "hbm")])
+def test_select_mass_split_and_whole_units(dtype, Hkv, Hq, ws, monkeypatch):
+    """A launch of few (request, layer, kv head) units splits each one's blocks
+    between workgroups, a launch of many gives a unit to one workgroup: 64 and
+    320 units of the same rows (256 or 512 workgroup slots), with parts that
+    are empty, partly filled and full."""
+    monkeypatch.setenv("FERRY_MASS_WS", ws or "lds")
+    n_req, L, k, mb = 8, 5, 8, 290
+    print(f"[mass] split dtype={dtype} Hkv={Hkv} Hq={Hq} ws={ws or 'default'}", flush=True)
+    p = Pair(n_req, L, Hkv, Hq, k, 16, mb, dtype, host_blocks=4099)
+    p.ex.ktiles_build()
+    rng = np.random.default_rng(dtype + 17)
+    ctx = np.array([290, 257, 256, 65, 33, 9, 8, 0], np.int32)
+    q = rng.standard_normal((n_req, L, Hq, 128)).astype(np.float32)
+    dq, dctx = torch.from_numpy(q).cuda(), torch.from_numpy(ctx).cuda()
+    sc = O.mass_scores(p.g, q, ctx)
+    for step in (1, 5):  # layers per launch
+        sel = torch.full((n_req, L, Hkv, k), -7, dtype=torch.int32, device="cuda")
+        for l0 in range(0, L, step):
+            p.ex.select_mass(dq, dctx, sel, layers=(l0, step))
+        torch.cuda.synchronize()
+        frac = _check_rows(p, sel.cpu().numpy().view(np.uint32), q, ctx, sc=sc)
+        print("[mass] exact rows", step, frac, flush=True)
+        assert frac >= 0.9
     assert p.ex.stats()["device_error"] == 0
 
 
