@@ -12,7 +12,9 @@
 // so the members' selections of the shared prefix land on the same slots.
 //
 // One workgroup of W = 4 wavefronts per (group, layer, kv head), two per CU
-// (the LDS is mostly the wavefronts' block rings).  The group's
+// (the LDS is mostly the wavefronts' block rings).  Launches of few sets run
+// W = 8 and split a set's members between workgroups (mpw members each, whole
+// query tiles): everything below then holds for a workgroup's own members.  The group's
 // query columns (member x query head, NTILE tiles of 16, attn_mfma.hpp) are
 // held by every wavefront; the blocks are split between the wavefronts.
 //  1. List: every member row's slots are OR-ed into a per-slot member mask in
@@ -43,6 +45,8 @@
 //     merges its wavefronts.
 // HBM bytes per launch: the distinct blocks of each group set once (plus q in,
 // out and the slot table), against k blocks per member row for k_attn_mfma.
+// A split set's workgroups each read their own members' distinct blocks, with
+// loads that stay in cache for the others.
 #include "attn_mfma.hpp"
 #include "kernels.hpp"
 
@@ -92,6 +96,18 @@ __device__ inline void wait_blocks(int later) {
   }
 }
 
+// Set and part of workgroup i in a launch whose sets are split between `parts`
+// workgroups: the parts of a set are 8 workgroups apart, which puts them on the
+// same XCD (workgroups go round the 8 XCDs), close in time, so a block that
+// several of them read is found in that XCD's L2.
+struct GroupPart {
+  int set, part;
+};
+__device__ inline GroupPart group_part(uint32_t i, int parts) {
+  const uint32_t r = i % (8u * (uint32_t)parts);
+  return {(int)(i / (8u * (uint32_t)parts) * 8u + r % 8u), (int)(r / 8u)};
+}
+
 // Exclusive prefix sum of v over the workgroup's threads (thread order);
 // *total = the sum over all.  `sh` is LDS scratch of W ints.  Barriers on
 // entry and exit, so `sh` can be reused right after.
@@ -121,11 +137,11 @@ __device__ inline int block_exclusive_scan(int v, int* sh, int* total) {
 
 }  // namespace
 
-template <int DT, int G, int NTILE, int W>
+template <int DT, int G, int NTILE, int W, bool SPLIT>
 __global__ __launch_bounds__(W * 64) void k_attn_group(
     Geo g, const float* __restrict__ q, const uint32_t* __restrict__ slots,
     const uint8_t* __restrict__ pool, const float* __restrict__ pool_scales,
-    float* __restrict__ out, float qscale, int l0, int nl, int* __restrict__ err,
+    float* __restrict__ out, float qscale, int l0, int nl, int split_mpw, int* __restrict__ err,
     unsigned long long* __restrict__ attn_blocks) {
   static_assert(G == 2 || G == 4 || G == 8, "GQA group of 2, 4 or 8 query heads");
   static_assert(NTILE >= 1 && NTILE <= kGroupMaxTiles, "query tiles per workgroup");
@@ -152,7 +168,8 @@ __global__ __launch_bounds__(W * 64) void k_attn_group(
   static_assert(NTILE <= W, "each wavefront stages at most one query tile");
 
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-  const int GK = g.group * g.k;
+  const int mpw = SPLIT ? split_mpw : g.group;  // members per workgroup
+  const int GK = mpw * g.k;
   uint8_t* rings = smem;                                                  // [W][R][BB]
   u32x4* qops = reinterpret_cast<u32x4*>(smem + W * RB);                  // [NQ][NTILE][4][64]
   uint32_t* lslot = reinterpret_cast<uint32_t*>(qops + NQ * NTILE * 4 * 64);  // [GK] list
@@ -165,10 +182,16 @@ __global__ __launch_bounds__(W * 64) void k_attn_group(
 
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int n = lane & 15, grp = lane >> 4;
-  const int h = blockIdx.x % g.Hkv;
-  const int l = l0 + (blockIdx.x / g.Hkv) % nl;
-  const int o = blockIdx.x / (nl * g.Hkv);
-  const int mem = min(g.group, g.n_req - o * g.group);  // member rows of this owner
+  // (owner, layer, kv head) of this workgroup's set, and its member rows
+  // [m0, m0 + mem): the owner's, or those of this workgroup's part
+  const GroupPart gp = SPLIT ? group_part(blockIdx.x, (g.group + mpw - 1) / mpw)
+                             : GroupPart{(int)blockIdx.x, 0};
+  const int h = gp.set % g.Hkv;
+  const int l = l0 + (gp.set / g.Hkv) % nl;
+  const int o = gp.set / (nl * g.Hkv);
+  const int m0 = o * g.group + gp.part * mpw;
+  const int mem = min(SPLIT ? min(mpw, g.group - gp.part * mpw) : mpw, g.n_req - m0);
+  if (SPLIT && (o >= g.n_owners || mem <= 0)) return;  // workgroup-uniform
   const uint32_t base = (uint32_t)((o * g.L + l) * g.Hkv + h) * (uint32_t)g.C;
 
   // The global reads of the prologue go out together, so the workgroup pays
@@ -178,7 +201,7 @@ __global__ __launch_bounds__(W * 64) void k_attn_group(
   float qx[4][8];
   if (wave < NTILE) {  // tile `wave`: column n is member wave*MPT + n/G
     const int mi = wave * MPT + n / G;
-    const size_t qrow = (size_t)((o * g.group + mi) * g.L + l) * g.Hq + (size_t)h * G + n % G;
+    const size_t qrow = (size_t)((m0 + mi) * g.L + l) * g.Hq + (size_t)h * G + n % G;
     q_load<DT>(mi < mem ? q + qrow * D : nullptr, grp, qx);
   }
   constexpr int SB = 4;  // selections in flight per thread
@@ -188,7 +211,7 @@ __global__ __launch_bounds__(W * 64) void k_attn_group(
       const int e = e0 + u * NT, mi = e / g.k;
       sv[u] = kNone;
       if (e < GK && mi < mem)
-        sv[u] = slots[((size_t)((o * g.group + mi) * g.L + l) * g.Hkv + h) * g.k + (e - mi * g.k)];
+        sv[u] = slots[((size_t)((m0 + mi) * g.L + l) * g.Hkv + h) * g.k + (e - mi * g.k)];
     }
   };
   uint32_t sv[SB];
@@ -196,7 +219,7 @@ __global__ __launch_bounds__(W * 64) void k_attn_group(
 
   // ---- 1. the distinct list of the group's selections
   for (int i = tid; i < g.C; i += NT) msk[i] = 0u;
-  for (int i = tid; i < g.group; i += NT) mcnt[i] = 0u;
+  for (int i = tid; i < mpw; i += NT) mcnt[i] = 0u;
   __syncthreads();
   bool bad = false;
   for (int e0 = tid; e0 < GK; e0 += NT * SB) {
@@ -308,7 +331,8 @@ __global__ __launch_bounds__(W * 64) void k_attn_group(
       const int tile = p / (T * RC), pr = (p / RC) % T;
       const int off = (tile * T + lds_row<ES>(pr)) * ROW + ((p % RC) ^ lds_chunk<ES>(pr)) * 16;
       __builtin_amdgcn_global_load_lds((glb_void*)(src + off),
-                                       (lds_void*)(ring + b * BB + i * 1024), 16, 0, 2 /* nt */);
+                                       (lds_void*)(ring + b * BB + i * 1024), 16, 0,
+                                       SPLIT ? 0 : 2 /* nt: each block is read once */);
     }
   };
   // K word w of lane (n, grp): token n, logical chunk 4w + grp.  V of token i:
@@ -448,7 +472,7 @@ __global__ __launch_bounds__(W * 64) void k_attn_group(
         const int mi = t * MPT + n / G;
         if (mi >= mem) continue;
         const size_t qrow =
-            (size_t)((o * g.group + mi) * g.L + l) * g.Hq + (size_t)h * G + n % G;
+            (size_t)((m0 + mi) * g.L + l) * g.Hq + (size_t)h * G + n % G;
         float4* dst = reinterpret_cast<float4*>(out + qrow * D + 32 * grp);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -461,27 +485,24 @@ __global__ __launch_bounds__(W * 64) void k_attn_group(
   }
 }
 
-#define FERRY_ATTN_GROUP_INST_W(DT, G, NTILE, W)                                          \
-  template __global__ void k_attn_group<DT, G, NTILE, W>(Geo, const float*, const uint32_t*, \
-                                                         const uint8_t*, const float*, float*, \
-                                                         float, int, int, int*,              \
-                                                         unsigned long long*);
-#define FERRY_ATTN_GROUP_INST(DT, G, NTILE)                       \
-  FERRY_ATTN_GROUP_INST_W(DT, G, NTILE, group_waves(DT))          \
-  FERRY_ATTN_GROUP_INST_W(DT, G, NTILE, kGroupWideWaves)
+#define FERRY_ATTN_GROUP_INST_W(DT, G, NTILE, W, SPLIT)                                    \
+  template __global__ void k_attn_group<DT, G, NTILE, W, SPLIT>(                            \
+      Geo, const float*, const uint32_t*, const uint8_t*, const float*, float*, float, int, \
+      int, int, int*, unsigned long long*);
+#define FERRY_ATTN_GROUP_INST(DT, G, NTILE, SPLIT)                \
+  FERRY_ATTN_GROUP_INST_W(DT, G, NTILE, group_waves(DT), SPLIT)   \
+  FERRY_ATTN_GROUP_INST_W(DT, G, NTILE, kGroupWideWaves, SPLIT)
+#define FERRY_ATTN_GROUP_INST_G(DT, G)     \
+  FERRY_ATTN_GROUP_INST(DT, G, 1, false)   \
+  FERRY_ATTN_GROUP_INST(DT, G, 2, false)   \
+  FERRY_ATTN_GROUP_INST(DT, G, 3, false)   \
+  FERRY_ATTN_GROUP_INST(DT, G, 4, false)   \
+  FERRY_ATTN_GROUP_INST(DT, G, 1, true)    \
+  FERRY_ATTN_GROUP_INST(DT, G, 2, true)
 #define FERRY_ATTN_GROUP_INST_DT(DT) \
-  FERRY_ATTN_GROUP_INST(DT, 2, 1)    \
-  FERRY_ATTN_GROUP_INST(DT, 2, 2)    \
-  FERRY_ATTN_GROUP_INST(DT, 2, 3)    \
-  FERRY_ATTN_GROUP_INST(DT, 2, 4)    \
-  FERRY_ATTN_GROUP_INST(DT, 4, 1)    \
-  FERRY_ATTN_GROUP_INST(DT, 4, 2)    \
-  FERRY_ATTN_GROUP_INST(DT, 4, 3)    \
-  FERRY_ATTN_GROUP_INST(DT, 4, 4)    \
-  FERRY_ATTN_GROUP_INST(DT, 8, 1)    \
-  FERRY_ATTN_GROUP_INST(DT, 8, 2)    \
-  FERRY_ATTN_GROUP_INST(DT, 8, 3)    \
-  FERRY_ATTN_GROUP_INST(DT, 8, 4)
+  FERRY_ATTN_GROUP_INST_G(DT, 2)     \
+  FERRY_ATTN_GROUP_INST_G(DT, 4)     \
+  FERRY_ATTN_GROUP_INST_G(DT, 8)
 FERRY_ATTN_GROUP_INST_DT(FERRY_F16)
 FERRY_ATTN_GROUP_INST_DT(FERRY_BF16)
 FERRY_ATTN_GROUP_INST_DT(FERRY_FP8_E4M3)

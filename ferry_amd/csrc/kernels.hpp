@@ -121,9 +121,10 @@ __global__ void k_attn_mfma(Geo g, const float* q, const uint32_t* slots, const 
                             int* err);
 
 // Prefix-group attention (attn_group.hip): one workgroup of W wavefronts per
-// (group, layer, kv head) reads each distinct block of the group's set once
-// and attends every member row; NTILE tiles of 16 query columns (group * G /
-// 16 rounded up); dynamic LDS of attn_group_lds_bytes().  The LDS holds each
+// (group, layer, kv head), with SPLIT per `mpw` of its members, reads each
+// distinct block of its members once and attends their rows; NTILE tiles of 16
+// query columns (members * G / 16 rounded up); dynamic LDS of
+// attn_group_lds_bytes().  The LDS holds each
 // wavefront's ring of blocks in flight: group_waves() = four wavefronts with
 // three fp8 blocks (or two 16-bit blocks) each let two workgroups share a CU.
 // Eight wavefronts with four fp8 blocks each (one workgroup per CU, 96 KiB in
@@ -141,10 +142,10 @@ constexpr int group_ring_blocks(int dtype) { return dtype == FERRY_FP8_E4M3 ? 3 
 constexpr int group_ring_bytes(int dtype) {
   return group_ring_blocks(dtype) * 2 * 16 * 128 * (dtype == FERRY_FP8_E4M3 ? 1 : 2);
 }
-template <int DT, int G, int NTILE, int W>
+template <int DT, int G, int NTILE, int W, bool SPLIT>
 __global__ void k_attn_group(Geo g, const float* q, const uint32_t* slots, const uint8_t* pool,
                              const float* pool_scales, float* out, float qscale, int l0, int nl,
-                             int* err, unsigned long long* attn_blocks);
+                             int mpw, int* err, unsigned long long* attn_blocks);
 // LDS of one k_attn_group workgroup: the wavefronts' rings, the Q^T operands
 // of every tile (fp16, or bf16 hi and lo parts: 4 KiB per part and tile), the
 // distinct list (slot and member mask per entry, at most group * k entries),

@@ -342,18 +342,38 @@ void launch_mfma(const AttnPlan& p, const dim3& grid, hipStream_t s, const AttnA
     hipLaunchKernelGGL((k_attn_mfma<DT, G, W, false>), grid, dim3(W * 64), 0, s, a.g, a.q,
                        a.slots, a.pool, a.pool_scales, a.out, a.qscale, a.l0, a.nl, a.err);
 }
-template <int DT, int G, int NT, int W>
-void launch_group_w(const dim3& grid, size_t lds, hipStream_t s, const AttnArgs& a) {
+// Query tiles per workgroup of a prefix-group launch: the fewest for which the
+// launch still has no more workgroups than the GPU has CUs, else all of the
+// set's.  A set of several tiles costs a workgroup their arithmetic one after
+// the other at every block; with CUs to spare its members are split between
+// workgroups of 1 or 2 tiles, each listing its own members' blocks.  They read
+// 1.1-1.4 times the set's distinct blocks between them, in part from the
+// XCD's L2 (group_part), which costs more than it gives once the CUs are full.
+// fp8, 16 members of 4 query heads (4 tiles), k 64, us per launch, 4 / 2 / 1
+// tiles per workgroup of 8 wavefronts: 8 sets 83 / 47 / 27, 64 sets
+// 85 / 50 / 31, 128 sets 91 / 57 / 64, 192 sets 95 / 115 / 101, 512 sets (4
+// wavefronts) 215 / 233 / 241.
+int group_tiles(int tiles, long sets, int cus) {
+  for (int t = 1; t < tiles; t = t == 1 ? 2 : tiles)
+    if (sets * ((tiles + t - 1) / t) <= (long)cus) return t;
+  return tiles;
+}
+// Members per workgroup: those of its tiles (16 / G each).
+int group_members(int tiles_per_wg, int tiles, int G, int group) {
+  return tiles_per_wg < tiles ? tiles_per_wg * 16 / G : group;
+}
+template <int DT, int G, int NT, int W, bool SPLIT>
+void launch_group_w(const dim3& grid, size_t lds, int mpw, hipStream_t s, const AttnArgs& a) {
   // more than the default 64 KiB of dynamic LDS: allowed once per instance and
   // device (the caller has made the context's device current)
   static std::atomic<uint64_t> allowed{0};
   int dev = 0;
   if (hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < 64 && !((allowed.load() >> dev) & 1u) &&
-      hipFuncSetAttribute(reinterpret_cast<const void*>(&k_attn_group<DT, G, NT, W>),
+      hipFuncSetAttribute(reinterpret_cast<const void*>(&k_attn_group<DT, G, NT, W, SPLIT>),
                           hipFuncAttributeMaxDynamicSharedMemorySize, kGroupMaxLds) == hipSuccess)
     allowed.fetch_or(1ull << dev);
-  hipLaunchKernelGGL((k_attn_group<DT, G, NT, W>), grid, dim3(W * 64), lds, s, a.g, a.q, a.slots,
-                     a.pool, a.pool_scales, a.out, a.qscale, a.l0, a.nl, a.err, a.attn_blocks);
+  hipLaunchKernelGGL((k_attn_group<DT, G, NT, W, SPLIT>), grid, dim3(W * 64), lds, s, a.g, a.q, a.slots,
+                     a.pool, a.pool_scales, a.out, a.qscale, a.l0, a.nl, mpw, a.err, a.attn_blocks);
 }
 // Wavefronts per workgroup of a prefix-group launch over `sets` group sets:
 // eight where the launch has no more sets than the GPU has CUs and the wider
@@ -364,26 +384,34 @@ int group_launch_waves(int dtype, int ntile, long gk, long sets, int cus, int fo
              ? kGroupWideWaves
              : group_waves(dtype);
 }
-template <int DT, int G, int NT>
-void launch_group(const dim3& grid, int cus, int force, hipStream_t s, const AttnArgs& a) {
-  const long gk = (long)a.g.group * a.g.k;
-  if (group_launch_waves(DT, NT, gk, grid.x, cus, force) == kGroupWideWaves)
-    launch_group_w<DT, G, NT, kGroupWideWaves>(
-        grid, attn_group_lds_bytes(DT, NT, gk, kGroupWideWaves), s, a);
+template <int DT, int G, int NT, bool SPLIT>
+void launch_group(long sets, int mpw, int cus, int force, hipStream_t s, const AttnArgs& a) {
+  const long gk = (long)mpw * a.g.k, parts = (a.g.group + mpw - 1) / mpw;
+  const dim3 grid((unsigned)(SPLIT ? (sets + 7) / 8 * 8 * parts : sets));
+  if (group_launch_waves(DT, NT, gk, sets, cus, force) == kGroupWideWaves)
+    launch_group_w<DT, G, NT, kGroupWideWaves, SPLIT>(
+        grid, attn_group_lds_bytes(DT, NT, gk, kGroupWideWaves), mpw, s, a);
   else
-    launch_group_w<DT, G, NT, group_waves(DT)>(
-        grid, attn_group_lds_bytes(DT, NT, gk, group_waves(DT)), s, a);
+    launch_group_w<DT, G, NT, group_waves(DT), SPLIT>(
+        grid, attn_group_lds_bytes(DT, NT, gk, group_waves(DT)), mpw, s, a);
 }
 template <int DT, int G>
 void launch_g(const AttnPlan& p, const dim3& grid, hipStream_t s, const AttnArgs& a) {
   if constexpr (DT != FERRY_F32 && G >= 2) {
     if (p.grouped) {
-      const dim3 ggrid((unsigned)(a.g.n_owners * a.nl * a.g.Hkv));
+      const long sets = (long)a.g.n_owners * a.nl * a.g.Hkv;
+      const int tpw = group_tiles(p.tiles, sets, p.cus);
+      const int mpw = group_members(tpw, p.tiles, G, a.g.group);
+      if (tpw < p.tiles) {
+        if (tpw == 1) launch_group<DT, G, 1, true>(sets, mpw, p.cus, p.group_w, s, a);
+        else launch_group<DT, G, 2, true>(sets, mpw, p.cus, p.group_w, s, a);
+        return;
+      }
       switch (p.tiles) {
-        case 1: launch_group<DT, G, 1>(ggrid, p.cus, p.group_w, s, a); return;
-        case 2: launch_group<DT, G, 2>(ggrid, p.cus, p.group_w, s, a); return;
-        case 3: launch_group<DT, G, 3>(ggrid, p.cus, p.group_w, s, a); return;
-        default: launch_group<DT, G, 4>(ggrid, p.cus, p.group_w, s, a); return;
+        case 1: launch_group<DT, G, 1, false>(sets, mpw, p.cus, p.group_w, s, a); return;
+        case 2: launch_group<DT, G, 2, false>(sets, mpw, p.cus, p.group_w, s, a); return;
+        case 3: launch_group<DT, G, 3, false>(sets, mpw, p.cus, p.group_w, s, a); return;
+        default: launch_group<DT, G, 4, false>(sets, mpw, p.cus, p.group_w, s, a); return;
       }
     }
   }
@@ -999,9 +1027,13 @@ int ferry_attn_kernel(const ferry_ctx* ctx, int32_t* kind, int32_t* waves) {
   const AttnPlan p = attn_plan(ctx);
   *kind = p.grouped ? FERRY_ATTN_GROUP : p.mfma ? FERRY_ATTN_MFMA : FERRY_ATTN_VALU;
   *waves = p.waves;
-  if (p.grouped)  // ferry_sparse_decode's launch: every layer's group sets
-    *waves = group_launch_waves(p.dtype, p.tiles, (long)ctx->g.group * ctx->g.k,
-                                (long)ctx->g.n_owners * ctx->g.L * ctx->g.Hkv, p.cus, p.group_w);
+  if (p.grouped) {  // ferry_sparse_decode's launch: every layer's group sets
+    const long sets = (long)ctx->g.n_owners * ctx->g.L * ctx->g.Hkv;
+    const int tpw = group_tiles(p.tiles, sets, p.cus);
+    *waves = group_launch_waves(p.dtype, tpw,
+                                (long)group_members(tpw, p.tiles, p.G, ctx->g.group) * ctx->g.k, sets,
+                                p.cus, p.group_w);
+  }
   return FERRY_OK;
 }
 
