@@ -6,7 +6,9 @@
 // the per-step top-k block selection of tools/capture_miss_trace.py:139-159.
 //
 // Work decomposition (HBM-bound, ~1-8 flop/byte): one workgroup per
-// (request, layer, kv head); its W wavefronts take every W-th selected block.  A block is K[T][D] then V[T][D].  Each 16-byte load instruction of a
+// (request, layer, kv head), several in a launch of few rows (SPLIT, merged by
+// the last of them: attn_common.hpp); their wavefronts deal the selected
+// blocks out between them.  A block is K[T][D] then V[T][D].  Each 16-byte load instruction of a
 // wavefront covers one contiguous KiB of the tile, so lane l holds the
 // EPV-element dim chunk (l % LPT) of token (l / LPT) + ld * TPL.  The q.K dot
 // product is reduced over the LPT lanes of a row with DPP row ops (no LDS);
@@ -89,13 +91,13 @@ struct Softmax {
 
 }  // namespace
 
-template <int DT, int G, int W, bool NT>
+template <int DT, int G, int W, bool NT, bool SPLIT>
 __global__ __launch_bounds__(W * 64) void k_attn(Geo g, const float* __restrict__ q,
                                               const uint32_t* __restrict__ slots,
                                               const uint8_t* __restrict__ pool,
                                               const float* __restrict__ pool_scales,
                                               float* __restrict__ out, float qscale, int l0,
-                                              int nl, int* __restrict__ err) {
+                                              int nl, int* __restrict__ err, RowSplit rs) {
   constexpr int ES = DT == FERRY_F32 ? 4 : (DT == FERRY_FP8_E4M3 ? 1 : 2);
   constexpr int D = 128, T = 16;
   constexpr int EPV = 16 / ES;   // elements per 16-byte word
@@ -111,10 +113,14 @@ __global__ __launch_bounds__(W * 64) void k_attn(Geo g, const float* __restrict_
   __shared__ int id_cnt[kMaxTopK / 64];
 
   // (request, layer in [l0, l0 + nl), kv head) of this workgroup
-  const int h = blockIdx.x % g.Hkv;
-  const int rl = (blockIdx.x / (nl * g.Hkv)) * g.L + l0 + (blockIdx.x / g.Hkv) % nl;
+  const int wrow = SPLIT ? blockIdx.x / rs.parts : blockIdx.x;  // row of the launch
+  const int part = SPLIT ? blockIdx.x % rs.parts : 0;
+  const int h = wrow % g.Hkv;
+  const int rl = (wrow / (nl * g.Hkv)) * g.L + l0 + (wrow / g.Hkv) % nl;
   const int row = rl * g.Hkv + h;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  // this wavefront takes blocks w0, w0 + WS, ... of the row
+  const int WS = SPLIT ? W * rs.parts : W, w0 = part * W + wave;
   const int dg = lane % LPT;
 
   float qv[G][EPV];
@@ -139,19 +145,19 @@ __global__ __launch_bounds__(W * 64) void k_attn(Geo g, const float* __restrict_
   // positions are dropped, so k is the number of blocks this row attends to.
   const int k = stage_row_ids<W>(slots + (size_t)row * g.k, g.k, ids, id_cnt);
   // Ring of NPF block buffers (NPF = 1: load, then consume).  While block j
-  // (= wave + W*j of the row) is consumed, blocks j+1 .. j+NPF-1 are in flight;
+  // (= w0 + WS*j of the row) is consumed, blocks j+1 .. j+NPF-1 are in flight;
   // the loop is unrolled by NPF so every buffer index is static, and every
   // iteration issues its loads so the compiler's load counters stay exact.
   // Past the end of the row those loads are never consumed: every lane then
   // reads the same 16 bytes of the last block, one line per instruction
   // (non-temporal loads would not find a re-read whole block in cache).
-  const int nb = k > wave ? (k - wave + W - 1) / W : 0;
+  const int nb = k > w0 ? (k - w0 + WS - 1) / WS : 0;
   // A slot outside the pool is read as slot 0 and reported once at the end
   // (no branch in the block loop).
   bool bad_slot = false;
   auto slot_at = [&](int j) -> uint64_t {
     const uint64_t slot =
-        (uint32_t)__builtin_amdgcn_readfirstlane((int)ids[wave + W * min(j, nb - 1)]);
+        (uint32_t)__builtin_amdgcn_readfirstlane((int)ids[w0 + WS * min(j, nb - 1)]);
     const bool bad = slot >= g.pool_slots;
     bad_slot |= bad;
     return bad ? 0 : slot;
@@ -275,21 +281,36 @@ __global__ __launch_bounds__(W * 64) void k_attn(Geo g, const float* __restrict_
 #pragma unroll
       for (int e = 0; e < EPV; ++e) o[e] += red[w][gq][c][2 + e] * a;
     }
-    // a row with no selected block (request not resident) attends to nothing: 0
-    const float inv = l > 0.0f ? 1.0f / l : 0.0f;
-    float* op = out + ((size_t)rl * g.Hq + (size_t)h * G + gq) * D + c * EPV;
+    if constexpr (SPLIT) {
+      float* st = rs.state + ((size_t)blockIdx.x * G + gq) * kPartFloats;
 #pragma unroll
-    for (int e = 0; e < EPV; ++e) op[e] = o[e] * inv;
+      for (int e = 0; e < EPV; e += 2) part_store2(st + 2 + c * EPV + e, o[e], o[e + 1]);
+      if (c == 0) part_store2(st, m, l);
+    } else {
+      // a row with no selected block (request not resident) attends to nothing: 0
+      const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+      float* op = out + ((size_t)rl * g.Hq + (size_t)h * G + gq) * D + c * EPV;
+#pragma unroll
+      for (int e = 0; e < EPV; ++e) op[e] = o[e] * inv;
+    }
+  }
+  if constexpr (SPLIT) {
+    __shared__ uint32_t seen;
+    __shared__ float2 fac[G * kMaxParts];
+    if (last_part(rs, wrow, &seen))  // workgroup-uniform
+      merge_row<G>(rs, wrow, fac, out + ((size_t)rl * g.Hq + (size_t)h * G) * D);
   }
 }
 
-#define FERRY_ATTN_INST(DT, G, W)                                                          \
-  template __global__ void k_attn<DT, G, W, false>(Geo, const float*, const uint32_t*,        \
-                                                   const uint8_t*, const float*, float*, float, \
-                                                   int, int, int*);                            \
-  template __global__ void k_attn<DT, G, W, true>(Geo, const float*, const uint32_t*,         \
-                                                  const uint8_t*, const float*, float*, float,  \
-                                                  int, int, int*);
+#define FERRY_ATTN_INST_S(DT, G, W, NT, SPLIT)                                            \
+  template __global__ void k_attn<DT, G, W, NT, SPLIT>(Geo, const float*, const uint32_t*, \
+                                                       const uint8_t*, const float*, float*, \
+                                                       float, int, int, int*, RowSplit);
+#define FERRY_ATTN_INST(DT, G, W)           \
+  FERRY_ATTN_INST_S(DT, G, W, false, false) \
+  FERRY_ATTN_INST_S(DT, G, W, true, false)  \
+  FERRY_ATTN_INST_S(DT, G, W, false, true)  \
+  FERRY_ATTN_INST_S(DT, G, W, true, true)
 #define FERRY_ATTN_INST_G(DT, W) \
   FERRY_ATTN_INST(DT, 1, W)      \
   FERRY_ATTN_INST(DT, 2, W)      \

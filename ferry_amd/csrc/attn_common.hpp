@@ -130,4 +130,90 @@ __device__ inline int stage_row_ids(const uint32_t* __restrict__ sl, int k, uint
   return total;
 }
 
+// ---- rows split between workgroups (launches of few rows) ----
+// `parts` workgroups attend one row's blocks, each writes its softmax state of
+// every query head to `state` (max, sum, then the 128 unnormalised outputs) and
+// adds one to the row's word of `count`; the one that finds parts - 1 there
+// merges the states and writes the row, in part order, so the result does not
+// depend on which workgroup came last.  It leaves the word 0 for the next
+// launch.  States and counts go through relaxed agent-scope atomics, which
+// complete past the XCDs' L2s (the workgroups may sit on different XCDs), and
+// each side waits for its own accesses, so no fence has to write back and
+// invalidate an L2: with those the merge of 256 workgroups took 10 us longer.
+// Both belong to one stream, so no other launch uses them meanwhile.
+struct RowSplit {
+  float* state;     // [rows * parts][G][kPartFloats]
+  uint32_t* count;  // [rows], 0 between launches
+  int parts;        // at most kMaxParts
+};
+constexpr int kPartFloats = 130;
+constexpr int kMaxParts = 8;
+
+__device__ inline void part_store2(float* p, float a, float b) {
+  astore64(reinterpret_cast<uint64_t*>(p),
+           (uint64_t)__builtin_bit_cast(uint32_t, a) | (uint64_t)__builtin_bit_cast(uint32_t, b) << 32);
+}
+__device__ inline float2 part_load2(const float* p) {
+  const uint64_t v = aload64(reinterpret_cast<const uint64_t*>(p));
+  return float2{__builtin_bit_cast(float, (uint32_t)v), __builtin_bit_cast(float, (uint32_t)(v >> 32))};
+}
+
+// Every thread of the workgroup calls it after its part_stores: true in every
+// thread of the row's last workgroup, whose part_loads then read every state.
+// `sh` is an LDS word.
+__device__ inline bool last_part(const RowSplit& rs, int row, uint32_t* sh) {
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wavefront's states have landed
+  __syncthreads();
+  if (threadIdx.x == 0)
+    *sh = __hip_atomic_fetch_add(rs.count + row, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __syncthreads();
+  const bool last = *sh == (uint32_t)rs.parts - 1u;
+  if (last && threadIdx.x == 0) astore(rs.count + row, 0u);
+  return last;
+}
+
+// The row's G * 128 outputs from its parts' states, by every thread of the last
+// workgroup: the (max, sum) pairs go to `fac` (LDS, [G * kMaxParts]) with one
+// load in flight per thread, become each part's factor 2^(m_p - M) / L there,
+// and a thread then sums its pairs of outputs four parts at a time (loads in
+// flight together).  Read one part after the other, 16 parts of 8 heads took
+// 20 us.
+template <int G>
+__device__ inline void merge_row(const RowSplit& rs, int row, float2* fac, float* __restrict__ out) {
+  const float* st = rs.state + (size_t)row * rs.parts * G * kPartFloats;
+  const int np = rs.parts, nt = blockDim.x;
+  for (int t = threadIdx.x; t < G * np; t += nt) {  // t = part * G + head
+    fac[(t % G) * kMaxParts + t / G] = part_load2(st + (size_t)t * kPartFloats);
+  }
+  __syncthreads();
+  if (threadIdx.x < G) {
+    float2* f = fac + threadIdx.x * kMaxParts;
+    float m = f[0].x, l = 0.0f;
+    for (int p = 1; p < np; ++p) m = fmaxf(m, f[p].x);
+    for (int p = 0; p < np; ++p) l += f[p].y * __builtin_amdgcn_exp2f(f[p].x - m);
+    // a row with no selected block (request not resident) attends to nothing: 0
+    const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+    for (int p = 0; p < np; ++p) f[p].y = __builtin_amdgcn_exp2f(f[p].x - m) * inv;
+  }
+  __syncthreads();
+  for (int t = threadIdx.x; t < G * 64; t += nt) {  // t = head * 64 + pair of dims
+    const float* o = st + (size_t)(t >> 6) * kPartFloats + 2 + 2 * (t & 63);
+    const float2* f = fac + (t >> 6) * kMaxParts;
+    float a = 0.0f, b = 0.0f;
+    for (int p0 = 0; p0 < np; p0 += 4) {
+      float2 v[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        v[u] = part_load2(o + (size_t)min(p0 + u, np - 1) * G * kPartFloats);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const float w = p0 + u < np ? f[p0 + u].y : 0.0f;
+        a = __builtin_fmaf(v[u].x, w, a);
+        b = __builtin_fmaf(v[u].y, w, b);
+      }
+    }
+    *reinterpret_cast<float2*>(out + 2 * t) = float2{a, b};
+  }
+}
+
 }  // namespace ferry_amd

@@ -11,7 +11,9 @@
 //   S^T[16 tok][16 hd] = K[16 tok][128] . Q^T[128][16 hd]   (4x mfma 16x16x32)
 //   O^T[128][16 hd]   += V^T[128][16 tok] . P^T[16 tok][16 hd] (8x mfma 16x16x16)
 // with the G heads padded to the 16 columns of the tile.  One workgroup per
-// (request, layer, kv head); its W wavefronts take every W-th block.
+// (request, layer, kv head), several in a launch of few rows (SPLIT, merged by
+// the last of them: attn_common.hpp); their wavefronts deal the blocks out
+// between them.
 //
 // Operand layouts, precision and the per-block arithmetic are in attn_mfma.hpp
 // (shared with the prefix-group kernel of attn_group.hip).
@@ -22,13 +24,13 @@ namespace ferry_amd {
 
 using namespace mx;
 
-template <int DT, int G, int W, bool NT>
+template <int DT, int G, int W, bool NT, bool SPLIT>
 __global__ __launch_bounds__(W * 64) void k_attn_mfma(Geo g, const float* __restrict__ q,
                                                    const uint32_t* __restrict__ slots,
                                                    const uint8_t* __restrict__ pool,
                                                    const float* __restrict__ pool_scales,
                                                    float* __restrict__ out, float qscale, int l0,
-                                                   int nl, int* __restrict__ err) {
+                                                   int nl, int* __restrict__ err, RowSplit rs) {
   static_assert(G >= 1 && G <= 16, "MFMA tile holds up to 16 query heads");
   static_assert(DT == FERRY_F16 || DT == FERRY_BF16 || DT == FERRY_FP8_E4M3, "16/8-bit KV");
   using S = Shape<DT>;
@@ -42,10 +44,14 @@ __global__ __launch_bounds__(W * 64) void k_attn_mfma(Geo g, const float* __rest
   __shared__ uint32_t ids[kMaxTopK];
   __shared__ int id_cnt[kMaxTopK / 64];
 
-  const int h = blockIdx.x % g.Hkv;
-  const int rl = (blockIdx.x / (nl * g.Hkv)) * g.L + l0 + (blockIdx.x / g.Hkv) % nl;
+  const int wrow = SPLIT ? blockIdx.x / rs.parts : blockIdx.x;  // row of the launch
+  const int part = SPLIT ? blockIdx.x % rs.parts : 0;
+  const int h = wrow % g.Hkv;
+  const int rl = (wrow / (nl * g.Hkv)) * g.L + l0 + (wrow / g.Hkv) % nl;
   const int row = rl * g.Hkv + h;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  // this wavefront takes blocks w0, w0 + WS, ... of the row
+  const int WS = SPLIT ? W * rs.parts : W, w0 = part * W + wave;
   const int n = lane & 15, grp = lane >> 4;
 
   // ---- Q^T operand of head n (0 for the padding columns n >= G)
@@ -59,13 +65,13 @@ __global__ __launch_bounds__(W * 64) void k_attn_mfma(Geo g, const float* __rest
   // (lgkmcnt) that never waits on the block loads in flight (vmcnt).  Empty
   // positions are dropped, so k is the number of blocks this row attends to.
   const int k = stage_row_ids<W>(slots + (size_t)row * g.k, g.k, ids, id_cnt);
-  const int nblk = k > wave ? (k - wave + W - 1) / W : 0;
+  const int nblk = k > w0 ? (k - w0 + WS - 1) / WS : 0;
   // A slot outside the pool is read as slot 0 and reported once at the end
   // (no branch in the block loop).
   bool bad_slot = false;
   auto slot_at = [&](int j) -> uint64_t {
     const uint64_t slot =
-        (uint32_t)__builtin_amdgcn_readfirstlane((int)ids[wave + W * min(j, nblk - 1)]);
+        (uint32_t)__builtin_amdgcn_readfirstlane((int)ids[w0 + WS * min(j, nblk - 1)]);
     const bool bad = slot >= g.pool_slots;
     bad_slot |= bad;
     return bad ? 0 : slot;
@@ -93,7 +99,7 @@ __global__ __launch_bounds__(W * 64) void k_attn_mfma(Geo g, const float* __rest
     }
   };
 
-  // Ring of NPF block buffers: while block j (= wave + W*j of the row) is
+  // Ring of NPF block buffers: while block j (= w0 + WS*j of the row) is
   // consumed, blocks j+1 .. j+NPF-1 are in flight.  The loop is unrolled by NPF
   // so every buffer index is static, and every iteration issues its loads (past
   // the end, one line of the last block) so the compiler's load counters stay
@@ -148,28 +154,52 @@ __global__ __launch_bounds__(W * 64) void k_attn_mfma(Geo g, const float* __rest
   }
   __syncthreads();
   // ---- merge the W wavefronts and write out
-  for (int t = threadIdx.x; t < G * D; t += blockDim.x) {
-    const int hq = t / D, d = t % D;
-    float mx = red_ml[0][hq][0];
-    for (int w = 1; w < W; ++w) mx = fmaxf(mx, red_ml[w][hq][0]);
-    float l = 0.0f, o = 0.0f;
-    for (int w = 0; w < W; ++w) {
-      const float a = exp2_fast(red_ml[w][hq][0] - mx);
-      l += red_ml[w][hq][1] * a;
-      o += red_o[w][hq][d] * a;
+  if constexpr (SPLIT) {
+    __shared__ uint32_t seen;
+    __shared__ float2 fac[G * kMaxParts];
+    for (int t = threadIdx.x; t < G * (D / 2); t += blockDim.x) {
+      const int hq = t / (D / 2), d = t % (D / 2) * 2;
+      float mx = red_ml[0][hq][0];
+      for (int w = 1; w < W; ++w) mx = fmaxf(mx, red_ml[w][hq][0]);
+      float l = 0.0f, o0 = 0.0f, o1 = 0.0f;
+      for (int w = 0; w < W; ++w) {
+        const float a = exp2_fast(red_ml[w][hq][0] - mx);
+        l += red_ml[w][hq][1] * a;
+        o0 += red_o[w][hq][d] * a;
+        o1 += red_o[w][hq][d + 1] * a;
+      }
+      float* st = rs.state + ((size_t)blockIdx.x * G + hq) * kPartFloats;
+      part_store2(st + 2 + d, o0, o1);
+      if (d == 0) part_store2(st, mx, l);
     }
-    // a row with no selected block (request not resident) attends to nothing: 0
-    out[((size_t)rl * g.Hq + (size_t)h * G + hq) * D + d] = l > 0.0f ? o / l : 0.0f;
+    if (last_part(rs, wrow, &seen))  // workgroup-uniform
+      merge_row<G>(rs, wrow, fac, out + ((size_t)rl * g.Hq + (size_t)h * G) * D);
+  } else {
+    for (int t = threadIdx.x; t < G * D; t += blockDim.x) {
+      const int hq = t / D, d = t % D;
+      float mx = red_ml[0][hq][0];
+      for (int w = 1; w < W; ++w) mx = fmaxf(mx, red_ml[w][hq][0]);
+      float l = 0.0f, o = 0.0f;
+      for (int w = 0; w < W; ++w) {
+        const float a = exp2_fast(red_ml[w][hq][0] - mx);
+        l += red_ml[w][hq][1] * a;
+        o += red_o[w][hq][d] * a;
+      }
+      // a row with no selected block (request not resident) attends to nothing: 0
+      out[((size_t)rl * g.Hq + (size_t)h * G + hq) * D + d] = l > 0.0f ? o / l : 0.0f;
+    }
   }
 }
 
-#define FERRY_ATTN_MFMA_INST(DT, G, W)                                                     \
-  template __global__ void k_attn_mfma<DT, G, W, false>(Geo, const float*, const uint32_t*,   \
-                                                        const uint8_t*, const float*, float*,  \
-                                                        float, int, int, int*);                \
-  template __global__ void k_attn_mfma<DT, G, W, true>(Geo, const float*, const uint32_t*,    \
-                                                       const uint8_t*, const float*, float*,   \
-                                                       float, int, int, int*);
+#define FERRY_ATTN_MFMA_INST_S(DT, G, W, NT, SPLIT)                                            \
+  template __global__ void k_attn_mfma<DT, G, W, NT, SPLIT>(Geo, const float*, const uint32_t*, \
+                                                            const uint8_t*, const float*,        \
+                                                            float*, float, int, int, int*, RowSplit);
+#define FERRY_ATTN_MFMA_INST(DT, G, W)             \
+  FERRY_ATTN_MFMA_INST_S(DT, G, W, false, false)   \
+  FERRY_ATTN_MFMA_INST_S(DT, G, W, true, false)    \
+  FERRY_ATTN_MFMA_INST_S(DT, G, W, false, true)    \
+  FERRY_ATTN_MFMA_INST_S(DT, G, W, true, true)
 #define FERRY_ATTN_MFMA_INST_G(DT, W) \
   FERRY_ATTN_MFMA_INST(DT, 2, W)      \
   FERRY_ATTN_MFMA_INST(DT, 4, W)      \

@@ -1,6 +1,7 @@
 // kernels.hpp -- device data structures and kernel declarations.
 #pragma once
 
+#include "attn_common.hpp"
 #include "common.hpp"
 
 namespace ferry_amd {
@@ -109,16 +110,18 @@ __global__ void k_step_close(unsigned long long* acc, unsigned long long* host);
 
 // Vector-ALU attention (attn.hip); W wavefronts per workgroup; NT selects
 // non-temporal K/V loads.
-template <int DT, int G, int W, bool NT>
+// SPLIT: a row's blocks are shared by rs.parts workgroups (attn_common.hpp).
+template <int DT, int G, int W, bool NT, bool SPLIT>
 __global__ void k_attn(Geo g, const float* q, const uint32_t* slots, const uint8_t* pool,
-                       const float* pool_scales, float* out, float qscale, int l0, int nl, int* err);
+                       const float* pool_scales, float* out, float qscale, int l0, int nl, int* err,
+                       RowSplit rs);
 
 // MFMA variant for GQA groups (G >= 2) of 16/8-bit KV (attn_mfma.hip); W
-// wavefronts per workgroup; NT as for k_attn.
-template <int DT, int G, int W, bool NT>
+// wavefronts per workgroup; NT and SPLIT as for k_attn.
+template <int DT, int G, int W, bool NT, bool SPLIT>
 __global__ void k_attn_mfma(Geo g, const float* q, const uint32_t* slots, const uint8_t* pool,
                             const float* pool_scales, float* out, float qscale, int l0, int nl,
-                            int* err);
+                            int* err, RowSplit rs);
 
 // Prefix-group attention (attn_group.hip): one workgroup of W wavefronts per
 // (group, layer, kv head), with SPLIT per `mpw` of its members, reads each

@@ -91,6 +91,9 @@ int resolve_scratch(int device, float** out) {
 }
 }  // namespace
 
+// Streams of a context that each have row-split state of their own.
+constexpr int kSplitStreams = 4;
+
 struct ferry_ctx {
   ferry_config cfg{};
   int device = 0;
@@ -156,6 +159,11 @@ struct ferry_ctx {
   float* scratch_dev = nullptr;    // this device's address of the static `scratch` array
   uint32_t* lane_live = nullptr;   // [n_req] 1 while the lane's request is a resident member
   uint32_t* trim_gen = nullptr;    // [n_owners] last ferry_members_leave that shrank the owner
+  float* split_state = nullptr;    // [kSplitStreams][2 CUs][G][kPartFloats] softmax states of split rows
+  uint32_t* split_count = nullptr;  // [kSplitStreams][CUs] finished parts of each row, 0 between launches
+  std::mutex split_mu;             // guards the two below
+  hipStream_t split_stream[kSplitStreams] = {};
+  int split_used = 0;
   uint32_t member_calls = 0;       // ferry_members_leave calls so far (trim generations)
 
   Ring ring(int which = 0) const {
@@ -242,7 +250,8 @@ void release(ferry_ctx* c) {
                  c->ring_entries, c->ring_state, c->ring_entries2, c->ring_state2,
                  c->ring_seg, c->ring_cap, c->worker_of_set,
                  c->stats, c->sel_counts, c->step_acc, c->done, c->err, c->probe_sink,
-                 c->probe_dst, c->sums, c->sum_scales, c->ktab, c->ktab_scales, c->mass_ws};
+                 c->probe_dst, c->sums, c->sum_scales, c->ktab, c->ktab_scales, c->mass_ws,
+                 c->split_state, c->split_count};
   for (void* p : dev)
     if (p) (void)hipFree(p);
   if (c->pend_host) (void)hipHostFree(c->pend_host);
@@ -268,6 +277,12 @@ uint32_t spread_hash(uint32_t x) {
   return x;
 }
 
+// One stream's split-row states: a launch has at most two workgroups per CU
+// (row_parts).
+size_t split_state_floats(const ferry_ctx* c) {
+  return (size_t)2 * c->cus * (size_t)(c->g.Hq / c->g.Hkv) * kPartFloats;
+}
+
 int check_ctx(const ferry_ctx* c) { return c ? FERRY_OK : fail(FERRY_EINVAL, "null context"); }
 
 }  // namespace
@@ -285,6 +300,7 @@ struct AttnArgs {
   int l0, nl;
   int* err;
   unsigned long long* attn_blocks;  // the group kernel adds the blocks it read (or null)
+  RowSplit rs;                      // workgroups per row of the per-row kernels, and their states
 };
 
 // Which attention kernel runs and how many wavefronts share one (request,
@@ -324,24 +340,27 @@ AttnPlan attn_plan(const ferry_ctx* ctx) {
   return p;
 }
 
+#define FERRY_ROW_LAUNCH(KERNEL, NT)                                                                \
+  do {                                                                                              \
+    if (a.rs.parts > 1)                                                                             \
+      hipLaunchKernelGGL((KERNEL<DT, G, W, NT, true>), dim3(grid.x * (unsigned)a.rs.parts),         \
+                         dim3(W * 64), 0, s, a.g, a.q, a.slots, a.pool, a.pool_scales, a.out,       \
+                         a.qscale, a.l0, a.nl, a.err, a.rs);                                        \
+    else                                                                                            \
+      hipLaunchKernelGGL((KERNEL<DT, G, W, NT, false>), grid, dim3(W * 64), 0, s, a.g, a.q,         \
+                         a.slots, a.pool, a.pool_scales, a.out, a.qscale, a.l0, a.nl, a.err, a.rs); \
+  } while (0)
 template <int DT, int G, int W>
 void launch_valu(const AttnPlan& p, const dim3& grid, hipStream_t s, const AttnArgs& a) {
-  if (p.nt)
-    hipLaunchKernelGGL((k_attn<DT, G, W, true>), grid, dim3(W * 64), 0, s, a.g, a.q, a.slots,
-                       a.pool, a.pool_scales, a.out, a.qscale, a.l0, a.nl, a.err);
-  else
-    hipLaunchKernelGGL((k_attn<DT, G, W, false>), grid, dim3(W * 64), 0, s, a.g, a.q, a.slots,
-                       a.pool, a.pool_scales, a.out, a.qscale, a.l0, a.nl, a.err);
+  if (p.nt) FERRY_ROW_LAUNCH(k_attn, true);
+  else FERRY_ROW_LAUNCH(k_attn, false);
 }
 template <int DT, int G, int W>
 void launch_mfma(const AttnPlan& p, const dim3& grid, hipStream_t s, const AttnArgs& a) {
-  if (p.nt)
-    hipLaunchKernelGGL((k_attn_mfma<DT, G, W, true>), grid, dim3(W * 64), 0, s, a.g, a.q,
-                       a.slots, a.pool, a.pool_scales, a.out, a.qscale, a.l0, a.nl, a.err);
-  else
-    hipLaunchKernelGGL((k_attn_mfma<DT, G, W, false>), grid, dim3(W * 64), 0, s, a.g, a.q,
-                       a.slots, a.pool, a.pool_scales, a.out, a.qscale, a.l0, a.nl, a.err);
+  if (p.nt) FERRY_ROW_LAUNCH(k_attn_mfma, true);
+  else FERRY_ROW_LAUNCH(k_attn_mfma, false);
 }
+#undef FERRY_ROW_LAUNCH
 // Query tiles per workgroup of a prefix-group launch: the fewest for which the
 // launch still has no more workgroups than the GPU has CUs, else all of the
 // set's.  A set of several tiles costs a workgroup their arithmetic one after
@@ -480,6 +499,46 @@ int check_bufs(std::initializer_list<std::pair<const void*, const char*>> bufs) 
   return FERRY_OK;
 }
 
+// Workgroups per row of a per-row attention launch.  A CU takes in some
+// 40-60 GB/s of blocks whatever its wavefronts keep in flight (8 wavefronts or
+// rings of 4 to 8 blocks measured the same), so a launch of few rows is bound
+// by its CUs: a row is split between as many workgroups as put one on every
+// CU, and between three where that is one but three put two on most (rows in
+// (CUs / 2, 2 CUs / 3]).  More, or more rows, only add to the merge.  A part's
+// wavefronts have two blocks each, and a row at most kMaxParts parts, past
+// which the merge takes what the shorter parts give.  us per launch, whole
+// rows / split, bf16, 4 query heads, k 128: 8 rows 22.8 / 10.4 (8 parts; 12:
+// 10.7), 64 rows 32.7 / 17.0 (4), 128 rows 39.9 / 27.1 (2; 4: 27.1), 160 rows
+// 40.7 / 33.2 (3; 2: 40.1), 192 rows 40.5 / 44.1 (2); fp32, 1 head, k 32:
+// 8 rows 10.5 / 7.6 (4), 128 rows 16.5 / 13.8 (2).
+int row_parts(long rows, int k, int waves, int cus) {
+  const long p = rows * 2 <= cus ? cus / rows : rows * 3 <= 2l * cus ? 3 : 1;
+  return (int)std::max<long>(1, std::min<long>(std::min<long>(p, kMaxParts), k / (2 * waves)));
+}
+
+// A stream's index among the first kSplitStreams streams that launched split
+// rows on this context; -1 (the launch then runs unsplit) for further streams,
+// for a stream being captured (a graph may be replayed on any stream) and for
+// the per-thread default stream (one handle, a stream per thread).  Streams
+// are told apart by handle: hipStreamDestroy returns once the stream's work is
+// done (measured: 42 ms behind a 42 ms kernel), so a handle that comes back
+// for a new stream has nothing of the old one in flight.
+int stream_slot(ferry_ctx* ctx, hipStream_t s) {
+  if (s == hipStreamPerThread) return -1;
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &cap) != hipSuccess) {
+    (void)hipGetLastError();
+    return -1;
+  }
+  if (cap != hipStreamCaptureStatusNone) return -1;
+  std::lock_guard<std::mutex> lk(ctx->split_mu);
+  for (int i = 0; i < ctx->split_used; ++i)
+    if (ctx->split_stream[i] == s) return i;
+  if (ctx->split_used == kSplitStreams) return -1;
+  ctx->split_stream[ctx->split_used] = s;
+  return ctx->split_used++;
+}
+
 // Attention of layers [l0, l0 + nl).  attn_blocks (decode steps only): the
 // prefix-group kernel adds the distinct blocks it reads there, which the next
 // step's layer chunking takes as the attention's bytes.
@@ -491,9 +550,18 @@ int decode_layers(ferry_ctx* ctx, int32_t l0, int32_t nl, const float* q, const 
   HIPC(hipSetDevice(ctx->device));
   const dim3 grid((unsigned)(g.n_req * nl * g.Hkv));
   const float qscale = (float)(1.4426950408889634 / std::sqrt((double)g.D));
-  const AttnArgs a{g, q, slots, ctx->pool, ctx->pool_scales, out, qscale, l0, nl, ctx->err,
-                   attn_blocks};
+  AttnArgs a{g, q, slots, ctx->pool, ctx->pool_scales, out, qscale, l0, nl, ctx->err,
+             attn_blocks, RowSplit{nullptr, nullptr, 1}};
   const AttnPlan p = attn_plan(ctx);
+  if (!p.grouped) {
+    const int parts = row_parts((long)grid.x, g.k, p.waves, p.cus);
+    if (parts > 1) {
+      const int slot = stream_slot(ctx, (hipStream_t)stream);
+      if (slot >= 0)
+        a.rs = RowSplit{ctx->split_state + (size_t)slot * split_state_floats(ctx),
+                        ctx->split_count + (size_t)slot * (size_t)ctx->cus, parts};
+    }
+  }
   launch_attn(p, grid, (hipStream_t)stream, a);
   HIPC(hipGetLastError());
   return FERRY_OK;
@@ -672,6 +740,8 @@ int ferry_ctx_create(const ferry_config* cfg, int device, ferry_ctx** out) {
   TRY(dalloc(&c->step_acc, 3));
   TRY(dalloc(&c->done, 1));
   TRY(dalloc(&c->err, 1));
+  TRY(dalloc(&c->split_state, kSplitStreams * split_state_floats(c)));
+  TRY(dalloc(&c->split_count, (size_t)kSplitStreams * c->cus));
 #define HIPT(x)                                                                        \
   do {                                                                                 \
     hipError_t e_ = (x);                                                               \
@@ -697,6 +767,7 @@ int ferry_ctx_create(const ferry_config* cfg, int device, ferry_ctx** out) {
   HIPT(hipHostGetDevicePointer((void**)&c->pend_dev, c->pend_host, 0));
   HIPT(hipMemset(c->done, 0, 4));
   HIPT(hipMemset(c->err, 0, 4));
+  HIPT(hipMemset(c->split_count, 0, (size_t)kSplitStreams * c->cus * 4));
   HIPT(hipMemset(c->pool, 0, nslots * g.bb));
   // pinned host tier, mapped into the device address space
   const size_t hbytes = (size_t)g.host_blocks * g.bb;

@@ -268,7 +268,7 @@ int ferry_sparse_decode(ferry_ctx* ctx, const float* q, const uint32_t* slots,
                         float* out, void* stream);
 
 /* Which attention kernel ferry_sparse_decode runs for this context:
- * *kind = FERRY_ATTN_VALU, FERRY_ATTN_MFMA (one workgroup per request row) or
+ * *kind = FERRY_ATTN_VALU, FERRY_ATTN_MFMA (workgroups of one request row) or
  * FERRY_ATTN_GROUP (one per prefix-group set), *waves = wavefronts per
  * workgroup of ferry_sparse_decode's launch over all L layers.  The
  * prefix-group kernel runs eight on a launch of no more group sets than the
@@ -278,7 +278,10 @@ int ferry_sparse_decode(ferry_ctx* ctx, const float* q, const uint32_t* slots,
  * one proxy kernel); for callers that report rooflines per kernel. */
 int ferry_attn_kernel(const ferry_ctx* ctx, int32_t* kind, int32_t* waves);
 
-/* Attention of layers [l0, l0 + nl) only. */
+/* Attention of layers [l0, l0 + nl) only.  A launch of few rows shares each
+ * row between several workgroups, which meet in memory that the context keeps
+ * for the stream (the first four streams that launch such rows; on others, and
+ * while a stream is being captured, a row has one workgroup). */
 int ferry_sparse_decode_layers(ferry_ctx* ctx, int32_t l0, int32_t nl, const float* q,
                                const uint32_t* slots, float* out, void* stream);
 

@@ -1,0 +1,94 @@
+"""Attention launches of few rows share each row between several workgroups,
+which meet in per-stream memory: parity with the oracle at the row counts where
+the number of workgroups changes, on ragged and empty rows, and the same
+result from concurrent streams, repeated launches and a captured graph."""
+import numpy as np
+import pytest
+import torch
+
+import ferry_amd as F
+from oracle import pyoracle as O
+
+from test_gpu_parity import TOL, Pair, _zipf_stream
+
+pytestmark = pytest.mark.gpu
+
+
+def _rel(a, b):
+    den = np.maximum(np.abs(b).max(axis=-1), 1e-30)
+    return (np.abs(a - b).max(axis=-1) / den).max()
+
+
+@pytest.mark.parametrize("dtype,Hkv,Hq,n_req,k", [
+    (F.F32, 1, 1, 1, 16),      # one row, 2 workgroups (256 CUs)
+    (F.BF16, 2, 8, 4, 67),     # 8 rows, 8 workgroups, the wavefronts' shares uneven
+    (F.FP8, 1, 8, 33, 33),     # 33 rows, 4 workgroups
+    (F.F16, 2, 2, 43, 24),     # 86 rows, 2 (vector ALUs)
+    (F.F16, 2, 4, 64, 40),     # 128 rows, 2
+    (F.F32, 2, 4, 65, 25),     # 130 rows, 3
+    (F.BF16, 2, 16, 85, 24),   # 170 rows, 3
+    (F.FP8, 3, 3, 57, 30),     # 171 rows, 1
+])
+def test_row_split_parity(dtype, Hkv, Hq, n_req, k):
+    mb, sels = _zipf_stream(n_req, 1, Hkv, k, 80, 160, 1, seed=k)
+    sel = np.array(sels[0], np.uint32).reshape(n_req, 1, Hkv, k).copy()
+    for r in range(n_req):  # ragged rows: whole, one block, none, holes
+        if r % 4 == 1:
+            sel[r, :, :, 1:] = F.EMPTY
+        elif r % 4 == 2:
+            sel[r] = F.EMPTY
+        elif r % 4 == 3:
+            sel[r, :, :, ::3] = F.EMPTY
+    p = Pair(n_req, 1, Hkv, Hq, k, 2 * k, mb, dtype)
+    p.step(sel.reshape(-1))
+    q = np.random.default_rng(k).standard_normal((n_req, 1, Hq, 128)).astype(np.float32)
+    dq = torch.from_numpy(q).cuda()
+    out, again = torch.full_like(dq, 7.0), torch.full_like(dq, -7.0)
+    p.ex.sparse_decode(dq, p.bufs["slots"], out)
+    p.ex.sparse_decode(dq, p.bufs["slots"], again)
+    torch.cuda.synchronize()
+    got = out.cpu().numpy().reshape(-1, 128).astype(np.float64)
+    ref = O.attention_f64(p.g, sel.reshape(-1), q).reshape(-1, 128)
+    none = np.repeat(np.all(sel == F.EMPTY, axis=-1).reshape(-1), Hq // Hkv)
+    assert np.all(got[none] == 0.0)
+    if not none.all():
+        assert _rel(got[~none], ref[~none]) < TOL[dtype]
+    assert torch.equal(out, again)  # parts are merged in part order
+    assert p.ex.stats()["device_error"] == 0
+
+
+def test_row_split_streams_and_graphs():
+    """Six streams at once on one context (four have split state, the others
+    run whole rows), each with queries and outputs of its own, and a graph
+    captured from one of them replayed between eager launches."""
+    n_req, Hkv, Hq, k = 8, 2, 8, 64
+    mb, sels = _zipf_stream(n_req, 1, Hkv, k, 80, 160, 1, seed=3)
+    p = Pair(n_req, 1, Hkv, Hq, k, 2 * k, mb, F.BF16)
+    p.step(sels[0])
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in range(6)]
+    qs = [torch.randn((n_req, 1, Hq, 128), device="cuda") for _ in streams]
+    outs = [torch.zeros_like(q) for q in qs]
+    torch.cuda.synchronize()
+    for _ in range(20):
+        for s, q, o in zip(streams, qs, outs):
+            p.ex.sparse_decode(q, p.bufs["slots"], o, stream=s)
+    torch.cuda.synchronize()
+    refs = [O.attention_f64(p.g, sels[0], q.cpu().numpy()).reshape(-1, 128) for q in qs]
+    for o, ref in zip(outs, refs):
+        assert _rel(o.cpu().numpy().reshape(-1, 128), ref) < TOL[F.BF16]
+    first = outs[0].clone()
+    g = torch.cuda.CUDAGraph()
+    gout = torch.zeros_like(qs[1])
+    with torch.cuda.graph(g, stream=streams[0]):
+        p.ex.sparse_decode(qs[1], p.bufs["slots"], gout, stream=streams[0])
+    for _ in range(3):
+        gout.zero_()
+        outs[0].zero_()
+        torch.cuda.synchronize()
+        g.replay()
+        p.ex.sparse_decode(qs[0], p.bufs["slots"], outs[0], stream=streams[0])
+        torch.cuda.synchronize()
+        assert _rel(gout.cpu().numpy().reshape(-1, 128), refs[1]) < TOL[F.BF16]
+        assert torch.equal(outs[0], first)
+    assert p.ex.stats()["device_error"] == 0
