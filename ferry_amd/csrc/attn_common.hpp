@@ -158,17 +158,18 @@ __device__ inline float2 part_load2(const float* p) {
   return float2{__builtin_bit_cast(float, (uint32_t)v), __builtin_bit_cast(float, (uint32_t)(v >> 32))};
 }
 
-// Every thread of the workgroup calls it after its part_stores: true in every
-// thread of the row's last workgroup, whose part_loads then read every state.
-// `sh` is an LDS word.
-__device__ inline bool last_part(const RowSplit& rs, int row, uint32_t* sh) {
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wavefront's states have landed
+// Every thread of the workgroup calls it after its agent-scope stores: true in
+// every thread of the last of a row's `parts` workgroups, whose agent-scope
+// loads then read what all of them stored.  `count` is the row's word, `sh` an
+// LDS word.
+__device__ inline bool last_part(int parts, uint32_t* count, uint32_t* sh) {
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wavefront's stores have landed
   __syncthreads();
   if (threadIdx.x == 0)
-    *sh = __hip_atomic_fetch_add(rs.count + row, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    *sh = __hip_atomic_fetch_add(count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   __syncthreads();
-  const bool last = *sh == (uint32_t)rs.parts - 1u;
-  if (last && threadIdx.x == 0) astore(rs.count + row, 0u);
+  const bool last = *sh == (uint32_t)parts - 1u;
+  if (last && threadIdx.x == 0) astore(count, 0u);
   return last;
 }
 

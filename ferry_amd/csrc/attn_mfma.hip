@@ -172,7 +172,7 @@ __global__ __launch_bounds__(W * 64) void k_attn_mfma(Geo g, const float* __rest
       part_store2(st + 2 + d, o0, o1);
       if (d == 0) part_store2(st, mx, l);
     }
-    if (last_part(rs, wrow, &seen))  // workgroup-uniform
+    if (last_part(rs.parts, rs.count + wrow, &seen))  // workgroup-uniform
       merge_row<G>(rs, wrow, fac, out + ((size_t)rl * g.Hq + (size_t)h * G) * D);
   } else {
     for (int t = threadIdx.x; t < G * D; t += blockDim.x) {

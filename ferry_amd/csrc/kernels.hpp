@@ -224,10 +224,14 @@ __global__ void k_summaries_build(Geo g, const uint8_t* host, const float* host_
                                   float* sum_scales);
 __global__ void k_summaries_tile(uint8_t* sums, float* scales, uint64_t host_blocks, uint64_t total,
                                  uint32_t rec);
-template <int DT, int G, bool LAYER, int W>
+// Passes of 4 blocks per wavefront in flight in the Quest scoring, and the
+// blocks a workgroup of 16 wavefronts scores in them.
+constexpr int select_inflight(int G) { return G >= 8 ? 2 : 4; }
+constexpr int select_pass(int G) { return 4 * 16 * select_inflight(G); }
+template <int DT, int G, bool LAYER, int W, bool SPLIT>
 __global__ void k_select_topk(Geo g, const float* q, const int32_t* ctx_blocks, const uint8_t* sums,
                               const float* sum_scales, uint64_t sum_mod, uint32_t* sel, int l0, int nl,
-                              int max_n, int* err);
+                              int max_n, int* err, int parts, uint32_t* row_keys, uint32_t* row_count);
 
 // Mass method of the top-k selection (select.hip): the dense K table, the
 // softmax-mass scoring and the radix top-k of each (request, layer).

@@ -150,6 +150,7 @@ struct ferry_ctx {
   size_t probe_dst_bytes = 0;
   uint8_t* sums = nullptr;         // top-k selection: K min/max records [sum_blocks][2][D]
   float* sum_scales = nullptr;     // ... and their K scales (fp8)
+  uint32_t* sel_keys = nullptr;    // [kSplitStreams][split rows][max_blocks] keys of split rows
   uint64_t sum_blocks = 0;         // records; block (set, b) uses (set*max_blocks + b) mod this
   uint8_t* ktab = nullptr;         // mass selection: K halves of host blocks [kt_records][T][D]
   float* ktab_scales = nullptr;    // ... and their K scales (fp8)
@@ -251,7 +252,7 @@ void release(ferry_ctx* c) {
                  c->ring_seg, c->ring_cap, c->worker_of_set,
                  c->stats, c->sel_counts, c->step_acc, c->done, c->err, c->probe_sink,
                  c->probe_dst, c->sums, c->sum_scales, c->ktab, c->ktab_scales, c->mass_ws,
-                 c->split_state, c->split_count};
+                 c->split_state, c->split_count, c->sel_keys};
   for (void* p : dev)
     if (p) (void)hipFree(p);
   if (c->pend_host) (void)hipHostFree(c->pend_host);
@@ -537,6 +538,29 @@ int stream_slot(ferry_ctx* ctx, hipStream_t s) {
   if (ctx->split_used == kSplitStreams) return -1;
   ctx->split_stream[ctx->split_used] = s;
   return ctx->split_used++;
+}
+
+// Rows of a Quest selection launch that may be split between workgroups.
+uint64_t select_split_rows(const ferry_ctx* ctx) {
+  const Geo& g = ctx->g;
+  return std::min<uint64_t>((uint64_t)g.n_req * g.L * g.Hkv, (uint64_t)ctx->cus / 2);
+}
+
+// Workgroups (of 16 wavefronts) per row of a launch over `rows` rows of `heads`
+// query heads each: as many as put one on every CU, each with at least one
+// pass of its wavefronts (select_pass blocks); 1 for rows that score in less
+// than the keys' way through memory takes (2 us: under 2048 bounds).  As in the
+// attention, only more CUs take in a row's records faster.  us per launch,
+// whole rows (of 16 wavefronts) / split, 8192 blocks: bf16, 4 heads: 8 rows
+// 109 / 23, 64 rows 121 / 65, 128 rows 129 / 106; fp8, 8 heads: 8 rows
+// 421 / 35, 128 rows 478 / 261; 2048 blocks: fp16, 1 head, 32 rows 21 / 14;
+// 512 blocks: bf16, 4 heads, 64 rows 14.8 / 13.7, fp16, 1 head, 32 rows
+// 10.3 / 10.7 (so left whole).
+int select_parts(const ferry_ctx* ctx, unsigned rows, int heads) {
+  const unsigned mb = (unsigned)ctx->g.max_blocks, cus = (unsigned)ctx->cus;
+  if (rows > select_split_rows(ctx) || mb * (unsigned)heads < 2048u) return 1;
+  const unsigned pass = (unsigned)select_pass(ctx->g.Hq / ctx->g.Hkv);
+  return (int)std::max(1u, std::min(cus / rows, (mb + pass - 1) / pass));
 }
 
 // Attention of layers [l0, l0 + nl).  attn_blocks (decode steps only): the
@@ -1267,6 +1291,13 @@ int ferry_summaries_build(ferry_ctx* ctx, uint64_t n_records, void* stream) {
       return rc;
     ctx->sum_blocks = S;
   }
+  if (!ctx->sel_keys && g.group == 1 && (uint64_t)g.max_blocks * 4 <= 65536) {  // what select_topk takes
+    const uint64_t words = kSplitStreams * select_split_rows(ctx) * (uint64_t)g.max_blocks;
+    if (hipMalloc(&ctx->sel_keys, words * 4) != hipSuccess) {  // selections then run unsplit
+      (void)hipGetLastError();
+      ctx->sel_keys = nullptr;
+    }
+  }
   const unsigned blocks = (unsigned)std::min<uint64_t>((g.host_blocks + 3) / 4, 16384);
   hipStream_t s = (hipStream_t)stream;
   switch (g.dtype) {
@@ -1318,6 +1349,9 @@ struct SelArgs {
   int l0, nl, max_n;
   int* err;
   int cus;
+  int parts;            // workgroups per row
+  uint32_t* row_keys;   // the stream's keys and counts of split rows
+  uint32_t* row_count;
 };
 
 // Wavefronts of a Quest selection workgroup (one row each).  A launch of no
@@ -1335,13 +1369,18 @@ int select_waves(unsigned rows, int cus) {
 
 template <int DT, int G, bool LAYER>
 void launch_sel(const dim3& grid, size_t lds, hipStream_t s, const SelArgs& a) {
-#define FERRY_SEL_LAUNCH(W)                                                                         \
-  hipLaunchKernelGGL((k_select_topk<DT, G, LAYER, W>), grid, dim3(64 * W), lds, s, a.g, a.q,         \
-                     a.ctx_blocks, a.sums, a.sum_scales, a.sum_mod, a.sel, a.l0, a.nl, a.max_n, a.err)
+#define FERRY_SEL_LAUNCH(W, SPLIT)                                                                  \
+  hipLaunchKernelGGL((k_select_topk<DT, G, LAYER, W, SPLIT>), dim3(grid.x * (unsigned)a.parts),      \
+                     dim3(64 * W), lds, s, a.g, a.q, a.ctx_blocks, a.sums, a.sum_scales, a.sum_mod,  \
+                     a.sel, a.l0, a.nl, a.max_n, a.err, a.parts, a.row_keys, a.row_count)
+  if (a.parts > 1) {
+    FERRY_SEL_LAUNCH(16, true);
+    return;
+  }
   switch (select_waves(grid.x, a.cus)) {
-    case 16: FERRY_SEL_LAUNCH(16); return;
-    case 8: FERRY_SEL_LAUNCH(8); return;
-    default: FERRY_SEL_LAUNCH(4); return;
+    case 16: FERRY_SEL_LAUNCH(16, false); return;
+    case 8: FERRY_SEL_LAUNCH(8, false); return;
+    default: FERRY_SEL_LAUNCH(4, false); return;
   }
 #undef FERRY_SEL_LAUNCH
 }
@@ -1389,9 +1428,18 @@ int ferry_select_topk_layers(ferry_ctx* ctx, int32_t l0, int32_t nl, const float
                               "of LDS");
   HIPC(hipSetDevice(ctx->device));
   const dim3 grid((unsigned)((size_t)g.n_req * nl * (layer ? 1 : g.Hkv)));
-  const SelArgs a{g,   q,   ctx_blocks,    ctx->sums, ctx->sum_scales, ctx->sum_blocks,
-                  sel, l0,  nl,            g.max_blocks, ctx->err,
-                  ctx->cus};
+  SelArgs a{g,   q,   ctx_blocks,    ctx->sums, ctx->sum_scales, ctx->sum_blocks,
+            sel, l0,  nl,            g.max_blocks, ctx->err,
+            ctx->cus, 1, nullptr, nullptr};
+  const int parts = ctx->sel_keys ? select_parts(ctx, grid.x, Gq) : 1;
+  if (parts > 1) {
+    const int slot = stream_slot(ctx, (hipStream_t)stream);
+    if (slot >= 0) {
+      a.parts = parts;
+      a.row_keys = ctx->sel_keys + (size_t)slot * select_split_rows(ctx) * g.max_blocks;
+      a.row_count = ctx->split_count + (size_t)slot * (size_t)ctx->cus;
+    }
+  }
   if (layer)
     launch_sel_dt<true>(g.dtype, G, grid, lds, (hipStream_t)stream, a);
   else

@@ -350,14 +350,21 @@ __device__ void topk_ascending(const uint32_t* keys, int n, int kk, uint32_t* hi
 // largest key by at most 4 radix passes of 8 bits; phase 3 writes the
 // selected block ids in ascending order (ties to lower ids).
 // Dynamic LDS: q[Gq][128] floats, then keys[max_n].
-template <int DT, int G, bool LAYER, int W>
+// SPLIT (launches of few rows, select_parts()): a row's blocks are scored by
+// `parts` workgroups, which leave the keys in row_keys[row][max_n] and count
+// themselves in row_count (both the stream's own, through agent-scope atomics,
+// as RowSplit's states are); the last of them takes the top k.  The keys are
+// the same, so is the selection.
+template <int DT, int G, bool LAYER, int W, bool SPLIT>
 __global__ __launch_bounds__(W * 64) void k_select_topk(Geo g, const float* __restrict__ q,
                                                         const int32_t* __restrict__ ctx_blocks,
                                                         const uint8_t* __restrict__ sums,
                                                         const float* __restrict__ sum_scales,
                                                         uint64_t sum_mod, uint32_t* __restrict__ sel,
                                                         int l0, int nl, int max_n,
-                                                        int* __restrict__ err) {
+                                                        int* __restrict__ err, int parts,
+                                                        uint32_t* __restrict__ row_keys,
+                                                        uint32_t* __restrict__ row_count) {
   constexpr int ES = DT == FERRY_F32 ? 4 : (DT == FERRY_FP8_E4M3 ? 1 : 2);
   constexpr int D = 128, NT = W * 64;
   constexpr uint32_t REC = 2 * D * ES;  // summary bytes per block
@@ -371,8 +378,10 @@ __global__ __launch_bounds__(W * 64) void k_select_topk(Geo g, const float* __re
   float* qs = reinterpret_cast<float*>(lds);
   uint32_t* keys = lds + Gq * D;
 
-  const int hrow = LAYER ? 0 : blockIdx.x % g.Hkv;
-  const int rl_idx = LAYER ? blockIdx.x : blockIdx.x / g.Hkv;  // (request, layer in range)
+  const int wrow = SPLIT ? blockIdx.x / parts : blockIdx.x;  // row of the launch
+  const int part = SPLIT ? blockIdx.x % parts : 0;
+  const int hrow = LAYER ? 0 : wrow % g.Hkv;
+  const int rl_idx = LAYER ? wrow : wrow / g.Hkv;  // (request, layer in range)
   const int r = rl_idx / nl, l = l0 + rl_idx % nl;
   const int rl = r * g.L + l;
   int n = ctx_blocks[r];
@@ -406,8 +415,8 @@ __global__ __launch_bounds__(W * 64) void k_select_topk(Geo g, const float* __re
     // U passes of 4 blocks per wavefront are loaded before any is scored: the
     // keys take most of the LDS at long contexts, so few workgroups share a
     // CU and each wavefront must keep several records in flight
-    constexpr int U = G >= 8 ? 2 : 4;
-    for (int b0 = 4 * wave; b0 < n; b0 += 4 * W * U) {
+    constexpr int U = select_inflight(G);
+    for (int b0 = 4 * (wave + W * U * part); b0 < n; b0 += 4 * W * U * (SPLIT ? parts : 1)) {
       float score[U];
       for (int hh = 0; hh < nkv; ++hh) {
         const int hk = LAYER ? hh : hrow;
@@ -448,15 +457,32 @@ __global__ __launch_bounds__(W * 64) void k_select_topk(Geo g, const float* __re
         const int b = b0 + 4 * W * u + grp;
         if (b < n && p == 0) {
           const uint32_t key = fkey(score[u]);
-          keys[b] = key;
-          atomicAdd(&hist[key >> 24], 1u);
+          if constexpr (SPLIT) {
+            astore(row_keys + (size_t)wrow * max_n + b, key);
+          } else {
+            keys[b] = key;
+            atomicAdd(&hist[key >> 24], 1u);
+          }
         }
       }
     }
+    if constexpr (SPLIT) {
+      if (!last_part(parts, row_count + wrow, sh)) return;  // workgroup-uniform
+      for (int i0 = tid; i0 < n; i0 += 4 * NT) {
+        uint32_t v[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          v[u] = aload(row_keys + (size_t)wrow * max_n + min(i0 + u * NT, n - 1));
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          if (i0 + u * NT < n) keys[i0 + u * NT] = v[u];
+      }
+    }
     __syncthreads();
-    topk_ascending<W, true>(keys, n, kk, hist, wtot, sh, out_row(LAYER ? 0 : hrow),
-                            LAYER ? g.Hkv : 1, (size_t)k);
+    topk_ascending<W, !SPLIT>(keys, n, kk, hist, wtot, sh, out_row(LAYER ? 0 : hrow),
+                              LAYER ? g.Hkv : 1, (size_t)k);
   } else {
+    if (part != 0) return;  // workgroup-uniform
     // a context of at most k blocks: every block, in order
     for (int j = tid; j < kk; j += NT)
       for (int hh = 0; hh < (LAYER ? g.Hkv : 1); ++hh) out_row(LAYER ? hh : hrow)[j] = (uint32_t)j;
@@ -1098,14 +1124,15 @@ FERRY_SUMS_INST(FERRY_F16)
 FERRY_SUMS_INST(FERRY_BF16)
 FERRY_SUMS_INST(FERRY_FP8_E4M3)
 
-#define FERRY_SEL_INST_W(DT, G, LAYER, W)                                                      \
-  template __global__ void k_select_topk<DT, G, LAYER, W>(Geo, const float*, const int32_t*,     \
-                                                          const uint8_t*, const float*, uint64_t,  \
-                                                          uint32_t*, int, int, int, int*);
-#define FERRY_SEL_INST(DT, G, LAYER) \
-  FERRY_SEL_INST_W(DT, G, LAYER, 4)  \
-  FERRY_SEL_INST_W(DT, G, LAYER, 8)  \
-  FERRY_SEL_INST_W(DT, G, LAYER, 16)
+#define FERRY_SEL_INST_W(DT, G, LAYER, W, SPLIT)                                                \
+  template __global__ void k_select_topk<DT, G, LAYER, W, SPLIT>(                                \
+      Geo, const float*, const int32_t*, const uint8_t*, const float*, uint64_t, uint32_t*, int, \
+      int, int, int*, int, uint32_t*, uint32_t*);
+#define FERRY_SEL_INST(DT, G, LAYER)        \
+  FERRY_SEL_INST_W(DT, G, LAYER, 4, false)  \
+  FERRY_SEL_INST_W(DT, G, LAYER, 8, false)  \
+  FERRY_SEL_INST_W(DT, G, LAYER, 16, false) \
+  FERRY_SEL_INST_W(DT, G, LAYER, 16, true)
 #define FERRY_SEL_INST_G(DT, LAYER) \
   FERRY_SEL_INST(DT, 1, LAYER)      \
   FERRY_SEL_INST(DT, 2, LAYER)      \

@@ -94,6 +94,49 @@ def test_select_workgroup_sizes_bit_exact(dtype, Hkv, Hq, mode, n_req):
     assert p.ex.stats()["device_error"] == 0
 
 
+@pytest.mark.parametrize("dtype,Hkv,Hq,mode,n_req", [
+    (F.BF16, 2, 8, F.TOPK_PER_HEAD, 13),    # 26 rows, 3 workgroups each (256 CUs)
+    (F.FP8, 1, 8, F.TOPK_PER_HEAD, 9),      # 9 rows, 6
+    (F.F32, 2, 8, F.TOPK_PER_HEAD, 64),     # 128 rows, 2
+    (F.F16, 2, 8, F.TOPK_LAYER_MAX, 13),    # 13 rows of all heads, 3
+])
+def test_select_split_rows_bit_exact(dtype, Hkv, Hq, mode, n_req):
+    """A launch of few rows shares each row's blocks between workgroups; the
+    contexts end inside, at and past a workgroup's share.  On three streams at
+    once, then in a graph (which is captured with whole rows)."""
+    k, mb = 12, 770
+    p = Pair(n_req, 1, Hkv, Hq, k, 16, mb, dtype, host_blocks=1031)
+    p.ex.summaries_build()
+    rng = np.random.default_rng(dtype + 5)
+    ctx = rng.choice([0, 12, 13, 127, 128, 129, 255, 256, 257, 512, 513, 768, 769, 770],
+                     n_req).astype(np.int32)
+    ctx[0] = mb
+    q = rng.standard_normal((n_req, 1, Hq, 128)).astype(np.float32)
+    dq, dctx = torch.from_numpy(q).cuda(), torch.from_numpy(ctx).cuda()
+    want = O.select_topk(p.g, q, ctx, mode)
+    streams = [torch.cuda.Stream() for _ in range(3)]
+    sels = [torch.full((n_req, 1, Hkv, k), -7, dtype=torch.int32, device="cuda") for _ in streams]
+    torch.cuda.synchronize()
+    for _ in range(5):
+        for s, sel in zip(streams, sels):
+            p.ex.select_topk(dq, dctx, sel, mode, stream=s)
+    torch.cuda.synchronize()
+    for sel in sels:
+        assert np.array_equal(sel.cpu().numpy().view(np.uint32), want)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=streams[0]):
+        p.ex.select_topk(dq, dctx, sels[0], mode, stream=streams[0])
+    for _ in range(3):
+        sels[0].fill_(-7)
+        torch.cuda.synchronize()
+        g.replay()
+        p.ex.select_topk(dq, dctx, sels[1], mode, stream=streams[0])
+        torch.cuda.synchronize()
+        assert np.array_equal(sels[0].cpu().numpy().view(np.uint32), want)
+        assert np.array_equal(sels[1].cpu().numpy().view(np.uint32), want)
+    assert p.ex.stats()["device_error"] == 0
+
+
 def test_one_record_per_block_gives_the_same_selection():
     """A table with a record per (set, block) (3x the host tier here) repeats
     the host-tier records and selects exactly what the small table does."""
