@@ -298,7 +298,7 @@ __global__ __launch_bounds__(W * 64) void k_attn(Geo g, const float* __restrict_
     __shared__ uint32_t seen;
     __shared__ float2 fac[G * kMaxParts];
     if (last_part(rs.parts, rs.count + wrow, &seen))  // workgroup-uniform
-      merge_row<G>(rs, wrow, fac, out + ((size_t)rl * g.Hq + (size_t)h * G) * D);
+      merge_row<G, W * 64>(rs, wrow, fac, out + ((size_t)rl * g.Hq + (size_t)h * G) * D);
   }
 }
 

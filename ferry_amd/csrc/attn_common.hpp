@@ -174,44 +174,49 @@ __device__ inline bool last_part(int parts, uint32_t* count, uint32_t* sh) {
 }
 
 // The row's G * 128 outputs from its parts' states, by every thread of the last
-// workgroup: the (max, sum) pairs go to `fac` (LDS, [G * kMaxParts]) with one
-// load in flight per thread, become each part's factor 2^(m_p - M) / L there,
-// and a thread then sums its pairs of outputs four parts at a time (loads in
-// flight together).  Read one part after the other, 16 parts of 8 heads took
-// 20 us.
-template <int G>
+// workgroup (NT threads).  Every load goes out first, the (max, sum) pairs and
+// the thread's own pairs of outputs, so the merge waits for memory once; the
+// pairs become each part's factor 2^(m_p - M) / L in `fac` (LDS,
+// [G * kMaxParts]).  (Read one part after the other, the states of 16 parts of
+// 8 heads took 20 us, four at a time behind the factors 3.)
+template <int G, int NT>
 __device__ inline void merge_row(const RowSplit& rs, int row, float2* fac, float* __restrict__ out) {
+  constexpr int NP = (G * 64 + NT - 1) / NT;  // pairs of outputs per thread
+  static_assert(G * kMaxParts <= NT, "a (max, sum) pair per thread");
   const float* st = rs.state + (size_t)row * rs.parts * G * kPartFloats;
-  const int np = rs.parts, nt = blockDim.x;
-  for (int t = threadIdx.x; t < G * np; t += nt) {  // t = part * G + head
-    fac[(t % G) * kMaxParts + t / G] = part_load2(st + (size_t)t * kPartFloats);
+  const int np = rs.parts, tid = threadIdx.x;
+  float2 ms = {0.0f, 0.0f}, v[NP][kMaxParts];
+  if (tid < G * np) ms = part_load2(st + (size_t)tid * kPartFloats);  // tid = part * G + head
+#pragma unroll
+  for (int i = 0; i < NP; ++i) {
+    const int t = min(tid + i * NT, G * 64 - 1);  // head * 64 + pair of dims
+#pragma unroll
+    for (int p = 0; p < kMaxParts; ++p)
+      v[i][p] = part_load2(st + ((size_t)min(p, np - 1) * G + (t >> 6)) * kPartFloats + 2 + 2 * (t & 63));
   }
+  if (tid < G * np) fac[(tid % G) * kMaxParts + tid / G] = ms;
   __syncthreads();
-  if (threadIdx.x < G) {
-    float2* f = fac + threadIdx.x * kMaxParts;
+  if (tid < G) {
+    float2* f = fac + tid * kMaxParts;
     float m = f[0].x, l = 0.0f;
     for (int p = 1; p < np; ++p) m = fmaxf(m, f[p].x);
     for (int p = 0; p < np; ++p) l += f[p].y * __builtin_amdgcn_exp2f(f[p].x - m);
     // a row with no selected block (request not resident) attends to nothing: 0
     const float inv = l > 0.0f ? 1.0f / l : 0.0f;
     for (int p = 0; p < np; ++p) f[p].y = __builtin_amdgcn_exp2f(f[p].x - m) * inv;
+    for (int p = np; p < kMaxParts; ++p) f[p].y = 0.0f;
   }
   __syncthreads();
-  for (int t = threadIdx.x; t < G * 64; t += nt) {  // t = head * 64 + pair of dims
-    const float* o = st + (size_t)(t >> 6) * kPartFloats + 2 + 2 * (t & 63);
-    const float2* f = fac + (t >> 6) * kMaxParts;
+#pragma unroll
+  for (int i = 0; i < NP; ++i) {
+    const int t = tid + i * NT;
+    if (t >= G * 64) break;
     float a = 0.0f, b = 0.0f;
-    for (int p0 = 0; p0 < np; p0 += 4) {
-      float2 v[4];
 #pragma unroll
-      for (int u = 0; u < 4; ++u)
-        v[u] = part_load2(o + (size_t)min(p0 + u, np - 1) * G * kPartFloats);
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const float w = p0 + u < np ? f[p0 + u].y : 0.0f;
-        a = __builtin_fmaf(v[u].x, w, a);
-        b = __builtin_fmaf(v[u].y, w, b);
-      }
+    for (int p = 0; p < kMaxParts; ++p) {
+      const float w = fac[(t >> 6) * kMaxParts + p].y;
+      a = __builtin_fmaf(v[i][p].x, w, a);
+      b = __builtin_fmaf(v[i][p].y, w, b);
     }
     *reinterpret_cast<float2*>(out + 2 * t) = float2{a, b};
   }

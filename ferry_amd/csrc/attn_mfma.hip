@@ -173,7 +173,7 @@ __global__ __launch_bounds__(W * 64) void k_attn_mfma(Geo g, const float* __rest
       if (d == 0) part_store2(st, mx, l);
     }
     if (last_part(rs.parts, rs.count + wrow, &seen))  // workgroup-uniform
-      merge_row<G>(rs, wrow, fac, out + ((size_t)rl * g.Hq + (size_t)h * G) * D);
+      merge_row<G, W * 64>(rs, wrow, fac, out + ((size_t)rl * g.Hq + (size_t)h * G) * D);
   } else {
     for (int t = threadIdx.x; t < G * D; t += blockDim.x) {
       const int hq = t / D, d = t % D;
