@@ -226,8 +226,8 @@ __global__ void k_summaries_tile(uint8_t* sums, float* scales, uint64_t host_blo
                                  uint32_t rec);
 // Passes of 4 blocks per wavefront in flight in the Quest scoring, and the
 // blocks a workgroup of 16 wavefronts scores in them.
-constexpr int select_inflight(int G) { return G >= 8 ? 2 : 4; }
-constexpr int select_pass(int G) { return 4 * 16 * select_inflight(G); }
+constexpr int kSelectInflight = 4;
+constexpr int kSelectPass = 4 * 16 * kSelectInflight;
 template <int DT, int G, bool LAYER, int W, bool SPLIT>
 __global__ void k_select_topk(Geo g, const float* q, const int32_t* ctx_blocks, const uint8_t* sums,
                               const float* sum_scales, uint64_t sum_mod, uint32_t* sel, int l0, int nl,

@@ -205,12 +205,9 @@ __global__ __launch_bounds__(256) void k_probe_sums(Geo g, const uint8_t* __rest
   if (lane == 0) sink[(size_t)blockIdx.x * W + wave] = x;
 }
 
-template __global__ void k_probe_sums<1, 2>(Geo, const uint8_t*, uint64_t, int, uint32_t*);
-template __global__ void k_probe_sums<1, 4>(Geo, const uint8_t*, uint64_t, int, uint32_t*);
-template __global__ void k_probe_sums<2, 2>(Geo, const uint8_t*, uint64_t, int, uint32_t*);
-template __global__ void k_probe_sums<2, 4>(Geo, const uint8_t*, uint64_t, int, uint32_t*);
-template __global__ void k_probe_sums<4, 2>(Geo, const uint8_t*, uint64_t, int, uint32_t*);
-template __global__ void k_probe_sums<4, 4>(Geo, const uint8_t*, uint64_t, int, uint32_t*);
+template __global__ void k_probe_sums<1, kSelectInflight>(Geo, const uint8_t*, uint64_t, int, uint32_t*);
+template __global__ void k_probe_sums<2, kSelectInflight>(Geo, const uint8_t*, uint64_t, int, uint32_t*);
+template __global__ void k_probe_sums<4, kSelectInflight>(Geo, const uint8_t*, uint64_t, int, uint32_t*);
 template __global__ void k_probe_ktab<2, kMassUnitWaves, kMassUnitInflight, 1>(Geo, const uint8_t*,
                                                                               uint64_t, int, uint32_t*);
 template __global__ void k_probe_ktab<4, kMassUnitWaves, kMassUnitInflight, 1>(Geo, const uint8_t*,

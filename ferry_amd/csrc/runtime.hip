@@ -508,10 +508,10 @@ int check_bufs(std::initializer_list<std::pair<const void*, const char*>> bufs) 
 // (CUs / 2, 2 CUs / 3]).  More, or more rows, only add to the merge.  A part's
 // wavefronts have two blocks each, and a row at most kMaxParts parts, past
 // which the merge takes what the shorter parts give.  us per launch, whole
-// rows / split, bf16, 4 query heads, k 128: 8 rows 22.8 / 10.4 (8 parts; 12:
-// 10.7), 64 rows 32.7 / 17.0 (4), 128 rows 39.9 / 27.1 (2; 4: 27.1), 160 rows
-// 40.7 / 33.2 (3; 2: 40.1), 192 rows 40.5 / 44.1 (2); fp32, 1 head, k 32:
-// 8 rows 10.5 / 7.6 (4), 128 rows 16.5 / 13.8 (2).
+// rows / split, bf16, 4 query heads, k 128: 8 rows 22.8 / 9.6 (8 parts), 64 rows
+// 32.7 / 16.7 (4), 128 rows 39.9 / 27.0 (2; 4 the same), 160 rows 40.7 / 33.0
+// (3; 2: 40.1), 192 rows 40.5 / 44.1 (2); fp32, 1 head, k 32: 8 rows 10.5 / 7.2
+// (4), 128 rows 16.5 / 13.7 (2).
 int row_parts(long rows, int k, int waves, int cus) {
   const long p = rows * 2 <= cus ? cus / rows : rows * 3 <= 2l * cus ? 3 : 1;
   return (int)std::max<long>(1, std::min<long>(std::min<long>(p, kMaxParts), k / (2 * waves)));
@@ -548,19 +548,17 @@ uint64_t select_split_rows(const ferry_ctx* ctx) {
 
 // Workgroups (of 16 wavefronts) per row of a launch over `rows` rows of `heads`
 // query heads each: as many as put one on every CU, each with at least one
-// pass of its wavefronts (select_pass blocks); 1 for rows that score in less
+// pass of its wavefronts (kSelectPass blocks); 1 for rows that score in less
 // than the keys' way through memory takes (2 us: under 2048 bounds).  As in the
 // attention, only more CUs take in a row's records faster.  us per launch,
 // whole rows (of 16 wavefronts) / split, 8192 blocks: bf16, 4 heads: 8 rows
-// 109 / 23, 64 rows 121 / 65, 128 rows 129 / 106; fp8, 8 heads: 8 rows
-// 421 / 35, 128 rows 478 / 261; 2048 blocks: fp16, 1 head, 32 rows 21 / 14;
+// 109 / 23, 64 rows 121 / 65, 128 rows 129 / 106; 2048 blocks: fp16, 1 head, 32 rows 21 / 14;
 // 512 blocks: bf16, 4 heads, 64 rows 14.8 / 13.7, fp16, 1 head, 32 rows
 // 10.3 / 10.7 (so left whole).
 int select_parts(const ferry_ctx* ctx, unsigned rows, int heads) {
   const unsigned mb = (unsigned)ctx->g.max_blocks, cus = (unsigned)ctx->cus;
   if (rows > select_split_rows(ctx) || mb * (unsigned)heads < 2048u) return 1;
-  const unsigned pass = (unsigned)select_pass(ctx->g.Hq / ctx->g.Hkv);
-  return (int)std::max(1u, std::min(cus / rows, (mb + pass - 1) / pass));
+  return (int)std::max(1u, std::min(cus / rows, (mb + kSelectPass - 1) / (unsigned)kSelectPass));
 }
 
 // Attention of layers [l0, l0 + nl).  attn_blocks (decode steps only): the
@@ -1359,12 +1357,14 @@ struct SelArgs {
 // records are scored by 16 wavefronts: four leave 8 KiB in flight per CU and
 // the row's arithmetic on one wavefront per SIMD.  Up to two rows per CU, 8;
 // more rows fill the CUs with workgroups of 4, whose top-k phases overlap the
-// others' loads better.  bf16, 4 query heads per kv head, 8192 blocks, us per
+// others' loads better; so do fp32 rows past one per CU, which wait for memory
+// (384 rows of 8192 blocks, 2 heads: 652 with 4, 710 with 8).  bf16, 4 query heads per kv head, 8192 blocks, us per
 // launch with 4 / 8 / 16 wavefronts: 128 rows 293 / 169 / 131, 256 rows
 // 321 / 201 / 176, 512 rows 379 / 344 / 345, 1024 rows 668 / 667 / 674; 512
 // blocks: 256 rows 24 / 18 / 17, 512 rows 30 / 27 / 34, 1024 rows 47 / 50 / 65.
-int select_waves(unsigned rows, int cus) {
-  return rows <= (unsigned)cus ? 16 : rows <= 2u * (unsigned)cus ? 8 : 4;
+int select_waves(int dtype, unsigned rows, int cus) {
+  if (rows <= (unsigned)cus) return 16;
+  return dtype != FERRY_F32 && rows <= 2u * (unsigned)cus ? 8 : 4;
 }
 
 template <int DT, int G, bool LAYER>
@@ -1377,7 +1377,7 @@ void launch_sel(const dim3& grid, size_t lds, hipStream_t s, const SelArgs& a) {
     FERRY_SEL_LAUNCH(16, true);
     return;
   }
-  switch (select_waves(grid.x, a.cus)) {
+  switch (select_waves(DT, grid.x, a.cus)) {
     case 16: FERRY_SEL_LAUNCH(16, false); return;
     case 8: FERRY_SEL_LAUNCH(8, false); return;
     default: FERRY_SEL_LAUNCH(4, false); return;
@@ -2059,14 +2059,13 @@ int ferry_bw_probe(ferry_ctx* ctx, int kind, const uint32_t* slots, uint64_t n, 
     if (kind == FERRY_PROBE_SUMS_READ) {
       const dim3 grid((unsigned)sum_grid), block(256);
       const int nb = (int)n, es = g.esize;
-      const bool u2 = g.Hq / g.Hkv >= 8;  // k_select_topk's passes in flight
       auto go = [&](auto kern) {
         hipLaunchKernelGGL(kern, grid, block, sum_lds, s, g, ctx->sums, ctx->sum_blocks, nb,
                            ctx->probe_sink);
       };
-      if (es == 1) u2 ? go(k_probe_sums<1, 2>) : go(k_probe_sums<1, 4>);
-      else if (es == 2) u2 ? go(k_probe_sums<2, 2>) : go(k_probe_sums<2, 4>);
-      else u2 ? go(k_probe_sums<4, 2>) : go(k_probe_sums<4, 4>);
+      if (es == 1) go(k_probe_sums<1, kSelectInflight>);
+      else if (es == 2) go(k_probe_sums<2, kSelectInflight>);
+      else go(k_probe_sums<4, kSelectInflight>);
       return hipGetLastError();
     }
     if (kind == FERRY_PROBE_HBM_COPY) {

@@ -52,10 +52,12 @@ __device__ inline float elem_f32(uint32_t v) {
     return (float)__builtin_bit_cast(_Float16, (uint16_t)v);
   } else if constexpr (DT == FERRY_BF16) {
     return bits_f32(v << 16);
-  } else {  // OCP E4M3FN: (-1)^s 2^(e-7) (1 + m/8), subnormal m 2^-9
-    const uint32_t s = (v & 0x80u) << 24, e = (v >> 3) & 0xFu, m = v & 7u;
-    if (e == 0) return bits_f32(f32_bits((float)m * 0.001953125f) | s);
-    return bits_f32(s | ((e + 120u) << 23) | (m << 20));
+  } else {
+    // OCP E4M3FN: (-1)^s 2^(e-7) (1 + m/8), subnormal m 2^-9.  The code's sign,
+    // exponent and mantissa placed in fp32's fields read as the value times
+    // 2^-120 (subnormal codes as fp32 subnormals), so one product is exact
+    const uint32_t t = (uint32_t)((int32_t)(v << 24) >> 4) & 0x87F00000u;
+    return bits_f32(t) * 0x1p120f;
   }
 }
 
@@ -86,6 +88,23 @@ __device__ inline void load8(const uint8_t* rec, int i0, float* f) {
     for (int e = 0; e < 8; ++e) f[e] = elem_f32<DT>((w[e >> 1] >> (16 * (e & 1))) & 0xFFFFu);
   }
 }
+
+// Records of one set: block b is record (set * max_blocks + b) mod n (the
+// tables' rule, host_index), the set's own part of it taken once.  A table of
+// at least max_blocks records, any but the smallest, needs one conditional
+// subtraction per block instead of a 64-bit remainder (~100 instructions a
+// lane).
+struct SetRecords {
+  uint64_t first, n;
+  bool once;  // launch-uniform
+  __device__ inline SetRecords(uint64_t set, uint64_t max_blocks, uint64_t n_)
+      : first(set * max_blocks % n_), n(n_), once(n_ >= max_blocks) {}
+  // b < max_blocks
+  __device__ inline uint64_t at(uint32_t b) const {
+    const uint64_t i = first + b;
+    return once ? (i >= n ? i - n : i) : i % n;
+  }
+};
 
 __device__ inline float fmax_det(float a, float b) { return a > b ? a : b; }
 
@@ -131,11 +150,13 @@ __device__ inline void transpose_level(float* v, int p) {
 // sum is formed in one lane group instead of all 16 lanes (G = 4: 5 swizzles
 // and 5 adds instead of 16 and 16); every sum is the same additions in the
 // same order as the butterfly's, and the maximum is the same chain, so the
-// result is bit-identical.  Head h ends in lane h * 16 / G of the row.
+// result is bit-identical.  Head h ends in lane h * 16 / G of the row.  `run`
+// (if not null) is the maximum over earlier heads, which the chain continues.
 template <int G>
-__device__ inline float heads_bound_max(float (&acc)[G], int p) {
+__device__ inline float heads_bound_max(float (&acc)[G], int p, const float* run = nullptr) {
   if constexpr (G == 1) {
-    return row16_sum(acc[0]);
+    const float v = row16_sum(acc[0]);
+    return run ? fmax_det(v, *run) : v;
   } else {
     transpose_level<8, G>(acc, p);
     if constexpr (G >= 4) transpose_level<4, G / 2>(acc, p);
@@ -144,7 +165,7 @@ __device__ inline float heads_bound_max(float (&acc)[G], int p) {
     if constexpr (G < 4) v += swz_xor<4>(v);
     if constexpr (G < 8) v += swz_xor<2>(v);
     v += swz_xor<1>(v);
-    float sk = v;
+    float sk = run ? fmax_det(v, *run) : v;
 #pragma unroll
     for (int h = 1; h < G; ++h) {
       float other;
@@ -399,55 +420,72 @@ __global__ __launch_bounds__(W * 64) void k_select_topk(Geo g, const float* __re
     // bytes counted as they are written, while the loads stream)
     const int grp = lane >> 4, p = lane & 15;
     for (int i = tid; i < 256; i += NT) hist[i] = 0;
-    // the row's query dims of this lane (8 per head), and whether each uses kmax
-    float qr[G][8];
-    if (!LAYER) {
+    // The query dims of this lane (8 per head) and whether each uses kmax.  Up
+    // to 4 heads of one kv head stay in registers, their signs as 32 lane masks
+    // in scalar registers.  Eight heads' 64 masks spilled (two lane reads per
+    // use, twice the scoring's instructions), so they are scored 4 at a time
+    // with queries from LDS, as a layer's rows are: 1024 rows of 8192 blocks
+    // 1187 -> 879 us in bf16, 1856 -> 871 in fp8 (with its shorter decoding).
+    constexpr int GH = G < 4 ? G : 4;
+    constexpr bool QLDS = LAYER || GH < G;
+    float qr[GH][8];
+    if (!QLDS) {
 #pragma unroll
-      for (int gq = 0; gq < G; ++gq)
+      for (int gq = 0; gq < GH; ++gq)
 #pragma unroll
         for (int e = 0; e < 8; ++e)
           qr[gq][e] = q[((size_t)rl * g.Hq + (size_t)(hrow * G + gq)) * D + 8 * p + e];
-      __syncthreads();
     } else {
-      for (int i = tid; i < Gq * D; i += NT) qs[i] = q[(size_t)rl * g.Hq * D + i];
-      __syncthreads();
+      for (int i = tid; i < Gq * D; i += NT)
+        qs[i] = q[((size_t)rl * g.Hq + (size_t)(LAYER ? 0 : hrow * G)) * D + i];
     }
+    __syncthreads();
     // U passes of 4 blocks per wavefront are loaded before any is scored: the
     // keys take most of the LDS at long contexts, so few workgroups share a
     // CU and each wavefront must keep several records in flight
-    constexpr int U = select_inflight(G);
+    constexpr int U = kSelectInflight;
     for (int b0 = 4 * (wave + W * U * part); b0 < n; b0 += 4 * W * U * (SPLIT ? parts : 1)) {
       float score[U];
       for (int hh = 0; hh < nkv; ++hh) {
         const int hk = LAYER ? hh : hrow;
-        const uint64_t set = (uint64_t)rl * g.Hkv + hk;
+        const SetRecords recs((uint64_t)rl * g.Hkv + hk, (uint64_t)g.max_blocks, sum_mod);
         float kmn[U][8], kmx[U][8];
         uint64_t hbs[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
           const int b = b0 + 4 * W * u + grp;
-          hbs[u] = host_index(set, b < n ? (uint32_t)b : 0u, (uint64_t)g.max_blocks, sum_mod);
+          hbs[u] = recs.at(b < n ? (uint32_t)b : 0u);
           const uint8_t* rec = sums + hbs[u] * REC;
           load8<DT>(rec, 8 * p, kmn[u]);
           load8<DT>(rec, D + 8 * p, kmx[u]);
         }
-        if (LAYER) {
+        float bound[U];
 #pragma unroll
-          for (int gq = 0; gq < G; ++gq)
+        for (int h0 = 0; h0 < G; h0 += GH) {
+          if (QLDS) {
+            asm volatile("" ::: "memory");  // read them here, not once for every head
 #pragma unroll
-            for (int e = 0; e < 8; ++e) qr[gq][e] = qs[(hh * G + gq) * D + 8 * p + e];
+            for (int gq = 0; gq < GH; ++gq)
+#pragma unroll
+              for (int e = 0; e < 8; ++e)
+                qr[gq][e] = qs[((LAYER ? hh * G : 0) + h0 + gq) * D + 8 * p + e];
+          }
+#pragma unroll
+          for (int u = 0; u < U; ++u) {
+            float acc[GH];
+#pragma unroll
+            for (int gq = 0; gq < GH; ++gq) {
+              acc[gq] = 0.0f;
+#pragma unroll
+              for (int e = 0; e < 8; ++e)
+                acc[gq] = __fmaf_rn(qr[gq][e], qr[gq][e] >= 0.0f ? kmx[u][e] : kmn[u][e], acc[gq]);
+            }
+            bound[u] = heads_bound_max<GH>(acc, p, h0 ? &bound[u] : nullptr);
+          }
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-          float acc[G];
-#pragma unroll
-          for (int gq = 0; gq < G; ++gq) {
-            acc[gq] = 0.0f;
-#pragma unroll
-            for (int e = 0; e < 8; ++e)
-              acc[gq] = __fmaf_rn(qr[gq][e], qr[gq][e] >= 0.0f ? kmx[u][e] : kmn[u][e], acc[gq]);
-          }
-          float sk = heads_bound_max<G>(acc, p);
+          float sk = bound[u];
           if constexpr (DT == FERRY_FP8_E4M3) sk = __fmul_rn(sk, sum_scales[hbs[u]]);
           score[u] = hh == 0 ? sk : fmax_det(sk, score[u]);
         }
@@ -645,7 +683,7 @@ __global__ __launch_bounds__(W * 64) void k_select_mass(Geo g, const float* __re
       continue;
     }
     for (int h = 0; h < g.Hkv; ++h) {
-      const uint64_t set = (uint64_t)rl * g.Hkv + h;
+      const SetRecords recs((uint64_t)rl * g.Hkv + h, (uint64_t)g.max_blocks, kt_mod);
       float qr[G][EPL];
 #pragma unroll
       for (int gq = 0; gq < G; ++gq)
@@ -662,7 +700,7 @@ __global__ __launch_bounds__(W * 64) void k_select_mass(Geo g, const float* __re
         for (int u = 0; u < U; ++u) {
           const int b = b0 + W * u;
           if (b < n) {  // wavefront-uniform
-            const uint64_t rec = host_index(set, (uint32_t)b, (uint64_t)g.max_blocks, kt_mod);
+            const uint64_t rec = recs.at((uint32_t)b);
             const u32x4* base = reinterpret_cast<const u32x4*>(kt + rec * KT);
 #pragma unroll
             for (int i = 0; i < NI; ++i) w[u][i] = __builtin_nontemporal_load(base + i * 64 + lane);
@@ -854,7 +892,7 @@ __global__ __launch_bounds__(W * 64) void k_mass_units(
     const int per = (nb + parts - 1) / parts;
     const int lo = min(nb, part * per), hi = min(nb, lo + per);
     if (split) ws = ws_all + (size_t)unit * max_n * G;
-    const uint64_t set = (uint64_t)rl * g.Hkv + h;
+    const SetRecords recs((uint64_t)rl * g.Hkv + h, (uint64_t)g.max_blocks, kt_mod);
     // ---- Q^T operand: k-step ks, this lane's 8 dims, head n (0 for pad heads)
     uint32_t qb[NQ][4][4];
 #pragma unroll
@@ -892,7 +930,7 @@ __global__ __launch_bounds__(W * 64) void k_mass_units(
       for (int u = 0; u < U; ++u) {
         const int b = b0 + W * u;
         if (b < hi) {  // wavefront-uniform
-          const uint64_t rec = host_index(set, (uint32_t)b, (uint64_t)g.max_blocks, kt_mod);
+          const uint64_t rec = recs.at((uint32_t)b);
           // lane-transposed record: this lane's word w is word 64 w + lane
           const u32x4* base = reinterpret_cast<const u32x4*>(kt + rec * KT) + lane;
 #pragma unroll
