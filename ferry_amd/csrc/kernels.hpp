@@ -89,6 +89,14 @@ template <bool SERIAL>
 __global__ void k_lru_step(Geo g, const uint32_t* sel, uint32_t* slots_out, uint32_t* miss_count,
                            ferry_miss* misses, uint8_t* miss_flag, SetState st, Ring ring, int l0,
                            int nl, unsigned long long* sel_counts, int* err);
+// One workgroup per set, for sets of at least kLruGroupSel selections a step.
+constexpr int kLruGroupWaves = 4;
+constexpr int kLruGroupSel = 256;
+constexpr int kLruGroupLds = 256;  // its own LDS words beside the set's, at most
+template <int W>
+__global__ void k_lru_group(Geo g, const uint32_t* sel, uint32_t* slots_out, uint32_t* miss_count,
+                            ferry_miss* misses, uint8_t* miss_flag, SetState st, Ring ring, int l0, int nl,
+                            unsigned long long* sel_counts, int* err);
 __global__ void k_sets_reset(Geo g, SetState st);
 __global__ void k_sets_reset_owners(Geo g, SetState st, const uint32_t* owners, uint32_t n, int* err);
 // Resident members: lanes leave (delta -1) or join (+1); owners that lost a

@@ -377,6 +377,293 @@ template __global__ void k_lru_step<true>(Geo, const uint32_t*, uint32_t*, uint3
                                           uint8_t*, SetState, Ring, int, int, unsigned long long*,
                                           int*);
 
+// The same step for sets of many selections (prefix groups: group * k
+// positions), one workgroup of W wavefronts per set: every pass of substep()
+// over positions, slots or misses is dealt out between the wavefronts, and the
+// ranks that order the misses and the new LRU order are counted per wavefront
+// over contiguous runs first.  Bound: the chain of dependent map and state
+// accesses, which one wavefront walked 64 positions at a time.  320 sets of
+// 1024 selections and 1536 slots: 45 us -> 22.5; 192 such sets beside a fetch,
+// whose host reads slow each access of the chain, 215 -> 65.  Results, state
+// and errors are k_lru_step's.  Needs the staged selections (lru_stages_sel);
+// below 256 selections a wavefront's run would be less than one 64-lane round.
+template <int W>
+__global__ __launch_bounds__(W * 64) void k_lru_group(Geo g, const uint32_t* __restrict__ sel,
+                                                      uint32_t* __restrict__ slots_out,
+                                                      uint32_t* __restrict__ miss_count,
+                                                      ferry_miss* __restrict__ misses,
+                                                      uint8_t* __restrict__ miss_flag, SetState st,
+                                                      Ring ring, int l0, int nl,
+                                                      unsigned long long* __restrict__ sel_counts,
+                                                      int* __restrict__ err) {
+  constexpr int NT = W * 64, U = 4;  // U rounds of loads in flight per thread
+  extern __shared__ uint32_t lds[];
+  __shared__ int wcnt[2][W];
+  __shared__ int sh_nv, sh_nsel;
+  __shared__ uint32_t sh_t0;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int idx = blockIdx.x;
+  const int set = ((idx / (nl * g.Hkv)) * g.L + l0 + (idx / g.Hkv) % nl) * g.Hkv + idx % g.Hkv;
+  const int C = g.C;
+  int* lastpos = (int*)lds;
+  uint32_t* sord = lds + C;
+  uint32_t* stag = lds + 2 * C;
+  uint32_t* smblk = lds + 3 * C;
+  uint32_t* svict = smblk + g.max_sel;
+  uint32_t* sown = st.own ? svict + g.max_sel : nullptr;  // [C] member masks
+  uint32_t* ssel = lds + lru_lds_words(g);                // [max_sel] selections
+  uint32_t* sslot = ssel + g.max_sel;                     // [max_sel] miss marks, then slots
+
+  SetView sv;
+  sv.h = set % g.Hkv;
+  sv.l = (set / g.Hkv) % g.L;
+  sv.o = set / (g.Hkv * g.L);
+  sv.n = min(g.group, g.n_req - sv.o * g.group) * g.k;
+  const int n = sv.n;
+
+  uint32_t* map = st.map + (size_t)set * (size_t)g.max_blocks;
+  uint32_t* gord = st.ord + (size_t)set * C;
+  uint32_t* gtag = st.tag + (size_t)set * C;
+  uint32_t* gown = st.own ? st.own + (size_t)set * C : nullptr;
+  const int fill = (int)st.fill[set];
+  const uint32_t worker = ring.worker_of_set[set];
+  const int cap = (int)set_capacity(g, st.members[sv.o]);
+  if (tid == 0) sh_nsel = 0;
+  for (int i0 = tid; i0 < C; i0 += NT * U) {
+    uint32_t o4[U], t4[U], w4[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int i = i0 + u * NT;
+      if (i < C) o4[u] = gord[i], t4[u] = gtag[i], w4[u] = sown ? gown[i] : 0u;
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int i = i0 + u * NT;
+      if (i < C) {
+        lastpos[i] = -1;
+        sord[i] = o4[u];
+        stag[i] = t4[u];
+        if (sown) sown[i] = w4[u];
+      }
+    }
+  }
+  // range check of every selected id before touching the map
+  bool bad = false;
+  int mine = 0;  // non-empty positions
+  for (int p0 = tid; p0 < n; p0 += NT * U) {
+    uint32_t x4[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int p = p0 + u * NT;
+      x4[u] = p < n ? sel[sel_index(g, sv, p)] : kNone;
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int p = p0 + u * NT;
+      if (p < n) ssel[p] = x4[u];
+      bad |= x4[u] != kNone && x4[u] >= (uint32_t)g.max_blocks;
+      mine += x4[u] != kNone;
+    }
+  }
+  if (__syncthreads_or(bad)) {  // uniform
+    if (tid == 0) {
+      set_error(err, FERRY_ERANGE);
+      miss_count[set] = 0;
+    }
+    return;
+  }
+  if (mine) atomicAdd(&sh_nsel, mine);
+
+  // this wavefront's accesses to the map have completed, then everyone's
+  auto map_sync = [&]() {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+  };
+  // positions p0 + u NT of a pass and their map entries
+  uint32_t xs[U], vs[U];
+  auto gather = [&](int p0) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) xs[u] = p0 + u * NT < n ? ssel[p0 + u * NT] : kNone;
+#pragma unroll
+    for (int u = 0; u < U; ++u) vs[u] = xs[u] != kNone ? aload(map + xs[u]) : kNone;
+  };
+  // phase 1: classify (hits mark their slot; misses race for first occurrence)
+  for (int p0 = tid; p0 < n; p0 += NT * U) {
+    gather(p0);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (xs[u] == kNone) continue;
+      if (vs[u] < (uint32_t)C) atomicMax(lastpos + vs[u], p0 + u * NT);
+      else atomicMin(map + xs[u], kPend | (uint32_t)(p0 + u * NT));
+    }
+  }
+  map_sync();
+  // phase 2: the misses, first occurrences marked ...
+  for (int p0 = tid; p0 < n; p0 += NT * U) {
+    gather(p0);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int p = p0 + u * NT;
+      if (p >= n) continue;
+      const bool is_miss = xs[u] != kNone && vs[u] == (kPend | (uint32_t)p);
+      if (miss_flag) miss_flag[sel_index(g, sv, p)] = is_miss ? 1 : 0;
+      sslot[p] = is_miss;
+    }
+  }
+  __syncthreads();
+  // ... and ranked over each wavefront's contiguous run of positions
+  const int span = (n + NT - 1) / NT * 64;
+  const int w0 = min(n, wave * span), w1 = min(n, w0 + span);
+  int cnt = 0;
+  for (int c = w0; c < w1; c += 64) {
+    const int p = c + lane;
+    cnt += __builtin_popcountll(ballot(p < w1 && sslot[p]));
+  }
+  if (lane == 0) wcnt[0][wave] = cnt;
+  __syncthreads();
+  int M = 0, r = 0;
+#pragma unroll
+  for (int w = 0; w < W; ++w) {
+    r += w < wave ? wcnt[0][w] : 0;
+    M += wcnt[0][w];
+  }
+  for (int c = w0; c < w1; c += 64) {
+    const int p = c + lane;
+    const bool is_miss = p < w1 && sslot[p];
+    const uint64_t mask = ballot(is_miss);
+    if (is_miss) smblk[r + lanes_below(mask)] = ssel[p];
+    r += __builtin_popcountll(mask);
+  }
+  // phase 3: victims = least recent untouched residents, oldest first; then M
+  // entries at the tail of this set's worker deque
+  const int freeslots = cap > fill ? cap - fill : 0;
+  const int need = M > freeslots ? M - freeslots : 0;
+  if (wave == 0) {
+    int nv = 0;
+    for (int c = 0; c < fill && nv < need; c += 64) {
+      const int i = c + lane;
+      const uint32_t o = i < fill ? sord[i] : 0u;
+      const bool untouched = i < fill && lastpos[o] < 0;
+      const uint64_t mask = ballot(untouched);
+      const int v = nv + lanes_below(mask);
+      if (untouched && v < need) svict[v] = o;
+      nv += __builtin_popcountll(mask);
+    }
+    if (lane == 0) {
+      sh_nv = nv;
+      sh_t0 = 0;
+      if (nv >= need && M > 0)
+        sh_t0 = (uint32_t)(atomicAdd((unsigned long long*)(ring.state + (size_t)worker * kStateStride),
+                                     (unsigned long long)M << 32) >> 32);
+    }
+  }
+  __syncthreads();
+  int rc = sh_nv < need ? FERRY_ECAPACITY : 0;
+  if (!rc && M > 0 && sh_t0 + (uint32_t)M > ring.cap[worker]) rc = FERRY_ESPIN;
+  if (rc) {  // uniform
+    for (int q = tid; q < M; q += NT) astore(map + smblk[q], kNone);
+    if (tid == 0) {
+      set_error(err, rc);
+      miss_count[set] = 0;
+    }
+    return;
+  }
+  // phase 4: assign slots, evict, publish block -> slot, write the ring
+  ferry_miss* mo = misses + (size_t)set * g.max_sel;
+  ferry_miss* rdst = ring.entries + ring.seg[worker] + sh_t0;
+  for (int q = tid; q < M; q += NT) {
+    ferry_miss m;
+    m.block = smblk[q];
+    m.evicted = kNone;
+    m.set = (uint32_t)set;
+    if (q < freeslots) {
+      m.slot = (uint32_t)(fill + q);
+    } else {
+      m.slot = svict[q - freeslots];
+      m.evicted = stag[m.slot];
+      if (m.evicted < (uint32_t)g.max_blocks) astore(map + m.evicted, kNone);
+    }
+    stag[m.slot] = m.block;
+    if (sown) sown[m.slot] = 0u;  // a new block: the slot's old members are dropped
+    astore(map + m.block, m.slot);
+    mo[q] = m;
+    rdst[q] = m;
+  }
+  map_sync();
+  // phase 4b: slot of every position; last occurrence per touched slot
+  for (int p0 = tid; p0 < n; p0 += NT * U) {
+    gather(p0);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int p = p0 + u * NT;
+      if (p >= n) continue;
+      const size_t gi = sel_index(g, sv, p);
+      if (xs[u] == kNone) {
+        slots_out[gi] = kNone;
+        continue;
+      }
+      sslot[p] = vs[u];
+      slots_out[gi] = (uint32_t)set * (uint32_t)C + vs[u];
+      atomicMax(lastpos + vs[u], p);
+      if (sown) atomicOr(sown + vs[u], 1u << (uint32_t)(p / g.k));  // member of position p
+    }
+  }
+  __syncthreads();
+  // phase 5: new LRU order: the untouched survivors in their old order, then
+  // the touched slots by their last occurrence, straight to the set's state
+  const int fspan = (fill + NT - 1) / NT * 64;
+  const int f0 = min(fill, wave * fspan), f1 = min(fill, f0 + fspan);
+  auto kept = [&](int i) { return i < f1 && lastpos[sord[i]] < 0; };
+  auto last_at = [&](int p) { return p < w1 && ssel[p] != kNone && lastpos[sslot[p]] == p; };
+  int nk = 0, ne = 0;
+  for (int c = f0; c < f1; c += 64) nk += __builtin_popcountll(ballot(kept(c + lane)));
+  for (int c = w0; c < w1; c += 64) ne += __builtin_popcountll(ballot(last_at(c + lane)));
+  if (lane == 0) wcnt[0][wave] = nk, wcnt[1][wave] = ne;
+  __syncthreads();
+  int at_k = 0, at_e = 0, total = 0;
+#pragma unroll
+  for (int w = 0; w < W; ++w) {
+    at_k += w < wave ? wcnt[0][w] : 0;
+    at_e += wcnt[0][w] + (w < wave ? wcnt[1][w] : 0);
+    total += wcnt[0][w] + wcnt[1][w];
+  }
+  const int nfill = fill + min(M, freeslots);
+  if (total != nfill) {  // uniform
+    if (tid == 0) {
+      set_error(err, FERRY_ESTATE);
+      miss_count[set] = 0;
+    }
+    return;
+  }
+  for (int c = f0; c < f1; c += 64) {
+    const bool k = kept(c + lane);
+    const uint64_t mask = ballot(k);
+    if (k) gord[at_k + lanes_below(mask)] = sord[c + lane];
+    at_k += __builtin_popcountll(mask);
+  }
+  for (int c = w0; c < w1; c += 64) {
+    const bool e = last_at(c + lane);
+    const uint64_t mask = ballot(e);
+    if (e) gord[at_e + lanes_below(mask)] = sslot[c + lane];
+    at_e += __builtin_popcountll(mask);
+  }
+  for (int i = nfill + tid; i < C; i += NT) gord[i] = kNone;
+  for (int i = tid; i < C; i += NT) {
+    gtag[i] = stag[i];
+    if (sown) gown[i] = sown[i];
+  }
+  if (tid == 0) {
+    st.fill[set] = (uint32_t)nfill;
+    miss_count[set] = (uint32_t)M;
+    if (sh_nsel)
+      atomicAdd(sel_counts + (size_t)(set % kSelCounters) * kSelStride, (unsigned long long)sh_nsel);
+  }
+}
+
+template __global__ void k_lru_group<kLruGroupWaves>(Geo, const uint32_t*, uint32_t*, uint32_t*,
+                                                     ferry_miss*, uint8_t*, SetState, Ring, int, int,
+                                                     unsigned long long*, int*);
+
 // Reset the sets of the listed owners (a new request takes over a lane):
 // one wavefront per set clears the map entries its tags point at, then the
 // tags, the order and the fill.  Owner ids must be < n_owners (checked).

@@ -1040,6 +1040,11 @@ int bookkeep_ring(ferry_ctx* ctx, int32_t l0, int32_t nl, const uint32_t* sel, u
     hipLaunchKernelGGL(k_lru_step<true>, grid, block, ctx->lru_lds, (hipStream_t)stream, g, sel, slots,
                        miss_count, misses, miss_flag, ctx->st, ctx->ring(which), l0, nl,
                        ctx->sel_counts, ctx->err);
+  else if (g.max_sel >= kLruGroupSel && lru_stages_sel(g) &&
+           lru_lds_wave_words(g) * 4 + kLruGroupLds <= 65536)
+    hipLaunchKernelGGL(k_lru_group<kLruGroupWaves>, dim3((unsigned)nsets), dim3(64 * kLruGroupWaves),
+                       lru_lds_wave_words(g) * 4, (hipStream_t)stream, g, sel, slots, miss_count, misses,
+                       miss_flag, ctx->st, ctx->ring(which), l0, nl, ctx->sel_counts, ctx->err);
   else
     hipLaunchKernelGGL(k_lru_step<false>, grid, block, ctx->lru_lds, (hipStream_t)stream, g, sel, slots,
                        miss_count, misses, miss_flag, ctx->st, ctx->ring(which), l0, nl,
