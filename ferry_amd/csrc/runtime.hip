@@ -156,6 +156,7 @@ struct ferry_ctx {
   float* ktab_scales = nullptr;    // ... and their K scales (fp8)
   uint64_t kt_records = 0;         // records, addressed like the summaries
   float* mass_ws = nullptr;        // per-workgroup (max, sum) of every block and query head
+  uint64_t mass_ws_size = 0;       // ... bytes; split units where it holds what they take
   int kt_perm = 0;                 // K table words lane-transposed for the matrix-core loads
   float* scratch_dev = nullptr;    // this device's address of the static `scratch` array
   uint32_t* lane_live = nullptr;   // [n_req] 1 while the lane's request is a resident member
@@ -1636,8 +1637,15 @@ int ferry_ktiles_build(ferry_ctx* ctx, uint64_t n_records, void* stream) {
       return rc;
     ctx->kt_records = S;
   }
-  if (!ctx->mass_ws && (uint64_t)g.max_blocks * 4 <= kMassLds)
-    HIPC(hipMalloc(&ctx->mass_ws, mass_ctx_bytes(ctx)));
+  if (!ctx->mass_ws && (uint64_t)g.max_blocks * 4 <= kMassLds) {
+    ctx->mass_ws_size = mass_ctx_bytes(ctx);
+    if (hipMalloc(&ctx->mass_ws, ctx->mass_ws_size) != hipSuccess) {
+      (void)hipGetLastError();
+      ctx->mass_ws = nullptr;
+      ctx->mass_ws_size = mass_ws_bytes(ctx, g.L, mass_wgs(ctx, g.L, ~0ull));  // whole units only
+      HIPC(hipMalloc(&ctx->mass_ws, ctx->mass_ws_size));
+    }
+  }
   ctx->kt_perm = g.dtype != FERRY_F32;
   const unsigned blocks = (unsigned)std::min<uint64_t>((g.host_blocks + 3) / 4, 16384);
   switch (KT / 1024) {
@@ -1787,7 +1795,7 @@ int ferry_select_mass_layers(ferry_ctx* ctx, int32_t l0, int32_t nl, const float
   if (int rc = check_select_mass(ctx, l0, nl, q, ctx_blocks, sel)) return rc;
   if (!ctx->mass_ws) return fail(FERRY_EINVAL, "no mass-selection workspace (ferry_ktiles_build failed)");
   return launch_select_mass(ctx, l0, nl, q, ctx_blocks, sel, stream, ctx->mass_ws,
-                            mass_wgs(ctx, nl, ~0ull), mass_ctx_bytes(ctx));
+                            mass_wgs(ctx, nl, ~0ull), ctx->mass_ws_size);
 }
 
 int ferry_select_mass(ferry_ctx* ctx, const float* q, const int32_t* ctx_blocks, uint32_t* sel,
