@@ -266,11 +266,11 @@ __global__ __launch_bounds__(W * 64) void k_attn_group(
   // own entries after them, ordered by (member, slot); equal keys are the same
   // block for the same member, so their order among themselves does not matter.
   // An entry's rank: the own entries of earlier members (their counts) and
-  // those of its own member's row before it, k positions instead of group * k
-  int cown = 0;
-  for (int e = tid; e < GK; e += NT) cown += own[e] != kNone;
+  // those of its own member's row before it, k positions instead of group * k.
+  // The counts' sum says how many there are (a scan over the entries for it
+  // took 0.6 us of a workgroup's list).
   int n_own = 0;
-  (void)block_exclusive_scan<W>(cown, sh, &n_own);
+  for (int m = 0; m < mpw; ++m) n_own += (int)mcnt[m];
   if (n_own > 0) {  // uniform
     for (int e = tid; e < GK; e += NT) {
       const uint32_t s = own[e];
