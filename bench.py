@@ -195,7 +195,7 @@ def rocprof_summary(db_path, last):
     closes = [i for i, r in enumerate(rows) if short(r[0]).endswith("k_step_close")]
     if closes:
         tail = [r for r in rows[closes[-1] + 1:]
-                if any(k in short(r[0]) for k in ("k_lru_step", "k_fetch", "k_attn"))]
+                if any(k in short(r[0]) for k in ("k_lru", "k_fetch", "k_attn"))]
         # an attention launch right after a fetch drain belongs to an event-timed
         # step; the ones after another attention launch are the back-to-back runs
         timed, b2b = [], []
