@@ -267,6 +267,10 @@ __global__ void k_mass_topk(Geo g, const int32_t* ctx_blocks, const float* mass,
 // persistent workgroups of k_select_mass (fp32 K); each holds max_blocks * G * 2
 // floats of workspace
 constexpr int kMassWgs = 2048;
+// Wavefronts per fp32 item in launches of few items, and the LDS such a
+// workgroup has beside the scores, at most.
+constexpr int kMassWideWaves = 8;
+constexpr size_t kMassWideLds = 12 * 1024;
 // k_mass_units: wavefronts per workgroup, K records in flight per wavefront,
 // and at most this many workgroups (the GPU's resident ones below that), each
 // with a max_blocks * G * 2-float workspace slice.  At the long-context GQA

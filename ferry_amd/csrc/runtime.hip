@@ -1700,16 +1700,29 @@ int launch_select_mass(ferry_ctx* ctx, int32_t l0, int32_t nl, const float* q,
   const int G = g.Hq / g.Hkv;
   const size_t lds = (size_t)g.max_blocks * 4;
   if (g.dtype == FERRY_F32) {  // vector ALUs, one (request, layer) item per workgroup pass
-#define FERRY_MASS_LAUNCH(GG)                                                                  \
-  hipLaunchKernelGGL((k_select_mass<FERRY_F32, GG, 4>), dim3((unsigned)wgs), dim3(256), lds, s, g, \
-                     q, ctx_blocks, ctx->ktab, ctx->ktab_scales, ctx->kt_records, ws, sel, l0, nl, \
+    // 8 wavefronts where items leave a CU one workgroup: twice the loads in
+    // flight, and the heads' dot products on two wavefronts per SIMD.  Past half
+    // as many items as CUs that only helps wide groups.  4096 blocks, 8 kv heads,
+    // us with 4 / 8: 1 item, 1 head 5695 / 4512, 2 heads 7418 / 4560, 8 heads
+    // 18382 / 9797; 512 blocks, 256 items: 2 heads 1312 / 1335, 8 heads
+    // 2424 / 1601.
+    const bool wide = wgs <= (uint64_t)(G >= 4 ? ctx->cus : ctx->cus / 2) && lds + kMassWideLds <= 65536;
+#define FERRY_MASS_LAUNCH_W(GG, W)                                                                \
+  hipLaunchKernelGGL((k_select_mass<FERRY_F32, GG, W>), dim3((unsigned)wgs), dim3(64 * W), lds, s, \
+                     g, q, ctx_blocks, ctx->ktab, ctx->ktab_scales, ctx->kt_records, ws, sel, l0, nl, \
                      g.max_blocks, ctx->err)
+#define FERRY_MASS_LAUNCH(GG)                              \
+  do {                                                     \
+    if (wide) FERRY_MASS_LAUNCH_W(GG, kMassWideWaves);     \
+    else FERRY_MASS_LAUNCH_W(GG, 4);                       \
+  } while (0)
     switch (G) {
       case 1: FERRY_MASS_LAUNCH(1); break;
       case 2: FERRY_MASS_LAUNCH(2); break;
       case 4: FERRY_MASS_LAUNCH(4); break;
       default: FERRY_MASS_LAUNCH(8); break;
     }
+#undef FERRY_MASS_LAUNCH_W
 #undef FERRY_MASS_LAUNCH
     HIPC(hipGetLastError());
     return FERRY_OK;

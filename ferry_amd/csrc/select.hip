@@ -1118,10 +1118,13 @@ __global__ __launch_bounds__(W * 64) void k_mass_topk(Geo g, const int32_t* __re
   }
 }
 
-#define FERRY_MASS_INST(DT, G)                                                                   \
-  template __global__ void k_select_mass<DT, G, 4>(Geo, const float*, const int32_t*,              \
+#define FERRY_MASS_INST_W(DT, G, W)                                                               \
+  template __global__ void k_select_mass<DT, G, W>(Geo, const float*, const int32_t*,              \
                                                    const uint8_t*, const float*, uint64_t, float*, \
                                                    uint32_t*, int, int, int, int*);
+#define FERRY_MASS_INST(DT, G) \
+  FERRY_MASS_INST_W(DT, G, 4)  \
+  FERRY_MASS_INST_W(DT, G, kMassWideWaves)
 #define FERRY_MASS_UNITS_INST(DT, G)                                                          \
   template __global__ void k_mass_units<DT, G, kMassUnitWaves, kMassUnitInflight>(            \
       Geo, const float*, const int32_t*, const uint8_t*, const float*, uint64_t, float*, float*, \

@@ -172,6 +172,29 @@ def test_select_mass_split_and_whole_units(dtype, Hkv, Hq, ws, monkeypatch):
     assert p.ex.stats()["device_error"] == 0
 
 
+@pytest.mark.parametrize("Hq", [2, 16])
+def test_select_mass_fp32_workgroup_sizes(Hq):
+    """fp32 items take 8 wavefronts in launches of few items and 4 in larger
+    ones (more than 128 items, or 256 with 4 heads or more per kv head, on 256
+    CUs): 70 and 280 items of the same rows, contexts around a wavefront's
+    share."""
+    n_req, L, Hkv, k, mb = 70, 4, 2, 8, 40
+    p = Pair(n_req, L, Hkv, Hq, k, 16, mb, F.F32, host_blocks=1031)
+    p.ex.ktiles_build()
+    rng = np.random.default_rng(Hq)
+    ctx = rng.choice([0, 8, 9, 15, 16, 17, 31, 32, 33, 40], n_req).astype(np.int32)
+    q = rng.standard_normal((n_req, L, Hq, 128)).astype(np.float32)
+    dq, dctx = torch.from_numpy(q).cuda(), torch.from_numpy(ctx).cuda()
+    sc = O.mass_scores(p.g, q, ctx)
+    for step in (1, 4):  # layers per launch
+        sel = torch.full((n_req, L, Hkv, k), -7, dtype=torch.int32, device="cuda")
+        for l0 in range(0, L, step):
+            p.ex.select_mass(dq, dctx, sel, layers=(l0, step))
+        torch.cuda.synchronize()
+        assert _check_rows(p, sel.cpu().numpy().view(np.uint32), q, ctx, sc=sc) >= 0.9
+    assert p.ex.stats()["device_error"] == 0
+
+
 @pytest.mark.parametrize("dtype", [F.F16, F.FP8])
 def test_zero_query_takes_the_lowest_ids(dtype):
     """q = 0: every token gets probability 1/(16 ctx), every block the same
