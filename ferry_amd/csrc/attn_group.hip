@@ -14,8 +14,10 @@
 // One workgroup of W = 4 wavefronts per (group, layer, kv head), two per CU
 // (the LDS is mostly the wavefronts' block rings).  Launches of few sets run
 // W = 8 and split a set's members between workgroups (mpw members each, whole
-// query tiles): everything below then holds for a workgroup's own members.  The group's
-// query columns (member x query head, NTILE tiles of 16, attn_mfma.hpp) are
+// query tiles).  Each of them lists the whole set, so that every block falls to
+// the wavefront, and after the blocks, that it would in one workgroup, and then
+// keeps its own members' entries: a member's output is the same bits whatever
+// the split.  The group's query columns (member x query head, NTILE tiles of 16, attn_mfma.hpp) are
 // held by every wavefront; the blocks are split between the wavefronts.
 //  1. List: every member row's slots are OR-ed into a per-slot member mask in
 //     LDS (one word per slot of the set).  A repeated selection in one row,
@@ -169,7 +171,7 @@ __global__ __launch_bounds__(W * 64) void k_attn_group(
 
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   const int mpw = SPLIT ? split_mpw : g.group;  // members per workgroup
-  const int GK = mpw * g.k;
+  const int GK = g.group * g.k;
   uint8_t* rings = smem;                                                  // [W][R][BB]
   u32x4* qops = reinterpret_cast<u32x4*>(smem + W * RB);                  // [NQ][NTILE][4][64]
   uint32_t* lslot = reinterpret_cast<uint32_t*>(qops + NQ * NTILE * 4 * 64);  // [GK] list
@@ -182,15 +184,17 @@ __global__ __launch_bounds__(W * 64) void k_attn_group(
 
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int n = lane & 15, grp = lane >> 4;
-  // (owner, layer, kv head) of this workgroup's set, and its member rows
-  // [m0, m0 + mem): the owner's, or those of this workgroup's part
+  // (owner, layer, kv head) of this workgroup's set, whose members are the
+  // `all` requests from o0, and the member rows it attends, `mem` from m0:
+  // the set's, or those of this workgroup's part
   const GroupPart gp = SPLIT ? group_part(blockIdx.x, (g.group + mpw - 1) / mpw)
                              : GroupPart{(int)blockIdx.x, 0};
   const int h = gp.set % g.Hkv;
   const int l = l0 + (gp.set / g.Hkv) % nl;
   const int o = gp.set / (nl * g.Hkv);
-  const int m0 = o * g.group + gp.part * mpw;
-  const int mem = min(SPLIT ? min(mpw, g.group - gp.part * mpw) : mpw, g.n_req - m0);
+  const int o0 = o * g.group, m0 = o0 + gp.part * mpw;
+  const int all = min(g.group, g.n_req - o0);
+  const int mem = min(mpw, all - gp.part * mpw);
   if (SPLIT && (o >= g.n_owners || mem <= 0)) return;  // workgroup-uniform
   const uint32_t base = (uint32_t)((o * g.L + l) * g.Hkv + h) * (uint32_t)g.C;
 
@@ -210,8 +214,8 @@ __global__ __launch_bounds__(W * 64) void k_attn_group(
     for (int u = 0; u < SB; ++u) {
       const int e = e0 + u * NT, mi = e / g.k;
       sv[u] = kNone;
-      if (e < GK && mi < mem)
-        sv[u] = slots[((size_t)((m0 + mi) * g.L + l) * g.Hkv + h) * g.k + (e - mi * g.k)];
+      if (e < GK && mi < all)
+        sv[u] = slots[((size_t)((o0 + mi) * g.L + l) * g.Hkv + h) * g.k + (e - mi * g.k)];
     }
   };
   uint32_t sv[SB];
@@ -219,7 +223,7 @@ __global__ __launch_bounds__(W * 64) void k_attn_group(
 
   // ---- 1. the distinct list of the group's selections
   for (int i = tid; i < g.C; i += NT) msk[i] = 0u;
-  for (int i = tid; i < mpw; i += NT) mcnt[i] = 0u;
+  for (int i = tid; i < g.group; i += NT) mcnt[i] = 0u;
   __syncthreads();
   bool bad = false;
   for (int e0 = tid; e0 < GK; e0 += NT * SB) {
@@ -270,7 +274,7 @@ __global__ __launch_bounds__(W * 64) void k_attn_group(
   // The counts' sum says how many there are (a scan over the entries for it
   // took 0.6 us of a workgroup's list).
   int n_own = 0;
-  for (int m = 0; m < mpw; ++m) n_own += (int)mcnt[m];
+  for (int m = 0; m < g.group; ++m) n_own += (int)mcnt[m];
   if (n_own > 0) {  // uniform
     for (int e = tid; e < GK; e += NT) {
       const uint32_t s = own[e];
@@ -287,7 +291,7 @@ __global__ __launch_bounds__(W * 64) void k_attn_group(
     }
   }
   const int nlist = n_in + n_own;
-  if (attn_blocks && tid == 0) atomicAdd(attn_blocks, (unsigned long long)nlist);
+  if (attn_blocks && tid == 0 && gp.part == 0) atomicAdd(attn_blocks, (unsigned long long)nlist);
   __syncthreads();  // the rings may now overwrite msk / own
 
   // ---- Q^T operands of every tile, staged in LDS lane by lane (wavefront w
@@ -307,6 +311,25 @@ __global__ __launch_bounds__(W * 64) void k_attn_group(
   uint32_t tile_bits[NTILE], col_bit[NTILE];
   Acc acc[NTILE];
   const uint32_t mem_bits = (uint32_t)((1ull << mem) - 1ull);
+  int nb = nlist > wave ? (nlist - wave + W - 1) / W : 0;  // this wavefront's entries
+  if constexpr (SPLIT) {
+    // of those, the ones that this part's members selected, moved up in place
+    // (only this wavefront touches its entries) with the members' bits from 0
+    int kept = 0;
+    for (int j0 = 0; j0 < nb; j0 += 64) {
+      const int j = j0 + lane;
+      const uint32_t mm = j < nb ? (lmask[wave + W * j] >> (gp.part * mpw)) & mem_bits : 0u;
+      const uint32_t s = j < nb ? lslot[wave + W * j] : 0u;
+      const uint64_t b = ballot(mm != 0u);
+      if (mm) {
+        const int at = wave + W * (kept + lanes_below(b));
+        lslot[at] = s;
+        lmask[at] = mm;
+      }
+      kept += __builtin_popcountll(b);
+    }
+    nb = kept;
+  }
 #pragma unroll
   for (int t = 0; t < NTILE; ++t) {
     const int mi = t * MPT + n / G;
@@ -317,7 +340,6 @@ __global__ __launch_bounds__(W * 64) void k_attn_group(
   __syncthreads();  // Q^T operands staged
 
   // ---- 2./3. this wavefront's entries wave, wave + W, ... through its ring
-  const int nb = nlist > wave ? (nlist - wave + W - 1) / W : 0;
   uint8_t* ring = rings + wave * RB;
   // block j of this wavefront into ring slot b: lane fills chunk p = i*64 +
   // lane of the block: LDS row pr of its tile holds token row lds_row(pr),

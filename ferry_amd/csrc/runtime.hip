@@ -367,13 +367,14 @@ void launch_mfma(const AttnPlan& p, const dim3& grid, hipStream_t s, const AttnA
 // launch still has no more workgroups than the GPU has CUs, else all of the
 // set's.  A set of several tiles costs a workgroup their arithmetic one after
 // the other at every block; with CUs to spare its members are split between
-// workgroups of 1 or 2 tiles, each listing its own members' blocks.  They read
-// 1.1-1.4 times the set's distinct blocks between them, in part from the
-// XCD's L2 (group_part), which costs more than it gives once the CUs are full.
-// fp8, 16 members of 4 query heads (4 tiles), k 64, us per launch, 4 / 2 / 1
-// tiles per workgroup of 8 wavefronts: 8 sets 83 / 47 / 27, 64 sets
-// 85 / 50 / 31, 128 sets 91 / 57 / 64, 192 sets 95 / 115 / 101, 512 sets (4
-// wavefronts) 215 / 233 / 241.
+// workgroups of 1 or 2 tiles, each attending its own members' entries of the
+// set's list.  They read 1.1-1.4 times the set's distinct blocks between them,
+// in part from the XCD's L2 (group_part), which costs more than it gives once
+// the CUs are full.  fp8, 16 members of 4 query heads (4 tiles), k 64, us per
+// launch, whole sets / split: 8 sets 77 / 29 (1 tile), 64 sets 77 / 32 (1),
+// 96 sets 82 / 50 (2), 128 sets 85 / 58 (2); bf16, 8 members of 8: 64 sets
+// 81 / 38 (1), 128 sets 87 / 67 (2).  Past that even workgroups that listed
+// only their own members, some 3 us less, lost: 192 sets 95 / 115 (2).
 int group_tiles(int tiles, long sets, int cus) {
   for (int t = 1; t < tiles; t = t == 1 ? 2 : tiles)
     if (sets * ((tiles + t - 1) / t) <= (long)cus) return t;
@@ -405,11 +406,13 @@ int group_launch_waves(int dtype, int ntile, long gk, long sets, int cus, int fo
              ? kGroupWideWaves
              : group_waves(dtype);
 }
+// `tiles` are the whole set's, which decide the wavefronts: a member's blocks
+// are dealt to them the same way whether its set is split or not.
 template <int DT, int G, int NT, bool SPLIT>
-void launch_group(long sets, int mpw, int cus, int force, hipStream_t s, const AttnArgs& a) {
-  const long gk = (long)mpw * a.g.k, parts = (a.g.group + mpw - 1) / mpw;
+void launch_group(int tiles, long sets, int mpw, int cus, int force, hipStream_t s, const AttnArgs& a) {
+  const long gk = (long)a.g.group * a.g.k, parts = (a.g.group + mpw - 1) / mpw;
   const dim3 grid((unsigned)(SPLIT ? (sets + 7) / 8 * 8 * parts : sets));
-  if (group_launch_waves(DT, NT, gk, sets, cus, force) == kGroupWideWaves)
+  if (group_launch_waves(DT, tiles, gk, sets, cus, force) == kGroupWideWaves)
     launch_group_w<DT, G, NT, kGroupWideWaves, SPLIT>(
         grid, attn_group_lds_bytes(DT, NT, gk, kGroupWideWaves), mpw, s, a);
   else
@@ -424,15 +427,15 @@ void launch_g(const AttnPlan& p, const dim3& grid, hipStream_t s, const AttnArgs
       const int tpw = group_tiles(p.tiles, sets, p.cus);
       const int mpw = group_members(tpw, p.tiles, G, a.g.group);
       if (tpw < p.tiles) {
-        if (tpw == 1) launch_group<DT, G, 1, true>(sets, mpw, p.cus, p.group_w, s, a);
-        else launch_group<DT, G, 2, true>(sets, mpw, p.cus, p.group_w, s, a);
+        if (tpw == 1) launch_group<DT, G, 1, true>(p.tiles, sets, mpw, p.cus, p.group_w, s, a);
+        else launch_group<DT, G, 2, true>(p.tiles, sets, mpw, p.cus, p.group_w, s, a);
         return;
       }
       switch (p.tiles) {
-        case 1: launch_group<DT, G, 1, false>(sets, mpw, p.cus, p.group_w, s, a); return;
-        case 2: launch_group<DT, G, 2, false>(sets, mpw, p.cus, p.group_w, s, a); return;
-        case 3: launch_group<DT, G, 3, false>(sets, mpw, p.cus, p.group_w, s, a); return;
-        default: launch_group<DT, G, 4, false>(sets, mpw, p.cus, p.group_w, s, a); return;
+        case 1: launch_group<DT, G, 1, false>(p.tiles, sets, mpw, p.cus, p.group_w, s, a); return;
+        case 2: launch_group<DT, G, 2, false>(p.tiles, sets, mpw, p.cus, p.group_w, s, a); return;
+        case 3: launch_group<DT, G, 3, false>(p.tiles, sets, mpw, p.cus, p.group_w, s, a); return;
+        default: launch_group<DT, G, 4, false>(p.tiles, sets, mpw, p.cus, p.group_w, s, a); return;
       }
     }
   }
@@ -1128,10 +1131,7 @@ int ferry_attn_kernel(const ferry_ctx* ctx, int32_t* kind, int32_t* waves) {
   *waves = p.waves;
   if (p.grouped) {  // ferry_sparse_decode's launch: every layer's group sets
     const long sets = (long)ctx->g.n_owners * ctx->g.L * ctx->g.Hkv;
-    const int tpw = group_tiles(p.tiles, sets, p.cus);
-    *waves = group_launch_waves(p.dtype, tpw,
-                                (long)group_members(tpw, p.tiles, p.G, ctx->g.group) * ctx->g.k, sets,
-                                p.cus, p.group_w);
+    *waves = group_launch_waves(p.dtype, p.tiles, (long)ctx->g.group * ctx->g.k, sets, p.cus, p.group_w);
   }
   return FERRY_OK;
 }

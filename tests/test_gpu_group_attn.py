@@ -107,6 +107,42 @@ def test_group_kernel_member_splits(dtype, Hkv, Hq, group, n_req, L):
 
 
 @pytest.mark.parametrize("waves", [4, 8])
+@pytest.mark.parametrize("dtype,Hq,group,n_req", [
+    (F.FP8, 8, 16, 32),   # G 4, 4 tiles
+    (F.F16, 16, 8, 15),   # G 8, 4 tiles; the last group has 7 members
+    (F.BF16, 8, 12, 22),  # G 4, 3 tiles; the last group has 10 members
+    (F.BF16, 4, 13, 26),  # G 2, 2 tiles, the second of 5 members
+])
+def test_group_kernel_split_gives_the_same_bits(dtype, Hq, group, n_req, waves, monkeypatch):
+    """160 sets run whole, the same sets in launches of 120 and of 4 are split
+    between workgroups of two tiles (of 3 or more) and of one: the same bits,
+    with repeated, empty and other sets' slots in the rows."""
+    monkeypatch.setenv("FERRY_GROUP_WAVES", str(waves))
+    L, Hkv, k = 40, 2, 16
+    gp, _, _ = _twins(dtype, Hkv, Hq, group, n_req, L=L, k=k, steps=1, waves=waves)
+    slots = gp.bufs["slots"].cpu().numpy().view(np.uint32).reshape(n_req, L, Hkv, k).copy()
+    for r in range(n_req):
+        for l in range(r % 3, L, 3):
+            row = slots[r, l, r % 2]
+            row[1:4] = row[0]
+            row[5] = slots[(r + group) % n_req, l, r % 2][0]
+            row[(r + l) % k] = F.EMPTY
+            if (r + l) % 7 == 0:
+                row[:] = F.EMPTY
+    ds = torch.from_numpy(slots.view(np.int32)).cuda()
+    q = 3.0 * torch.randn((n_req, L, Hq, 128), device="cuda")
+    whole = torch.empty_like(q)
+    gp.ex.sparse_decode(q, ds, whole)
+    for step in (30, 1):
+        out = torch.full_like(q, 7.0)
+        for l0 in range(0, L, step):
+            gp.ex.sparse_decode_layers(l0, min(step, L - l0), q, ds, out)
+        torch.cuda.synchronize()
+        assert torch.equal(out, whole), step
+    assert gp.ex.stats()["device_error"] == 0
+
+
+@pytest.mark.parametrize("waves", [4, 8])
 def test_group_kernel_many_repeats_at_large_k(waves, monkeypatch):
     # 256 selections per row drawn with replacement from contexts of 40-120
     # blocks: most of a row repeats, and every repeat is an entry of its own,
