@@ -177,8 +177,8 @@ __device__ inline bool last_part(int parts, uint32_t* count, uint32_t* sh) {
 // workgroup (NT threads).  Every load goes out first, the (max, sum) pairs and
 // the thread's own pairs of outputs, so the merge waits for memory once; the
 // pairs become each part's factor 2^(m_p - M) / L in `fac` (LDS,
-// [G * kMaxParts]).  (Read one part after the other, the states of 16 parts of
-// 8 heads took 20 us, four at a time behind the factors 3.)
+// [G * kMaxParts]).  Loads past the last part repeat it and are left out of the
+// sums: a factor of 0 would make NaN of an infinite output.
 template <int G, int NT>
 __device__ inline void merge_row(const RowSplit& rs, int row, float2* fac, float* __restrict__ out) {
   constexpr int NP = (G * 64 + NT - 1) / NT;  // pairs of outputs per thread
@@ -204,7 +204,6 @@ __device__ inline void merge_row(const RowSplit& rs, int row, float2* fac, float
     // a row with no selected block (request not resident) attends to nothing: 0
     const float inv = l > 0.0f ? 1.0f / l : 0.0f;
     for (int p = 0; p < np; ++p) f[p].y = __builtin_amdgcn_exp2f(f[p].x - m) * inv;
-    for (int p = np; p < kMaxParts; ++p) f[p].y = 0.0f;
   }
   __syncthreads();
 #pragma unroll
@@ -214,6 +213,7 @@ __device__ inline void merge_row(const RowSplit& rs, int row, float2* fac, float
     float a = 0.0f, b = 0.0f;
 #pragma unroll
     for (int p = 0; p < kMaxParts; ++p) {
+      if (p >= np) break;  // launch-uniform
       const float w = fac[(t >> 6) * kMaxParts + p].y;
       a = __builtin_fmaf(v[i][p].x, w, a);
       b = __builtin_fmaf(v[i][p].y, w, b);

@@ -57,6 +57,62 @@ def test_row_split_parity(dtype, Hkv, Hq, n_req, k):
     assert p.ex.stats()["device_error"] == 0
 
 
+class _Pool:
+    def __init__(self, ex):
+        self.__cuda_array_interface__ = dict(shape=(ex.pool_slots, ex.block_bytes), typestr="|u1",
+                                             version=2, data=(ex.pool_ptrs()[0], False))
+
+
+def _whole_and_layered(dtype, Hkv, Hq, k, waves, monkeypatch, edit=None):
+    """One executor's attention over 200 rows at once (whole rows) and layer by
+    layer (10 rows: parts); edit(pool, slots) first changes stored values."""
+    monkeypatch.setenv("FERRY_ATTN_WAVES", str(waves))
+    n_req, L = 10 // Hkv, 20
+    print(f"[row split] dtype={dtype} Hkv={Hkv} Hq={Hq} k={k} waves={waves}", flush=True)
+    mb, sels = _zipf_stream(n_req, L, Hkv, k, 80, 160, 1, seed=k)
+    p = Pair(n_req, L, Hkv, Hq, k, 2 * k, mb, dtype)
+    p.step(sels[0])
+    torch.cuda.synchronize()
+    if edit:
+        edit(torch.as_tensor(_Pool(p.ex), device="cuda"), p.bufs["slots"].view(n_req, L, Hkv, k))
+    q = torch.randn((n_req, L, Hq, 128), device="cuda", generator=torch.Generator("cuda").manual_seed(k))
+    whole, parts = torch.full_like(q, 7.0), torch.full_like(q, -7.0)
+    p.ex.sparse_decode(q, p.bufs["slots"], whole)
+    for l in range(L):
+        p.ex.sparse_decode_layers(l, 1, q, p.bufs["slots"], parts)
+    torch.cuda.synchronize()
+    assert p.ex.attn_kernel()[1] == waves
+    assert p.ex.stats()["device_error"] == 0
+    return whole, parts
+
+
+@pytest.mark.parametrize("pos", [0, 1, 39])
+@pytest.mark.parametrize("dtype,Hkv,Hq,np_dtype", [(F.F32, 1, 2, torch.float32), (F.F16, 2, 2, torch.float16),
+                                                   (F.BF16, 2, 8, torch.bfloat16)])
+def test_infinite_values_in_parts_are_those_of_whole_rows(dtype, Hkv, Hq, np_dtype, pos, monkeypatch):
+    """40 blocks in 5 parts of 4 wavefronts: blocks 0 and 1 are in the first part,
+    39 in the last.  Infinities and NaN come out where a whole row has them, and
+    nowhere else."""
+    def edit(pool, slots):
+        for l in range(slots.shape[1]):
+            for r in range(slots.shape[0]):
+                v = pool[int(slots[r, l, 0, pos])].view(np_dtype).view(2, 16, 128)[1]
+                v[r % 16, 5] = float("inf")
+                v[3, 77] = -float("inf")
+
+    whole, parts = _whole_and_layered(dtype, Hkv, Hq, 40, 4, monkeypatch, edit)
+    hit = (~torch.isfinite(whole)).any()
+    assert bool(hit)
+    assert torch.equal(torch.isnan(whole), torch.isnan(parts))
+    assert torch.equal(torch.isinf(whole), torch.isinf(parts))
+    inf = torch.isinf(whole)
+    assert torch.equal(whole[inf], parts[inf])
+    if dtype != F.BF16:  # a bf16 weight's second term may be 0
+        assert bool(inf.any()) and not bool(torch.isnan(whole).any())
+    fin = torch.isfinite(whole)
+    assert float((whole - parts)[fin].abs().max()) < 1e-4
+
+
 def test_row_split_streams_and_graphs():
     """Six streams at once on one context (four have split state, the others
     run whole rows), each with queries and outputs of its own, and a graph
