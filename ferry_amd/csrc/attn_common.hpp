@@ -130,21 +130,25 @@ __device__ inline int stage_row_ids(const uint32_t* __restrict__ sl, int k, uint
   return total;
 }
 
-// ---- rows split between workgroups (launches of few rows) ----
-// `parts` workgroups attend one row's blocks, each writes its softmax state of
-// every query head to `state` (max, sum, then the 128 unnormalised outputs) and
-// adds one to the row's word of `count`; the one that finds parts - 1 there
-// merges the states and writes the row, in part order, so the result does not
-// depend on which workgroup came last.  It leaves the word 0 for the next
-// launch.  States and counts go through relaxed agent-scope atomics, which
-// complete past the XCDs' L2s (the workgroups may sit on different XCDs), and
-// each side waits for its own accesses, so no fence has to write back and
-// invalidate an L2: with those the merge of 256 workgroups took 10 us longer.
-// Both belong to one stream, so no other launch uses them meanwhile.
+// ---- rows in parts (launches of few rows) ----
+// One row's blocks are attended in `parts` parts, each by a workgroup of its
+// own (kSplitRow).  Each writes its softmax state of every query head to
+// `state` (max, sum, then the 128 unnormalised outputs) and adds one to the
+// row's word of `count`; the one that finds parts - 1 there merges the states
+// and writes the row, in part order, so the result does not depend on which
+// workgroup came last.  It leaves the word 0 for the next launch.  States and
+// counts go through relaxed agent-scope atomics, which complete past the XCDs'
+// L2s (the workgroups may sit on different XCDs), and each side waits for its
+// own accesses, so no fence has to write back and invalidate an L2.  Both
+// belong to one stream, so no other launch uses them meanwhile.
+// A launch without them (kRowAlone) attends a row's parts one after the other
+// in one workgroup, with the states in LDS: the same parts, the same merge, the
+// same bits.
+enum RowMode { kWholeRow, kSplitRow, kRowAlone };
 struct RowSplit {
   float* state;     // [rows * parts][G][kPartFloats]
   uint32_t* count;  // [rows], 0 between launches
-  int parts;        // at most kMaxParts
+  int parts;        // of every row, at most kMaxParts; 1: whole rows
 };
 constexpr int kPartFloats = 130;
 constexpr int kMaxParts = 8;
@@ -173,26 +177,30 @@ __device__ inline bool last_part(int parts, uint32_t* count, uint32_t* sh) {
   return last;
 }
 
-// The row's G * 128 outputs from its parts' states, by every thread of the last
-// workgroup (NT threads).  Every load goes out first, the (max, sum) pairs and
+// The row's G * 128 outputs from its parts' states `st` ([parts][G]
+// [kPartFloats], in LDS with LOCAL), by every thread of the workgroup that has
+// them all (NT threads).  Every load goes out first, the (max, sum) pairs and
 // the thread's own pairs of outputs, so the merge waits for memory once; the
 // pairs become each part's factor 2^(m_p - M) / L in `fac` (LDS,
 // [G * kMaxParts]).  Loads past the last part repeat it and are left out of the
 // sums: a factor of 0 would make NaN of an infinite output.
-template <int G, int NT>
-__device__ inline void merge_row(const RowSplit& rs, int row, float2* fac, float* __restrict__ out) {
+template <int G, int NT, bool LOCAL>
+__device__ inline void merge_row(const float* st, int np, float2* fac, float* __restrict__ out) {
   constexpr int NP = (G * 64 + NT - 1) / NT;  // pairs of outputs per thread
   static_assert(G * kMaxParts <= NT, "a (max, sum) pair per thread");
-  const float* st = rs.state + (size_t)row * rs.parts * G * kPartFloats;
-  const int np = rs.parts, tid = threadIdx.x;
+  const int tid = threadIdx.x;
+  auto load2 = [](const float* p) {
+    if constexpr (LOCAL) return *reinterpret_cast<const float2*>(p);
+    else return part_load2(p);
+  };
   float2 ms = {0.0f, 0.0f}, v[NP][kMaxParts];
-  if (tid < G * np) ms = part_load2(st + (size_t)tid * kPartFloats);  // tid = part * G + head
+  if (tid < G * np) ms = load2(st + (size_t)tid * kPartFloats);  // tid = part * G + head
 #pragma unroll
   for (int i = 0; i < NP; ++i) {
     const int t = min(tid + i * NT, G * 64 - 1);  // head * 64 + pair of dims
 #pragma unroll
     for (int p = 0; p < kMaxParts; ++p)
-      v[i][p] = part_load2(st + ((size_t)min(p, np - 1) * G + (t >> 6)) * kPartFloats + 2 + 2 * (t & 63));
+      v[i][p] = load2(st + ((size_t)min(p, np - 1) * G + (t >> 6)) * kPartFloats + 2 + 2 * (t & 63));
   }
   if (tid < G * np) fac[(tid % G) * kMaxParts + tid / G] = ms;
   __syncthreads();

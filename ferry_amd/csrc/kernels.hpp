@@ -118,15 +118,15 @@ __global__ void k_step_close(unsigned long long* acc, unsigned long long* host);
 
 // Vector-ALU attention (attn.hip); W wavefronts per workgroup; NT selects
 // non-temporal K/V loads.
-// SPLIT: a row's blocks are shared by rs.parts workgroups (attn_common.hpp).
-template <int DT, int G, int W, bool NT, bool SPLIT>
+// MODE: whole rows, or rows in rs.parts parts (attn_common.hpp).
+template <int DT, int G, int W, bool NT, RowMode MODE>
 __global__ void k_attn(Geo g, const float* q, const uint32_t* slots, const uint8_t* pool,
                        const float* pool_scales, float* out, float qscale, int l0, int nl, int* err,
                        RowSplit rs);
 
 // MFMA variant for GQA groups (G >= 2) of 16/8-bit KV (attn_mfma.hip); W
-// wavefronts per workgroup; NT and SPLIT as for k_attn.
-template <int DT, int G, int W, bool NT, bool SPLIT>
+// wavefronts per workgroup; NT and MODE as for k_attn (parts: bf16 only).
+template <int DT, int G, int W, bool NT, RowMode MODE>
 __global__ void k_attn_mfma(Geo g, const float* q, const uint32_t* slots, const uint8_t* pool,
                             const float* pool_scales, float* out, float qscale, int l0, int nl,
                             int* err, RowSplit rs);

@@ -302,7 +302,7 @@ struct AttnArgs {
   int l0, nl;
   int* err;
   unsigned long long* attn_blocks;  // the group kernel adds the blocks it read (or null)
-  RowSplit rs;                      // workgroups per row of the per-row kernels, and their states
+  RowSplit rs;                      // parts per row of the per-row kernels, and their states (or null)
 };
 
 // Which attention kernel runs and how many wavefronts share one (request,
@@ -342,27 +342,38 @@ AttnPlan attn_plan(const ferry_ctx* ctx) {
   return p;
 }
 
-#define FERRY_ROW_LAUNCH(KERNEL, NT)                                                                \
-  do {                                                                                              \
-    if (a.rs.parts > 1)                                                                             \
-      hipLaunchKernelGGL((KERNEL<DT, G, W, NT, true>), dim3(grid.x * (unsigned)a.rs.parts),         \
-                         dim3(W * 64), 0, s, a.g, a.q, a.slots, a.pool, a.pool_scales, a.out,       \
-                         a.qscale, a.l0, a.nl, a.err, a.rs);                                        \
-    else                                                                                            \
-      hipLaunchKernelGGL((KERNEL<DT, G, W, NT, false>), grid, dim3(W * 64), 0, s, a.g, a.q,         \
-                         a.slots, a.pool, a.pool_scales, a.out, a.qscale, a.l0, a.nl, a.err, a.rs); \
-  } while (0)
+#define FERRY_ROW_LAUNCH_M(KERNEL, NT, MODE, WGS, LDS)                                             \
+  hipLaunchKernelGGL((KERNEL<DT, G, W, NT, MODE>), dim3(WGS), dim3(W * 64), LDS, s, a.g, a.q, a.slots, \
+                     a.pool, a.pool_scales, a.out, a.qscale, a.l0, a.nl, a.err, a.rs)
+#define FERRY_ROW_LAUNCH_PARTS(KERNEL, NT)                                            \
+  if (a.rs.state)                                                                     \
+    FERRY_ROW_LAUNCH_M(KERNEL, NT, kSplitRow, grid.x * (unsigned)a.rs.parts, 0);      \
+  else                                                                                \
+    FERRY_ROW_LAUNCH_M(KERNEL, NT, kRowAlone, grid.x, (size_t)a.rs.parts * G * kPartFloats * sizeof(float))
 template <int DT, int G, int W>
 void launch_valu(const AttnPlan& p, const dim3& grid, hipStream_t s, const AttnArgs& a) {
-  if (p.nt) FERRY_ROW_LAUNCH(k_attn, true);
-  else FERRY_ROW_LAUNCH(k_attn, false);
+  if (a.rs.parts > 1) {
+    if (p.nt) { FERRY_ROW_LAUNCH_PARTS(k_attn, true); }
+    else { FERRY_ROW_LAUNCH_PARTS(k_attn, false); }
+    return;
+  }
+  if (p.nt) FERRY_ROW_LAUNCH_M(k_attn, true, kWholeRow, grid.x, 0);
+  else FERRY_ROW_LAUNCH_M(k_attn, false, kWholeRow, grid.x, 0);
 }
 template <int DT, int G, int W>
 void launch_mfma(const AttnPlan& p, const dim3& grid, hipStream_t s, const AttnArgs& a) {
-  if (p.nt) FERRY_ROW_LAUNCH(k_attn_mfma, true);
-  else FERRY_ROW_LAUNCH(k_attn_mfma, false);
+  if constexpr (DT == FERRY_BF16) {
+    if (a.rs.parts > 1) {
+      if (p.nt) { FERRY_ROW_LAUNCH_PARTS(k_attn_mfma, true); }
+      else { FERRY_ROW_LAUNCH_PARTS(k_attn_mfma, false); }
+      return;
+    }
+  }
+  if (p.nt) FERRY_ROW_LAUNCH_M(k_attn_mfma, true, kWholeRow, grid.x, 0);
+  else FERRY_ROW_LAUNCH_M(k_attn_mfma, false, kWholeRow, grid.x, 0);
 }
-#undef FERRY_ROW_LAUNCH
+#undef FERRY_ROW_LAUNCH_PARTS
+#undef FERRY_ROW_LAUNCH_M
 // Query tiles per workgroup of a prefix-group launch: the fewest for which the
 // launch still has no more workgroups than the GPU has CUs, else all of the
 // set's.  A set of several tiles costs a workgroup their arithmetic one after
@@ -504,25 +515,32 @@ int check_bufs(std::initializer_list<std::pair<const void*, const char*>> bufs) 
   return FERRY_OK;
 }
 
-// Workgroups per row of a per-row attention launch.  A CU takes in some
-// 40-60 GB/s of blocks whatever its wavefronts keep in flight (8 wavefronts or
-// rings of 4 to 8 blocks measured the same), so a launch of few rows is bound
-// by its CUs: a row is split between as many workgroups as put one on every
-// CU, and between three where that is one but three put two on most (rows in
-// (CUs / 2, 2 CUs / 3]).  More, or more rows, only add to the merge.  A part's
-// wavefronts have two blocks each, and a row at most kMaxParts parts, past
-// which the merge takes what the shorter parts give.  us per launch, whole
-// rows / split, bf16, 4 query heads, k 128: 8 rows 22.8 / 9.6 (8 parts), 64 rows
-// 32.7 / 16.7 (4), 128 rows 39.9 / 27.0 (2; 4 the same), 160 rows 40.7 / 33.0
-// (3; 2: 40.1), 192 rows 40.5 / 44.1 (2); fp32, 1 head, k 32: 8 rows 10.5 / 7.2
-// (4), 128 rows 16.5 / 13.7 (2).
-int row_parts(long rows, int k, int waves, int cus) {
-  const long p = rows * 2 <= cus ? cus / rows : rows * 3 <= 2l * cus ? 3 : 1;
-  return (int)std::max<long>(1, std::min<long>(std::min<long>(p, kMaxParts), k / (2 * waves)));
+// Parts of each row in a per-row attention launch (one workgroup each).  A CU
+// takes in some 40-60 GB/s of blocks whatever its wavefronts keep in flight (8
+// wavefronts or rings of 4 to 8 blocks measured the same), so a launch of few
+// rows is bound by its CUs: a row is split between as many workgroups as put
+// one on every CU, and between three where that is one but three put two on
+// most (rows in (CUs / 2, 2 CUs / 3]).  More, or more rows, only add to the
+// merge.  A part's wavefronts have two blocks each, and a row at most kMaxParts
+// parts, past which the merge takes what the shorter parts give.  us per launch, whole
+// rows / split, bf16, 4 query heads, k 128: 8 rows 31.2 / 10.9 (8 parts), 64 rows
+// 34.0 / 18.4 (4), 128 rows 40.8 / 28.2 (2), 160 rows 41.6 / 35.5 (3), 192 rows
+// 41.8 (44.1 in 2); fp32, 1 head, k 32: 8 rows 12.7 / 8.1 (4), 128 rows
+// 17.2 / 15.3 (2).
+// The parts change the order of a row's sums, so they are for the kernels whose
+// sums and weights keep what 32-bit sums show (fp32 weights; two bf16 terms).
+// fp8 and grouped fp16 KV round each weight to fp16 against the running maximum
+// of the wavefront, which other parts would change: their outputs would move by
+// 3e-4 with the number of rows (8 rows of 64 fp8 blocks, 4 heads: 8.0 us in
+// parts, 12.4 whole).
+int row_parts(const AttnPlan& p, long rows, int k) {
+  if (p.grouped || (p.mfma && p.dtype != FERRY_BF16)) return 1;
+  const long n = rows * 2 <= p.cus ? p.cus / rows : rows * 3 <= 2l * p.cus ? 3 : 1;
+  return (int)std::max<long>(1, std::min<long>(std::min<long>(n, kMaxParts), k / (2 * p.waves)));
 }
 
 // A stream's index among the first kSplitStreams streams that launched split
-// rows on this context; -1 (the launch then runs unsplit) for further streams,
+// rows on this context; -1 (a workgroup then takes a whole row) for further streams,
 // for a stream being captured (a graph may be replayed on any stream) and for
 // the per-thread default stream (one handle, a stream per thread).  Streams
 // are told apart by handle: hipStreamDestroy returns once the stream's work is
@@ -579,13 +597,12 @@ int decode_layers(ferry_ctx* ctx, int32_t l0, int32_t nl, const float* q, const 
   AttnArgs a{g, q, slots, ctx->pool, ctx->pool_scales, out, qscale, l0, nl, ctx->err,
              attn_blocks, RowSplit{nullptr, nullptr, 1}};
   const AttnPlan p = attn_plan(ctx);
-  if (!p.grouped) {
-    const int parts = row_parts((long)grid.x, g.k, p.waves, p.cus);
-    if (parts > 1) {
-      const int slot = stream_slot(ctx, (hipStream_t)stream);
-      if (slot >= 0)
-        a.rs = RowSplit{ctx->split_state + (size_t)slot * split_state_floats(ctx),
-                        ctx->split_count + (size_t)slot * (size_t)ctx->cus, parts};
+  a.rs.parts = row_parts(p, (long)grid.x, g.k);
+  if (a.rs.parts > 1) {
+    const int slot = stream_slot(ctx, (hipStream_t)stream);
+    if (slot >= 0) {
+      a.rs.state = ctx->split_state + (size_t)slot * split_state_floats(ctx);
+      a.rs.count = ctx->split_count + (size_t)slot * (size_t)ctx->cus;
     }
   }
   launch_attn(p, grid, (hipStream_t)stream, a);

@@ -278,10 +278,14 @@ int ferry_sparse_decode(ferry_ctx* ctx, const float* q, const uint32_t* slots,
  * one proxy kernel); for callers that report rooflines per kernel. */
 int ferry_attn_kernel(const ferry_ctx* ctx, int32_t* kind, int32_t* waves);
 
-/* Attention of layers [l0, l0 + nl) only.  A launch of few rows shares each
- * row between several workgroups, which meet in memory that the context keeps
- * for the stream (the first four streams that launch such rows; on others, and
- * while a stream is being captured, a row has one workgroup). */
+/* Attention of layers [l0, l0 + nl) only.  A launch of few (request, layer,
+ * kv head) rows of fp32, bf16 or ungrouped fp16 KV attends each row in parts,
+ * whose number follows from the rows of the launch, k and the GPU's CUs: such a
+ * row's sums run in another order than in a launch of many rows and differ from
+ * it in their last bits.  Several workgroups share a row's parts; they meet in
+ * memory that the context keeps for the stream (the first four streams that
+ * launch such rows).  On others, and while a stream is being captured, one
+ * workgroup attends the parts one after the other: slower, the same bits. */
 int ferry_sparse_decode_layers(ferry_ctx* ctx, int32_t l0, int32_t nl, const float* q,
                                const uint32_t* slots, float* out, void* stream);
 

@@ -1,7 +1,9 @@
-"""Attention launches of few rows share each row between several workgroups,
-which meet in per-stream memory: parity with the oracle at the row counts where
-the number of workgroups changes, on ragged and empty rows, and the same
-result from concurrent streams, repeated launches and a captured graph."""
+"""Attention launches of few rows attend each row in parts, shared between
+several workgroups that meet in per-stream memory, or one after the other in one
+workgroup where there is none: parity with the oracle at the row counts where
+the number of parts changes, on ragged and empty rows, infinite values as in
+whole rows, and the same bits from concurrent streams, repeated launches and a
+captured graph.  Rows whose weights are rounded to fp16 are always whole."""
 import numpy as np
 import pytest
 import torch
@@ -22,12 +24,15 @@ def _rel(a, b):
 @pytest.mark.parametrize("dtype,Hkv,Hq,n_req,k", [
     (F.F32, 1, 1, 1, 16),      # one row, 2 workgroups (256 CUs)
     (F.BF16, 2, 8, 4, 67),     # 8 rows, 8 workgroups, the wavefronts' shares uneven
-    (F.FP8, 1, 8, 33, 33),     # 33 rows, 4 workgroups
+    (F.BF16, 1, 8, 33, 33),    # 33 rows, 4 workgroups
+    (F.FP8, 1, 8, 33, 33),     # 33 rows, 1 (fp16 weights)
     (F.F16, 2, 2, 43, 24),     # 86 rows, 2 (vector ALUs)
-    (F.F16, 2, 4, 64, 40),     # 128 rows, 2
+    (F.BF16, 2, 4, 64, 40),    # 128 rows, 2
+    (F.F16, 2, 4, 64, 40),     # 128 rows, 1 (fp16 weights)
     (F.F32, 2, 4, 65, 25),     # 130 rows, 3
     (F.BF16, 2, 16, 85, 24),   # 170 rows, 3
-    (F.FP8, 3, 3, 57, 30),     # 171 rows, 1
+    (F.BF16, 3, 6, 57, 30),    # 171 rows, 1
+    (F.FP8, 3, 3, 57, 30),
 ])
 def test_row_split_parity(dtype, Hkv, Hq, n_req, k):
     mb, sels = _zipf_stream(n_req, 1, Hkv, k, 80, 160, 1, seed=k)
@@ -86,6 +91,23 @@ def _whole_and_layered(dtype, Hkv, Hq, k, waves, monkeypatch, edit=None):
     return whole, parts
 
 
+@pytest.mark.parametrize("waves", [4, 8])
+@pytest.mark.parametrize("dtype,Hkv,Hq", [(F.FP8, 2, 8), (F.FP8, 2, 2), (F.F16, 2, 4), (F.F16, 1, 8)])
+def test_fp16_weights_do_not_depend_on_the_launch(dtype, Hkv, Hq, waves, monkeypatch):
+    whole, layered = _whole_and_layered(dtype, Hkv, Hq, 48, waves, monkeypatch)
+    assert torch.equal(whole, layered)
+
+
+@pytest.mark.parametrize("waves", [4, 8])
+@pytest.mark.parametrize("dtype,Hkv,Hq", [(F.F32, 1, 1), (F.F32, 2, 16), (F.F16, 2, 2), (F.BF16, 2, 2),
+                                          (F.BF16, 2, 4), (F.BF16, 1, 8)])
+def test_parts_differ_from_whole_rows_by_rounding_only(dtype, Hkv, Hq, waves, monkeypatch):
+    # both within half the fp32 (or two-term bf16) tolerance of the 64-bit result
+    whole, parts = _whole_and_layered(dtype, Hkv, Hq, 48, waves, monkeypatch)
+    tol = 5e-5 if dtype == F.BF16 and Hq > Hkv else 1e-5
+    assert _rel(parts.cpu().numpy(), whole.cpu().numpy()) < tol
+
+
 @pytest.mark.parametrize("pos", [0, 1, 39])
 @pytest.mark.parametrize("dtype,Hkv,Hq,np_dtype", [(F.F32, 1, 2, torch.float32), (F.F16, 2, 2, torch.float16),
                                                    (F.BF16, 2, 8, torch.bfloat16)])
@@ -114,9 +136,10 @@ def test_infinite_values_in_parts_are_those_of_whole_rows(dtype, Hkv, Hq, np_dty
 
 
 def test_row_split_streams_and_graphs():
-    """Six streams at once on one context (four have split state, the others
-    run whole rows), each with queries and outputs of its own, and a graph
-    captured from one of them replayed between eager launches."""
+    """Six streams at once on one context (not all have split state), each with
+    queries and outputs of its own, then with the same queries, and a graph
+    captured from one of them replayed between eager launches: the same bits
+    from all of them."""
     n_req, Hkv, Hq, k = 8, 2, 8, 64
     mb, sels = _zipf_stream(n_req, 1, Hkv, k, 80, 160, 1, seed=3)
     p = Pair(n_req, 1, Hkv, Hq, k, 2 * k, mb, F.BF16)
@@ -134,6 +157,14 @@ def test_row_split_streams_and_graphs():
     for o, ref in zip(outs, refs):
         assert _rel(o.cpu().numpy().reshape(-1, 128), ref) < TOL[F.BF16]
     first = outs[0].clone()
+    torch.cuda.synchronize()
+    for s, o in zip(streams, outs):
+        p.ex.sparse_decode(qs[0], p.bufs["slots"], o, stream=s)
+    torch.cuda.synchronize()
+    for o in outs:
+        assert torch.equal(o, first)
+    second = torch.empty_like(first)
+    p.ex.sparse_decode(qs[1], p.bufs["slots"], second)
     g = torch.cuda.CUDAGraph()
     gout = torch.zeros_like(qs[1])
     with torch.cuda.graph(g, stream=streams[0]):
@@ -145,6 +176,6 @@ def test_row_split_streams_and_graphs():
         g.replay()
         p.ex.sparse_decode(qs[0], p.bufs["slots"], outs[0], stream=streams[0])
         torch.cuda.synchronize()
-        assert _rel(gout.cpu().numpy().reshape(-1, 128), refs[1]) < TOL[F.BF16]
+        assert torch.equal(gout, second)
         assert torch.equal(outs[0], first)
     assert p.ex.stats()["device_error"] == 0
