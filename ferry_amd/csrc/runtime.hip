@@ -16,6 +16,7 @@
 #include <initializer_list>
 #include <map>
 #include <mutex>
+#include <optional>
 #include <utility>
 #include <vector>
 
@@ -91,8 +92,14 @@ int resolve_scratch(int device, float** out) {
 }
 }  // namespace
 
-// Streams of a context that each have row-split state of their own.
+// Split states of a context, each for the launches of one stream at a time: the
+// first for the default stream, the others for streams that programs create.
 constexpr int kSplitStreams = 4;
+struct SplitSlot {
+  hipStream_t stream = nullptr;  // last user
+  hipEvent_t done = nullptr;     // recorded behind its last launch
+  bool lost = false;             // that record failed: nobody can tell when it ends
+};
 
 struct ferry_ctx {
   ferry_config cfg{};
@@ -163,9 +170,8 @@ struct ferry_ctx {
   uint32_t* trim_gen = nullptr;    // [n_owners] last ferry_members_leave that shrank the owner
   float* split_state = nullptr;    // [kSplitStreams][2 CUs][G][kPartFloats] softmax states of split rows
   uint32_t* split_count = nullptr;  // [kSplitStreams][CUs] finished parts of each row, 0 between launches
-  std::mutex split_mu;             // guards the two below
-  hipStream_t split_stream[kSplitStreams] = {};
-  int split_used = 0;
+  std::mutex split_mu;             // guards the slots past the first, from choice to record
+  SplitSlot split_slot[kSplitStreams];
   uint32_t member_calls = 0;       // ferry_members_leave calls so far (trim generations)
 
   Ring ring(int which = 0) const {
@@ -263,6 +269,8 @@ void release(ferry_ctx* c) {
   }
   for (hipEvent_t e : c->events) (void)hipEventDestroy(e);
   for (hipEvent_t e : c->booked) (void)hipEventDestroy(e);
+  for (SplitSlot& t : c->split_slot)
+    if (t.done) (void)hipEventDestroy(t.done);
   delete c;
 }
 
@@ -539,28 +547,83 @@ int row_parts(const AttnPlan& p, long rows, int k) {
   return (int)std::max<long>(1, std::min<long>(std::min<long>(n, kMaxParts), k / (2 * p.waves)));
 }
 
-// A stream's index among the first kSplitStreams streams that launched split
-// rows on this context; -1 (a workgroup then takes a whole row) for further streams,
-// for a stream being captured (a graph may be replayed on any stream) and for
-// the per-thread default stream (one handle, a stream per thread).  Streams
-// are told apart by handle: hipStreamDestroy returns once the stream's work is
-// done (measured: 42 ms behind a 42 ms kernel), so a handle that comes back
-// for a new stream has nothing of the old one in flight.
-int stream_slot(ferry_ctx* ctx, hipStream_t s) {
-  if (s == hipStreamPerThread) return -1;
-  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(s, &cap) != hipSuccess) {
-    (void)hipGetLastError();
-    return -1;
+// The split state of a launch on stream `s`: `slot`, or -1 where there is none
+// (a workgroup then takes a whole row): for a stream being captured (a graph may
+// be replayed on any stream), for the per-thread default stream (one handle, a
+// stream per thread), and while other streams use all slots.  The default
+// stream has slot 0: it is never destroyed and runs its launches in order.  Any
+// other stream keeps the slot of its handle, takes a new one or one whose last
+// launch is done, and finish(), called behind the launch, records that launch's
+// end.  A handle may come back for a new stream while the old one's launch still
+// runs, so even a slot's own handle waits for its event, in the stream.  (Event
+// and wait: 8 rows of 128 bf16 blocks 13.8 us a launch on a created stream, 11.0
+// on the default one, 31 in whole rows.)  The lock is held from choice to record.
+class SplitLease {
+ public:
+  SplitLease(ferry_ctx* ctx, hipStream_t s) : ctx_(ctx), s_(s) {
+    if (s == hipStreamPerThread) return;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &cap) != hipSuccess) {
+      (void)hipGetLastError();
+      return;
+    }
+    if (cap != hipStreamCaptureStatusNone) return;
+    if (s == nullptr || s == hipStreamLegacy) {  // two names of the default stream
+      slot = 0;
+      return;
+    }
+    lk_ = std::unique_lock<std::mutex>(ctx->split_mu);
+    const int i = choose();
+    if (i > 0) {
+      ctx->split_slot[i].stream = s;
+      slot = i;
+    } else {
+      lk_.unlock();
+    }
   }
-  if (cap != hipStreamCaptureStatusNone) return -1;
-  std::lock_guard<std::mutex> lk(ctx->split_mu);
-  for (int i = 0; i < ctx->split_used; ++i)
-    if (ctx->split_stream[i] == s) return i;
-  if (ctx->split_used == kSplitStreams) return -1;
-  ctx->split_stream[ctx->split_used] = s;
-  return ctx->split_used++;
-}
+  int finish() {
+    if (slot <= 0) return FERRY_OK;
+    SplitSlot& t = ctx_->split_slot[slot];
+    const hipError_t e = hipEventRecord(t.done, s_);
+    if (e == hipSuccess) return FERRY_OK;
+    t.lost = true;
+    return fail(FERRY_EHIP, std::string("split state: ") + hipGetErrorString(e));
+  }
+  int slot = -1;
+
+ private:
+  int choose() {
+    SplitSlot* t = ctx_->split_slot;
+    for (int i = 1; i < kSplitStreams; ++i)
+      if (t[i].done && !t[i].lost && t[i].stream == s_) {
+        if (hipStreamWaitEvent(s_, t[i].done, 0) == hipSuccess) return i;
+        (void)hipGetLastError();
+        return -1;
+      }
+    for (int i = 1; i < kSplitStreams; ++i)
+      if (!t[i].done) {
+        if (hipEventCreateWithFlags(&t[i].done, hipEventDisableTiming) == hipSuccess) return i;
+        (void)hipGetLastError();
+        t[i].done = nullptr;
+        return -1;
+      }
+    // another thread's capture is not ended by a query in relaxed mode
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    if (hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) {
+      (void)hipGetLastError();
+      return -1;
+    }
+    int free = -1;
+    for (int i = 1; i < kSplitStreams && free < 0; ++i)
+      if (!t[i].lost && hipEventQuery(t[i].done) == hipSuccess) free = i;
+    (void)hipGetLastError();  // hipErrorNotReady of the slots in use
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    return free;
+  }
+  ferry_ctx* ctx_;
+  hipStream_t s_;
+  std::unique_lock<std::mutex> lk_;
+};
 
 // Rows of a Quest selection launch that may be split between workgroups.
 uint64_t select_split_rows(const ferry_ctx* ctx) {
@@ -598,16 +661,17 @@ int decode_layers(ferry_ctx* ctx, int32_t l0, int32_t nl, const float* q, const 
              attn_blocks, RowSplit{nullptr, nullptr, 1}};
   const AttnPlan p = attn_plan(ctx);
   a.rs.parts = row_parts(p, (long)grid.x, g.k);
+  std::optional<SplitLease> lease;
   if (a.rs.parts > 1) {
-    const int slot = stream_slot(ctx, (hipStream_t)stream);
-    if (slot >= 0) {
-      a.rs.state = ctx->split_state + (size_t)slot * split_state_floats(ctx);
-      a.rs.count = ctx->split_count + (size_t)slot * (size_t)ctx->cus;
+    lease.emplace(ctx, (hipStream_t)stream);
+    if (lease->slot >= 0) {
+      a.rs.state = ctx->split_state + (size_t)lease->slot * split_state_floats(ctx);
+      a.rs.count = ctx->split_count + (size_t)lease->slot * (size_t)ctx->cus;
     }
   }
   launch_attn(p, grid, (hipStream_t)stream, a);
   HIPC(hipGetLastError());
-  return FERRY_OK;
+  return lease ? lease->finish() : FERRY_OK;
 }
 
 // A record table and its fp8 scales, allocated together or not at all: on a
@@ -1465,12 +1529,13 @@ int ferry_select_topk_layers(ferry_ctx* ctx, int32_t l0, int32_t nl, const float
             sel, l0,  nl,            g.max_blocks, ctx->err,
             ctx->cus, 1, nullptr, nullptr};
   const int parts = ctx->sel_keys ? select_parts(ctx, grid.x, Gq) : 1;
+  std::optional<SplitLease> lease;
   if (parts > 1) {
-    const int slot = stream_slot(ctx, (hipStream_t)stream);
-    if (slot >= 0) {
+    lease.emplace(ctx, (hipStream_t)stream);
+    if (lease->slot >= 0) {
       a.parts = parts;
-      a.row_keys = ctx->sel_keys + (size_t)slot * select_split_rows(ctx) * g.max_blocks;
-      a.row_count = ctx->split_count + (size_t)slot * (size_t)ctx->cus;
+      a.row_keys = ctx->sel_keys + (size_t)lease->slot * select_split_rows(ctx) * g.max_blocks;
+      a.row_count = ctx->split_count + (size_t)lease->slot * (size_t)ctx->cus;
     }
   }
   if (layer)
@@ -1478,7 +1543,7 @@ int ferry_select_topk_layers(ferry_ctx* ctx, int32_t l0, int32_t nl, const float
   else
     launch_sel_dt<false>(g.dtype, G, grid, lds, (hipStream_t)stream, a);
   HIPC(hipGetLastError());
-  return FERRY_OK;
+  return lease ? lease->finish() : FERRY_OK;
 }
 
 int ferry_select_topk(ferry_ctx* ctx, const float* q, const int32_t* ctx_blocks, int mode, uint32_t* sel,

@@ -283,9 +283,10 @@ int ferry_attn_kernel(const ferry_ctx* ctx, int32_t* kind, int32_t* waves);
  * whose number follows from the rows of the launch, k and the GPU's CUs: such a
  * row's sums run in another order than in a launch of many rows and differ from
  * it in their last bits.  Several workgroups share a row's parts; they meet in
- * memory that the context keeps for the stream (the first four streams that
- * launch such rows).  On others, and while a stream is being captured, one
- * workgroup attends the parts one after the other: slower, the same bits. */
+ * memory that the context keeps for the default stream and for three created
+ * streams at a time (a stream that comes later takes it over once the launches
+ * of another are done).  With more in use, and while a stream is being captured,
+ * one workgroup attends the parts one after the other: slower, the same bits. */
 int ferry_sparse_decode_layers(ferry_ctx* ctx, int32_t l0, int32_t nl, const float* q,
                                const uint32_t* slots, float* out, void* stream);
 

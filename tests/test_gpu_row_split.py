@@ -4,6 +4,9 @@ workgroup where there is none: parity with the oracle at the row counts where
 the number of parts changes, on ragged and empty rows, infinite values as in
 whole rows, and the same bits from concurrent streams, repeated launches and a
 captured graph.  Rows whose weights are rounded to fp16 are always whole."""
+import ctypes
+import threading
+
 import numpy as np
 import pytest
 import torch
@@ -178,4 +181,102 @@ def test_row_split_streams_and_graphs():
         torch.cuda.synchronize()
         assert torch.equal(gout, second)
         assert torch.equal(outs[0], first)
+    assert p.ex.stats()["device_error"] == 0
+
+
+class _Streams:
+    """Streams created and destroyed through the HIP runtime (torch keeps its own)."""
+
+    def __init__(self):
+        self.hip = ctypes.CDLL("libamdhip64.so.7")  # the runtime already loaded with torch
+
+    def create(self):
+        h = ctypes.c_void_p()
+        assert self.hip.hipStreamCreate(ctypes.byref(h)) == 0
+        return torch.cuda.ExternalStream(h.value)
+
+    def destroy(self, s):
+        assert self.hip.hipStreamDestroy(ctypes.c_void_p(s.cuda_stream)) == 0
+
+
+def _few_rows(k=128, seed=3):
+    n_req, Hkv, Hq = 4, 2, 8
+    mb, sels = _zipf_stream(n_req, 1, Hkv, k, 200, 400, 1, seed=seed)
+    p = Pair(n_req, 1, Hkv, Hq, k, 2 * k, mb, F.BF16)
+    p.step(sels[0])
+    qs = [torch.randn((n_req, 1, Hq, 128), device="cuda") for _ in range(8)]
+    want = [torch.empty_like(q) for q in qs]
+    for q, w in zip(qs, want):
+        p.ex.sparse_decode(q, p.bufs["slots"], w)
+    torch.cuda.synchronize()
+    return p, qs, want
+
+
+def test_streams_that_come_and_go():
+    """Streams destroyed behind queued launches, whose handles new streams may
+    get: the same bits from all.  Split state goes back to later streams: the
+    last of twenty is as fast as the first."""
+    p, qs, want = _few_rows()
+    st = _Streams()
+    outs = [torch.zeros_like(qs[0]) for _ in range(40)]
+    torch.cuda.synchronize()
+    for i in range(40):
+        s = st.create()
+        with torch.cuda.stream(s):
+            torch.cuda._sleep(200_000)
+        for _ in range(3):
+            p.ex.sparse_decode(qs[i % 8], p.bufs["slots"], outs[i], stream=s)
+        st.destroy(s)
+    torch.cuda.synchronize()
+    for i, o in enumerate(outs):
+        assert torch.equal(o, want[i % 8]), i
+    us = []
+    for i in range(20):
+        s = st.create()
+        best = float("inf")
+        for _ in range(3):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            with torch.cuda.stream(s):
+                torch.cuda._sleep(4_000_000)
+            a.record(s)
+            for _ in range(64):
+                p.ex.sparse_decode(qs[0], p.bufs["slots"], outs[0], stream=s)
+            b.record(s)
+            s.synchronize()
+            best = min(best, a.elapsed_time(b) / 64e-3)
+        us.append(best)
+        st.destroy(s)
+    print("[row split] us per launch on 20 streams:", [round(x, 1) for x in us], flush=True)
+    assert max(us[4:]) < 1.6 * min(us[:3])  # one workgroup per row takes 3 times as long
+    assert p.ex.stats()["device_error"] == 0
+
+
+@pytest.mark.parametrize("shared", [False, True])
+def test_host_threads_on_one_context(shared):
+    """Four host threads launch on one context, each on a stream of its own or
+    all on one."""
+    p, qs, want = _few_rows(k=64, seed=5)
+    one = torch.cuda.Stream()
+    errors = []
+
+    def work(t):
+        try:
+            s = one if shared else torch.cuda.Stream()
+            outs = [torch.zeros_like(q) for q in qs]
+            torch.cuda.synchronize()
+            for _ in range(50):
+                for i in range(t, t + 4):
+                    p.ex.sparse_decode(qs[i % 8], p.bufs["slots"], outs[i % 8], stream=s)
+            s.synchronize()
+            for i in range(t, t + 4):
+                assert torch.equal(outs[i % 8], want[i % 8]), (t, i)
+        except BaseException as e:  # reported by the test's own thread
+            errors.append(e)
+
+    threads = [threading.Thread(target=work, args=(t,)) for t in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors, errors
     assert p.ex.stats()["device_error"] == 0
