@@ -259,8 +259,11 @@ __global__ void k_mass_units(Geo g, const float* q, const int32_t* ctx_blocks, c
                              unsigned* counter, int parts, int l0, int nl, int max_n, int* err);
 __global__ void k_mass_reset(unsigned* counter);
 template <int G>
-__global__ void k_mass_finish(Geo g, const int32_t* ctx_blocks, const float* lsum, const float* part_ms,
-                              int parts, float* score, int nl, int max_n);
+__global__ void k_mass_lse(Geo g, const int32_t* ctx_blocks, const float* pairs, float2* state, int nl,
+                           int max_n);
+template <int G>
+__global__ void k_mass_finish(Geo g, const int32_t* ctx_blocks, const float* pairs, const float2* state,
+                              int logs, float* score, int nl, int max_n);
 template <int W>
 __global__ void k_mass_topk(Geo g, const int32_t* ctx_blocks, const float* mass, int rows, uint32_t* sel,
                             int l0, int nl, int max_n);

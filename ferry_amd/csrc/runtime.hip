@@ -1662,10 +1662,10 @@ uint64_t mass_ws_bytes(ferry_ctx* ctx, int nl, uint64_t wgs) {
 // workgroup's loads in flight, so each unit is split: about two parts per slot
 // while a part has 256 blocks (the second hides the first's start), at least
 // one part per slot while a part has 32.  us per one-layer launch, 8192 / 512
-// blocks: bf16 128 units whole 859 / 75, split in 4 696 / 61, in 2 719 / 57;
-// 32 units whole 788 / 67, in 8 190 / 26; 8 units whole 778 / 65, in 16
-// 75 / 21; 256 units whole 1314 / 100, in 2 1408 / 99; fp8 128 units whole
-// 805 / 70, in 8 427 / 55, in 4 430 / 46.
+// blocks, whole and split by this rule: bf16 128 units 859 / 76 and 750 / 66, 32
+// units 827 / 67 and 214 / 36, 8 units 813 / 66 and 83 / 27; fp8 128 units
+// 814 / 67 and 438 / 48.  256 bf16 units in 2 parts each scored in no less time
+// than whole.  The lists are the same either way.
 int mass_parts(ferry_ctx* ctx, int nl) {
   const Geo& g = ctx->g;
   const uint64_t units = (uint64_t)g.n_req * nl * g.Hkv, mb = (uint64_t)g.max_blocks;
@@ -1676,19 +1676,19 @@ int mass_parts(ferry_ctx* ctx, int nl) {
   return (int)std::max<uint64_t>(1, std::max(large, std::min(slots / units, mb / 32)));
 }
 
-// Workspace of such a launch: the log-sums (a float per block and query head
-// of every unit), the parts' (max, sum) and a score per block of every item,
-// each 256-byte aligned.
+// Workspace of such a launch: the (max, sum) of every block and query head of
+// every unit, those of every unit's kMassUnitWaves chains and a score per block
+// of every item, each 256-byte aligned.
 struct MassSplit {
-  uint64_t ms, score, bytes;  // offsets in bytes; the log-sums are at 0
+  uint64_t state, score, bytes;  // offsets in bytes; the blocks' pairs are at 0
 };
-MassSplit mass_split_layout(ferry_ctx* ctx, int nl, int parts) {
+MassSplit mass_split_layout(ferry_ctx* ctx, int nl) {
   const Geo& g = ctx->g;
   const uint64_t units = (uint64_t)g.n_req * nl * g.Hkv, G = (uint64_t)(g.Hq / g.Hkv);
   auto up = [](uint64_t b) { return (b + 255) / 256 * 256; };
   MassSplit m;
-  m.ms = up(units * g.max_blocks * G * sizeof(float));
-  m.score = m.ms + up(units * parts * G * 2 * sizeof(float));
+  m.state = up(units * g.max_blocks * G * 2 * sizeof(float));
+  m.score = m.state + up(units * kMassUnitWaves * G * 2 * sizeof(float));
   m.bytes = m.score + (uint64_t)g.n_req * nl * g.max_blocks * sizeof(float);
   return m;
 }
@@ -1698,8 +1698,7 @@ uint64_t mass_ctx_bytes(ferry_ctx* ctx) {
   const Geo& g = ctx->g;
   uint64_t need = mass_ws_bytes(ctx, g.L, mass_wgs(ctx, g.L, ~0ull));
   for (int nl = 1; nl <= g.L; ++nl) {
-    const int parts = mass_parts(ctx, nl);
-    if (parts > 1) need = std::max(need, mass_split_layout(ctx, nl, parts).bytes);
+    if (mass_parts(ctx, nl) > 1) need = std::max(need, mass_split_layout(ctx, nl).bytes);
   }
   return need;
 }
@@ -1816,13 +1815,13 @@ int launch_select_mass(ferry_ctx* ctx, int32_t l0, int32_t nl, const float* q,
   float* slices = ulds ? nullptr : reinterpret_cast<float*>(wsb + kMassCounterBytes);
   float* mass = reinterpret_cast<float*>(wsb + mass_mass_offset(ctx, wgs));
   int parts = mass_parts(ctx, nl);
-  const MassSplit split = mass_split_layout(ctx, nl, parts);
+  const MassSplit split = mass_split_layout(ctx, nl);
   if (parts > 1 && split.bytes > ws_bytes) parts = 1;
   if (parts > 1) {
     wgs = (uint64_t)g.n_req * nl * g.Hkv * parts;
     ulds = 0;
     slices = ws;
-    mass = reinterpret_cast<float*>(wsb + split.ms);
+    mass = nullptr;
   } else {
     hipLaunchKernelGGL(k_mass_reset, dim3(1), dim3(64), 0, s, counter);
     HIPC(hipGetLastError());
@@ -1850,10 +1849,16 @@ int launch_select_mass(ferry_ctx* ctx, int32_t l0, int32_t nl, const float* q,
   if (parts > 1) {  // fewer units than workgroup slots, so every item has a grid row
     float* score = reinterpret_cast<float*>(wsb + split.score);
     const dim3 fgrid((unsigned)((g.max_blocks + 255) / 256), (unsigned)(g.n_req * nl));
-    const size_t flds = (size_t)g.Hq * sizeof(float);
-#define FERRY_MASS_FINISH(GG)                                                                          \
-  hipLaunchKernelGGL(k_mass_finish<GG>, fgrid, dim3(256), flds, s, g, ctx_blocks, slices, mass, parts, \
-                     score, nl, g.max_blocks)
+    const size_t flds = (size_t)g.Hq * sizeof(float4);
+    float2* state = reinterpret_cast<float2*>(wsb + split.state);
+    const unsigned chains = (unsigned)((g.n_req * nl * g.Hkv + 7) / 8 * 8 * kMassUnitWaves);
+#define FERRY_MASS_FINISH(GG)                                                                           \
+  do {                                                                                                  \
+    hipLaunchKernelGGL(k_mass_lse<GG>, dim3(chains), dim3(64 * GG), 0, s, g, ctx_blocks, slices, state, \
+                       nl, g.max_blocks);                                                               \
+    hipLaunchKernelGGL(k_mass_finish<GG>, fgrid, dim3(256), flds, s, g, ctx_blocks, slices, state,      \
+                       mass_in_lds(ctx) ? 1 : 0, score, nl, g.max_blocks);                              \
+  } while (0)
     switch (G) {
       case 1: FERRY_MASS_FINISH(1); break;
       case 2: FERRY_MASS_FINISH(2); break;

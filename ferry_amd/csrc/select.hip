@@ -612,9 +612,84 @@ constexpr int ilog2c(int x) { return x <= 1 ? 0 : 1 + ilog2c(x / 2); }
 // (m, s) of a softmax in the exp2 domain merged with another
 __device__ inline void lse_merge(float& m, float& s, float om, float os) {
   const float mn = fmaxf(m, om);
-  s = mn == -INFINITY ? 0.0f : s * exp2f(m - mn) + os * exp2f(om - mn);
+  s = mn == -INFINITY ? 0.0f : __builtin_fmaf(s, exp2f(m - mn), os * exp2f(om - mn));
   m = mn;
 }
+
+// Chains: a unit's blocks b of one remainder b % kMassChains, merged in order,
+// and the chains' states merged after them, chain 0 first.  That is the order in
+// which a workgroup of kMassUnitWaves wavefronts takes a whole unit in, and every
+// split of a unit goes back to it, so (M, S) has the same bits.
+constexpr int kMassChains = kMassUnitWaves;
+
+// Maximum over lanes 0 .. lane of the wavefront (DPP row shifts within the
+// rows of 16 lanes, then the rows' last lanes broadcast to the rows after them).
+__device__ inline float prefix_max(float x) {
+  const int ninf = __builtin_bit_cast(int, -INFINITY);
+#define FERRY_MAX_DPP(CTRL, ROWS)                                                                  \
+  x = fmaxf(x, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(ninf, __builtin_bit_cast(int, x), \
+                                                                     CTRL, ROWS, 0xF, false)))
+  FERRY_MAX_DPP(0x111, 0xF);  // row_shr:1
+  FERRY_MAX_DPP(0x112, 0xF);
+  FERRY_MAX_DPP(0x114, 0xF);
+  FERRY_MAX_DPP(0x118, 0xF);
+  FERRY_MAX_DPP(0x142, 0xA);  // row_bcast:15 into rows 1 and 3
+  FERRY_MAX_DPP(0x143, 0xC);  // row_bcast:31 into rows 2 and 3
+#undef FERRY_MAX_DPP
+  return x;
+}
+
+// The (m, s) that lse_merge leaves of the states state(0) .. state(steps - 1)
+// one after the other, by one wavefront, in every lane.  The maxima, and with
+// them every factor, do not wait for the sums: a batch of 64 steps takes them
+// from a prefix maximum, and only one fma a step is left in order, from `tile`
+// (64 float2 of LDS, the wavefront's own).  Four batches are in flight.
+template <class State>
+__device__ inline float2 chain_state(int steps, State state, float2* tile) {
+  constexpr int NB = 4;
+  const int lane = threadIdx.x & 63;
+  steps = __builtin_amdgcn_readfirstlane(steps);
+  if (steps == 0) return {-INFINITY, 0.0f};
+  // loads past the end repeat the last step (and are not used), so that every
+  // batch issues its load and the load counter stays exact
+  auto at = [&](int i) { return state(min(i, steps - 1)); };
+  float cm = -INFINITY, s = 0.0f;
+  float2 buf[NB];
+#pragma unroll
+  for (int u = 0; u < NB; ++u) buf[u] = at(64 * u + lane);
+  for (int i0 = 0; i0 < steps; i0 += 64 * NB) {
+#pragma unroll
+    for (int u = 0; u < NB; ++u) {
+      const int left = steps - i0 - 64 * u;
+      if (left <= 0) break;  // wavefront-uniform
+      float2 v = buf[u];
+      buf[u] = at(i0 + 64 * (u + NB) + lane);
+      if (lane >= left) v = float2{-INFINITY, 0.0f};
+      const float mx = fmaxf(cm, prefix_max(v.x));
+      float before = __shfl_up(mx, 1);
+      if (lane == 0) before = cm;
+      const bool any = mx != -INFINITY;
+      tile[lane] = float2{any ? exp2f(before - mx) : 0.0f, any ? v.y * exp2f(v.x - mx) : 0.0f};
+      wave_fence();
+      if (left >= 64) {
+#pragma unroll
+        for (int j = 0; j < 64; ++j) s = __builtin_fmaf(s, tile[j].x, tile[j].y);
+      } else {
+        for (int j = 0; j < left; ++j) s = __builtin_fmaf(s, tile[j].x, tile[j].y);
+      }
+      wave_fence();
+      cm = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, mx), 63));
+    }
+  }
+  return {cm, s};
+}
+
+// A block's mass of one query head added to `acc`: from its (m, s) and the
+// head's (M, 1 / S), or from its log2-sum-exp2 and the head's.
+__device__ inline float add_mass(float acc, float m, float s, float M, float zi) {
+  return __builtin_fmaf(exp2f(m - M) * s, zi, acc);
+}
+__device__ inline float add_log_mass(float acc, float l, float L) { return acc + exp2f(l - L); }
 
 }  // namespace
 
@@ -829,10 +904,11 @@ __global__ __launch_bounds__(W * 64) void k_select_mass(Geo g, const float* __re
 //
 // parts > 1 (a launch of few units, mass_parts()): a unit's blocks are split
 // between `parts` workgroups, one part each (grid units * parts, no counter).
-// Every block's log-sums go to ws_all[unit][b][G] (G floats per 2-4 KiB
-// record), the part's (M, S) to mass[unit][part][G][2], and k_mass_finish
-// forms the masses once every part is done.  A unit per workgroup left half
-// the CUs idle at the long-context GQA shape's one-layer launch (128 units).
+// Every block's (m_b, s_b) go to ws_all[unit][b][G][2] (8 G bytes per 2-4 KiB
+// record); k_mass_lse merges them in the order of a whole unit
+// and k_mass_finish forms the masses, so the masses are a whole unit's bit for
+// bit.  A unit per workgroup left half the CUs idle at the long-context GQA
+// shape's one-layer launch (128 units).
 template <int DT, int G, int W, int U>
 __global__ __launch_bounds__(W * 64) void k_mass_units(
     Geo g, const float* __restrict__ q, const int32_t* __restrict__ ctx_blocks,
@@ -891,7 +967,7 @@ __global__ __launch_bounds__(W * 64) void k_mass_units(
     const int part = split ? (int)(blockIdx.x % (unsigned)parts) : 0;
     const int per = (nb + parts - 1) / parts;
     const int lo = min(nb, part * per), hi = min(nb, lo + per);
-    if (split) ws = ws_all + (size_t)unit * max_n * G;
+    if (split) ws = ws_all + (size_t)unit * max_n * G * 2;
     const SetRecords recs((uint64_t)rl * g.Hkv + h, (uint64_t)g.max_blocks, kt_mod);
     // ---- Q^T operand: k-step ks, this lane's 8 dims, head n (0 for pad heads)
     uint32_t qb[NQ][4][4];
@@ -973,18 +1049,17 @@ __global__ __launch_bounds__(W * 64) void k_mass_units(
         float e = (exp2f(x[0] - m) + exp2f(x[1] - m)) + (exp2f(x[2] - m) + exp2f(x[3] - m));
         e = sum_over_groups(e);
         if (head_lane) {
-          if (split) {
-            ws[(size_t)b * G + n] = m + log2f(e);
-          } else if (in_lds) {
+          if (in_lds) {
             lws[b * G + n] = m + log2f(e);  // the block's log2-sum-exp2
           } else {
             ws[((size_t)b * G + n) * 2] = m;
             ws[((size_t)b * G + n) * 2 + 1] = e;
           }
-          lse_merge(run_m, run_s, m, e);
+          if (!split) lse_merge(run_m, run_s, m, e);
         }
       }
     }
+    if (split) break;  // launch-uniform: one part per workgroup
     // the workgroup's (M, S) of every query head
     if (head_lane) {
       red_m[wave][n] = run_m;
@@ -994,28 +1069,22 @@ __global__ __launch_bounds__(W * 64) void k_mass_units(
     if (tid < G) {
       float mm = -INFINITY, ss = 0.0f;
       for (int w = 0; w < W; ++w) lse_merge(mm, ss, red_m[w][tid], red_s[w][tid]);
-      if (split) {  // k_mass_finish merges the parts' (M, S)
-        float* ms = mass + ((size_t)blockIdx.x * G + tid) * 2;
-        ms[0] = mm;
-        ms[1] = ss;
-      }
       lse_m[tid] = mm;
       lse_zi[tid] = 1.0f / ss;
       lse_l[tid] = mm + log2f(ss);  // the unit's log2-sum-exp2
     }
-    if (split) break;  // launch-uniform: one part per workgroup
     __syncthreads();
     float* mrow = mass + (size_t)unit * max_n;
     for (int b = tid; b < nb; b += NT) {
       float acc = 0.0f;
       if (in_lds) {
 #pragma unroll
-        for (int gq = 0; gq < G; ++gq) acc += exp2f(lws[b * G + gq] - lse_l[gq]);
+        for (int gq = 0; gq < G; ++gq) acc = add_log_mass(acc, lws[b * G + gq], lse_l[gq]);
       } else {
 #pragma unroll
         for (int gq = 0; gq < G; ++gq)
-          acc += exp2f(ws[((size_t)b * G + gq) * 2] - lse_m[gq]) * ws[((size_t)b * G + gq) * 2 + 1] *
-                 lse_zi[gq];
+          acc = add_mass(acc, ws[((size_t)b * G + gq) * 2], ws[((size_t)b * G + gq) * 2 + 1], lse_m[gq],
+                         lse_zi[gq]);
       }
       mrow[b] = acc;
     }
@@ -1026,28 +1095,53 @@ __global__ void k_mass_reset(unsigned* counter) {
   if (blockIdx.x == 0 && threadIdx.x == 0) *counter = 0u;
 }
 
-// k_mass_finish (after a k_mass_units launch with parts > 1): the score of
-// every block of every (request, layer) item, one thread per block.  A query
-// head's log2-sum-exp2 L is merged over its parts once per workgroup; the
-// block's score is exp2(l_b - L) summed over the query heads of a kv head, then
-// over the kv heads, in k_mass_topk's order.  Grid (blocks / 256, items);
-// dynamic LDS: a float per query head of the layer.
+// k_mass_lse (after a k_mass_units launch with parts > 1): one workgroup per
+// chain of a unit, a wavefront per query head; state[unit][chain][head] = (m, s)
+// of the chain.  The chains of a unit, which read the same lines, are 8
+// workgroups apart: on one XCD, behind one L2.  Grid: units rounded up to 8, times
+// kMassChains.  Bound by instructions (the scan, the two exp2 and the 64 fmas of
+// each batch): 128 units of 8192 blocks and 4 heads 24 us, beside 695 of their
+// scoring, of 512 blocks 4.8 beside 46.
+template <int G>
+__global__ __launch_bounds__(64 * G) void k_mass_lse(Geo g, const int32_t* __restrict__ ctx_blocks,
+                                                     const float* __restrict__ pairs,
+                                                     float2* __restrict__ state, int nl, int max_n) {
+  __shared__ __attribute__((aligned(16))) float2 tile[G][64];
+  const int h = threadIdx.x >> 6, c = blockIdx.x / 8 % kMassChains;
+  const int unit = blockIdx.x / (8 * kMassChains) * 8 + blockIdx.x % 8;
+  if (unit >= g.n_req * nl * g.Hkv) return;  // workgroup-uniform
+  int nb = ctx_blocks[unit / g.Hkv / nl];
+  if (nb < 0 || nb > max_n || nb > g.max_blocks) nb = 0;  // k_mass_units latched the error
+  if (nb <= g.k) return;                                   // workgroup-uniform
+  const float2* p = reinterpret_cast<const float2*>(pairs) + ((size_t)unit * max_n + c) * G + h;
+  const float2 st = chain_state(nb > c ? (nb - c + kMassChains - 1) / kMassChains : 0,
+                                [&](int i) { return p[(size_t)i * kMassChains * G]; }, tile[h]);
+  if ((threadIdx.x & 63) == 0) state[((size_t)unit * kMassChains + c) * G + h] = st;
+}
+
+// k_mass_finish (after k_mass_lse): the score of every block of every (request,
+// layer) item, one thread per block.  A query head's chains are merged once per
+// workgroup, in order; the block's mass is summed over the query heads of a kv
+// head, in the form whole units of the context use (`logs`: from the block's
+// log-sum), then over the kv heads, in k_mass_topk's order.  Grid (blocks / 256,
+// items); dynamic LDS: a float4 per query head of the layer.
 template <int G>
 __global__ __launch_bounds__(256) void k_mass_finish(Geo g, const int32_t* __restrict__ ctx_blocks,
-                                                     const float* __restrict__ lsum,
-                                                     const float* __restrict__ part_ms, int parts,
+                                                     const float* __restrict__ pairs,
+                                                     const float2* __restrict__ state, int logs,
                                                      float* __restrict__ score, int nl, int max_n) {
-  extern __shared__ float lse[];  // [Hkv * G]
+  extern __shared__ float4 lse_sh[];  // [Hkv * G]
   const int tid = threadIdx.x, item = blockIdx.y;
   int nb = ctx_blocks[item / nl];
   if (nb < 0 || nb > max_n || nb > g.max_blocks) nb = 0;  // k_mass_units latched the error
   if (nb <= g.k || (int)blockIdx.x * 256 >= nb) return;    // workgroup-uniform
   const size_t u0 = (size_t)item * g.Hkv;
   for (int i = tid; i < g.Hkv * G; i += 256) {
-    const float* ms = part_ms + ((u0 + i / G) * parts * G + i % G) * 2;
+    const float2* st = state + (u0 + i / G) * kMassChains * G + i % G;
     float mm = -INFINITY, ss = 0.0f;
-    for (int p = 0; p < parts; ++p) lse_merge(mm, ss, ms[(size_t)p * G * 2], ms[(size_t)p * G * 2 + 1]);
-    lse[i] = mm + log2f(ss);
+#pragma unroll
+    for (int c = 0; c < kMassChains; ++c) lse_merge(mm, ss, st[c * G].x, st[c * G].y);
+    lse_sh[i] = float4{mm, 1.0f / ss, mm + log2f(ss), 0.0f};
   }
   __syncthreads();
   const int b = blockIdx.x * 256 + tid;
@@ -1055,10 +1149,14 @@ __global__ __launch_bounds__(256) void k_mass_finish(Geo g, const int32_t* __res
   float s = 0.0f;
 #pragma unroll 4
   for (int hh = 0; hh < g.Hkv; ++hh) {
-    const float* l = lsum + ((u0 + hh) * max_n + b) * G;
+    const float2* p = reinterpret_cast<const float2*>(pairs) + ((u0 + hh) * max_n + b) * G;
     float acc = 0.0f;
 #pragma unroll
-    for (int gq = 0; gq < G; ++gq) acc += exp2f(l[gq] - lse[hh * G + gq]);
+    for (int gq = 0; gq < G; ++gq) {
+      const float2 v = p[gq];
+      const float4 z = lse_sh[hh * G + gq];
+      acc = logs ? add_log_mass(acc, v.x + log2f(v.y), z.z) : add_mass(acc, v.x, v.y, z.x, z.y);
+    }
     s = hh == 0 ? acc : s + acc;
   }
   score[(size_t)item * max_n + b] = s;
@@ -1146,8 +1244,9 @@ FERRY_MASS_UNITS_INST_G(FERRY_FP8_E4M3)
                                           int, int);
 FERRY_MASS_TOPK_INST(kMassTopkWaves)
 FERRY_MASS_TOPK_INST(kMassTopkWideWaves)
-#define FERRY_MASS_FINISH_INST(G)                                                                  \
-  template __global__ void k_mass_finish<G>(Geo, const int32_t*, const float*, const float*, int, \
+#define FERRY_MASS_FINISH_INST(G)                                                                    \
+  template __global__ void k_mass_lse<G>(Geo, const int32_t*, const float*, float2*, int, int);       \
+  template __global__ void k_mass_finish<G>(Geo, const int32_t*, const float*, const float2*, int,    \
                                             float*, int, int);
 FERRY_MASS_FINISH_INST(1)
 FERRY_MASS_FINISH_INST(2)

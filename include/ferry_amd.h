@@ -389,9 +389,9 @@ int ferry_select_topk_layers(ferry_ctx* ctx, int32_t l0, int32_t nl, const float
  * content changes.  The selection keeps each block's mass per kv head (16-bit
  * and fp8 K, about n_req * L * kv_heads * max_blocks * 4 bytes) and, for fp32
  * and fp8 K or where max_blocks * q_heads / kv_heads floats exceed 144 KiB of
- * LDS, each block's softmax max and sum, and for launches of few (request,
- * layer, kv head) units, whose blocks several workgroups share, each block's
- * log-sum per query head, in a workspace of the context allocated by
+ * LDS, or where a launch has few (request, layer, kv head) units, whose blocks
+ * several workgroups then share, each block's softmax max and sum per query
+ * head, in a workspace of the context allocated by
  * ferry_ktiles_build, so two ferry_select_mass calls on one
  * context must not run concurrently. */
 int ferry_ktiles_build(ferry_ctx* ctx, uint64_t n_records, void* stream);

@@ -172,6 +172,53 @@ def test_select_mass_split_and_whole_units(dtype, Hkv, Hq, ws, monkeypatch):
     assert p.ex.stats()["device_error"] == 0
 
 
+_TORCH = {F.F32: torch.float32, F.F16: torch.float16, F.BF16: torch.bfloat16, F.FP8: torch.float8_e4m3fn}
+
+
+def near_tie_executor(dtype, n_req, L, Hkv, Hq, k, mb, seed=0, base=64.0, spread=0.05):
+    """An executor and queries whose blocks' scores lie close together: logits of
+    about 16 base (log2 units) that differ in one dimension (by 0.13 spread) and,
+    for fp8, in the block's scale.  What a rounding of the sums changes shows in
+    the lists."""
+    ex = F.Executor(n_req, L, Hkv, k, 8, mb, q_heads=Hq, dtype=dtype, host_blocks=4099)
+    g = torch.Generator().manual_seed(seed)
+    kv = torch.ones((4099, 2, 16, 128))
+    kv[:, 0, :, 0] = torch.randn((4099, 16), generator=g)
+    host, scales = ex.hosttier_array()
+    torch.from_numpy(host).copy_(kv.to(_TORCH[dtype]).view(torch.uint8).view(-1))
+    if scales is not None:
+        torch.from_numpy(scales).view(4099, 2).copy_(1.0 + 1e-5 * torch.randn((4099, 2), generator=g))
+    ex.ktiles_build()
+    q = base * (1.0 + 0.01 * torch.randn((n_req, L, Hq, 128), generator=g))
+    q[..., 0] = spread * torch.randn((n_req, L, Hq), generator=g)
+    return ex, q.cuda()
+
+
+@pytest.mark.parametrize("G", [1, 2, 4, 8])
+@pytest.mark.parametrize("dtype,ws", [(F.BF16, "lds"), (F.F16, "hbm"), (F.FP8, "lds")])
+def test_split_units_give_the_lists_of_whole_units(dtype, ws, G, monkeypatch):
+    """Units split between workgroups (64 of them, a layer at a time), fewer and
+    longer parts (16 at a time) and whole units (320 at once) merge a block's
+    softmax states in one order: the same lists, with near-ties at the k-th
+    block."""
+    monkeypatch.setenv("FERRY_MASS_WS", ws)
+    n_req, L, Hkv, k, mb = 8, 5, 8, 16, 1003
+    print(f"[mass] split = whole dtype={dtype} G={G} ws={ws}", flush=True)
+    ex, q = near_tie_executor(dtype, n_req, L, Hkv, Hkv * G, k, mb)
+    ctx = torch.tensor([1003, 1000, 997, 513, 65, 17, 16, 0], dtype=torch.int32, device="cuda")
+    sels = []
+    for step in (5, 1, 2):
+        sel = torch.full((n_req, L, Hkv, k), -7, dtype=torch.int32, device="cuda")
+        for l0 in range(0, L, step):
+            ex.select_mass(q, ctx, sel, layers=(l0, min(step, L - l0)))
+        sels.append(sel)
+    torch.cuda.synchronize()
+    assert ex.stats()["device_error"] == 0
+    assert torch.equal(sels[0], sels[1])
+    assert torch.equal(sels[0], sels[2])
+    assert sels[0][0, 0, 0].unique().numel() == k
+
+
 @pytest.mark.parametrize("Hq", [2, 16])
 def test_select_mass_fp32_workgroup_sizes(Hq):
     """fp32 items take 8 wavefronts in launches of few items and 4 in larger

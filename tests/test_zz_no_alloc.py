@@ -2,10 +2,10 @@
 selection with its workspace (per-workgroup (max, sum) slices and, for 16-bit
 and fp8 K, the per-kv-head block masses) in the library's static per-GPU array
 instead of the context's, through the C-ABI.  Its page lists must equal
-ferry_select_mass's bit for bit (same kernels, same arithmetic per (request,
-layer, kv head) unit and (request, layer) item, only fewer workgroups sharing
-the work and, where the masses of every layer do not fit, layer ranges run one
-after the other) on two calls
+ferry_select_mass's bit for bit (the same arithmetic per (request, layer, kv
+head) unit and (request, layer) item, in the same order, whether a launch splits
+its units or not; only fewer workgroups share the work and, where the masses of
+every layer do not fit, layer ranges run one after the other) on two calls
 in a row, the second with smaller inputs, which finds the first call's data
 still in the shared array, and on a second, smaller executor on the same
 GPU.  It is collected last: it must pass alone in a fresh process and after
@@ -15,6 +15,8 @@ import pytest
 import torch
 
 import ferry_amd as F
+
+from test_gpu_mass import near_tie_executor
 
 pytestmark = pytest.mark.gpu
 
@@ -92,6 +94,24 @@ def test_noalloc_select_mass_layer_ranges():
     a, b = _both(ex, q, ctx, (B, L, Hkv, k))
     assert np.array_equal(a, b)
     assert np.all(a[2:, ..., :k] >= 0) and np.all(a[1, ..., k - 3:] == -1)
+    ex.close()
+
+
+@pytest.mark.parametrize("dtype,B,Hkv,G,L,mb", [
+    (F.BF16, 16, 8, 1, 9, 15360),  # ranges of 8 layers and of 1, whose 128 units are split
+    (F.FP8, 32, 8, 8, 1, 8192),    # 256 units, split in the context's workspace, whole in the array
+])
+def test_noalloc_decides_its_launches_for_itself(dtype, B, Hkv, G, L, mb, monkeypatch):
+    """Where the two entry points split or widen different launches, the lists
+    are the same, with near-ties at the k-th block."""
+    monkeypatch.delenv("FERRY_MASS_WS", raising=False)
+    k = 64
+    print(f"[noalloc] launches dtype={dtype} B={B} Hkv={Hkv} G={G} L={L} max_blocks={mb}", flush=True)
+    ex, q = near_tie_executor(dtype, B, L, Hkv, Hkv * G, k, mb)
+    ctx = np.full(B, mb, np.int32)
+    ctx[1::3] = mb - 1001
+    a, b = _both(ex, q.cpu().numpy(), ctx, (B, L, Hkv, k))
+    assert np.array_equal(a, b)
     ex.close()
 
 
