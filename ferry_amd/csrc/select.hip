@@ -709,6 +709,10 @@ __device__ inline float add_log_mass(float acc, float l, float L) { return acc +
 // The scores then go through the same radix top-k as the Quest method and the
 // layer's list is written to every kv head's row.  Dynamic LDS: max_n floats;
 // workspace: max_n * G * 2 floats per workgroup.
+// With four wavefronts the running (M, S) are chains of the blocks of one
+// remainder b % (4 U), merged wavefront by wavefront.  Eight wavefronts leave
+// them to a pass over the workspace that walks those chains in that order
+// (chain_state), so both give the same bits.
 template <int DT, int G, int W>
 __global__ __launch_bounds__(W * 64) void k_select_mass(Geo g, const float* __restrict__ q,
                                                         const int32_t* __restrict__ ctx_blocks,
@@ -731,7 +735,11 @@ __global__ __launch_bounds__(W * 64) void k_select_mass(Geo g, const float* __re
   __shared__ uint32_t hist[256];
   __shared__ uint32_t wtot[2 * W];
   __shared__ uint32_t sh[3];
-  __shared__ float xl[W][XW];
+  constexpr bool CHAINS = W > 4;
+  constexpr int NCH = 4 * U;  // chains
+  static_assert(!CHAINS || NCH * G <= NE, "a red_m entry per chain and head");
+  // logits, and then chain_state's tile
+  __shared__ __attribute__((aligned(16))) float xl[W][CHAINS && XW < 128 ? 128 : XW];
   __shared__ float red_m[NE], red_s[NE], lse_m[G], lse_zi[G];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int p = lane % LPT, t = lane / LPT;
@@ -824,14 +832,25 @@ __global__ __launch_bounds__(W * 64) void k_select_mass(Geo g, const float* __re
               const int gq = (idx >> 4) % G;
               ws[((size_t)b * G + gq) * 2] = m;
               ws[((size_t)b * G + gq) * 2 + 1] = sm;
-              lse_merge(run_m[rr], run_s[rr], m, sm);
+              if constexpr (!CHAINS) lse_merge(run_m[rr], run_s[rr], m, sm);
             }
           }
         }
         wave_fence();
       }
       // the workgroup's (M, S) of every query head
-      if ((lane & 15) == 0) {
+      if constexpr (CHAINS) {
+        __syncthreads();  // every block's state is in the workspace
+        const float2* st = reinterpret_cast<const float2*>(ws);
+        for (int e = wave; e < NCH * G; e += W) {  // chain e / G of head e % G
+          const int c = e / G;
+          const float2 ms = chain_state(
+              n > c ? (n - c + NCH - 1) / NCH : 0,
+              [&](int i) { return st[(size_t)(c + NCH * i) * G + e % G]; },
+              reinterpret_cast<float2*>(xl[wave]));
+          if (lane == 0) red_m[e] = ms.x, red_s[e] = ms.y;
+        }
+      } else if ((lane & 15) == 0) {
 #pragma unroll
         for (int rr = 0; rr < R; ++rr) {
           red_m[(wave * 4 + (lane >> 4)) * R + rr] = run_m[rr];
@@ -841,10 +860,13 @@ __global__ __launch_bounds__(W * 64) void k_select_mass(Geo g, const float* __re
       __syncthreads();
       if (tid < G) {
         float mm = -INFINITY, ss = 0.0f;
-        for (int e = 0; e < NE; ++e) {
+        for (int e = 0; e < 16 * R; ++e) {
           const int c = e / R, rr = e % R;  // entry of lane 16 (c % 4) of wave c / 4, tile row rr
           const int idx = (c % 4) * 16 + 64 * rr;
-          if (idx < XW && (idx >> 4) % G == tid) lse_merge(mm, ss, red_m[e], red_s[e]);
+          if (idx < XW && (idx >> 4) % G == tid) {
+            const int at = CHAINS ? (c / 4 + 4 * (idx / (16 * G))) * G + tid : e;
+            lse_merge(mm, ss, red_m[at], red_s[at]);
+          }
         }
         lse_m[tid] = mm;
         lse_zi[tid] = 1.0f / ss;

@@ -242,6 +242,25 @@ def test_select_mass_fp32_workgroup_sizes(Hq):
     assert p.ex.stats()["device_error"] == 0
 
 
+@pytest.mark.parametrize("G", [1, 2, 4, 8])
+def test_fp32_lists_do_not_depend_on_the_wavefronts(G):
+    """70 fp32 items run with 8 wavefronts, 280 with 4: the same lists, with
+    near-ties at the k-th block and contexts that end anywhere in a pass."""
+    n_req, L, Hkv, k, mb = 70, 4, 2, 150, 1333
+    ex, q = near_tie_executor(F.F32, n_req, L, Hkv, Hkv * G, k, mb, base=1.0, spread=2e-3)
+    ctx = torch.arange(n_req, dtype=torch.int32, device="cuda") * 19 % (mb + 1)
+    ctx[0] = mb
+    sels = []
+    for step in (4, 1):
+        sel = torch.full((n_req, L, Hkv, k), -7, dtype=torch.int32, device="cuda")
+        for l0 in range(0, L, step):
+            ex.select_mass(q, ctx, sel, layers=(l0, step))
+        sels.append(sel)
+    torch.cuda.synchronize()
+    assert torch.equal(sels[0], sels[1])
+    assert ex.stats()["device_error"] == 0
+
+
 @pytest.mark.parametrize("dtype", [F.F16, F.FP8])
 def test_zero_query_takes_the_lowest_ids(dtype):
     """q = 0: every token gets probability 1/(16 ctx), every block the same

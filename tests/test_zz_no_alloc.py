@@ -100,6 +100,7 @@ def test_noalloc_select_mass_layer_ranges():
 @pytest.mark.parametrize("dtype,B,Hkv,G,L,mb", [
     (F.BF16, 16, 8, 1, 9, 15360),  # ranges of 8 layers and of 1, whose 128 units are split
     (F.FP8, 32, 8, 8, 1, 8192),    # 256 units, split in the context's workspace, whole in the array
+    (F.F32, 64, 2, 2, 3, 4096),    # 192 items of 4 wavefronts, 8 in launches of up to 128
 ])
 def test_noalloc_decides_its_launches_for_itself(dtype, B, Hkv, G, L, mb, monkeypatch):
     """Where the two entry points split or widen different launches, the lists
