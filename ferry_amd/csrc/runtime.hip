@@ -636,10 +636,11 @@ uint64_t select_split_rows(const ferry_ctx* ctx) {
 // pass of its wavefronts (kSelectPass blocks); 1 for rows that score in less
 // than the keys' way through memory takes (2 us: under 2048 bounds).  As in the
 // attention, only more CUs take in a row's records faster.  us per launch,
-// whole rows (of 16 wavefronts) / split, 8192 blocks: bf16, 4 heads: 8 rows
-// 109 / 23, 64 rows 121 / 65, 128 rows 129 / 106; 2048 blocks: fp16, 1 head, 32 rows 21 / 14;
-// 512 blocks: bf16, 4 heads, 64 rows 14.8 / 13.7, fp16, 1 head, 32 rows
-// 10.3 / 10.7 (so left whole).
+// whole rows (of 16 wavefronts) / split: bf16, 4 heads, 8192 blocks, 8 rows
+// 109 / 24, 64 rows 121 / 60, 128 rows 129 / 101-106; 512 blocks (2048 bounds)
+// 8 rows 13.1 / 12.6, 64 rows 13.9 / 14.1, 128 rows 15.0 / 14.9; fp16, 1 head, 2048
+// blocks 32 rows 24 / 15, 128 rows 33.5 / 31.5, 512 blocks (left whole) 64 rows
+// 10.4 / 12.2.
 int select_parts(const ferry_ctx* ctx, unsigned rows, int heads) {
   const unsigned mb = (unsigned)ctx->g.max_blocks, cus = (unsigned)ctx->cus;
   if (rows > select_split_rows(ctx) || mb * (unsigned)heads < 2048u) return 1;
@@ -1449,19 +1450,29 @@ struct SelArgs {
   uint32_t* row_count;
 };
 
-// Wavefronts of a Quest selection workgroup (one row each).  A launch of no
-// more rows than CUs has one workgroup per CU whatever its size, so a row's
-// records are scored by 16 wavefronts: four leave 8 KiB in flight per CU and
-// the row's arithmetic on one wavefront per SIMD.  Up to two rows per CU, 8;
-// more rows fill the CUs with workgroups of 4, whose top-k phases overlap the
-// others' loads better; so do fp32 rows past one per CU, which wait for memory
-// (384 rows of 8192 blocks, 2 heads: 652 with 4, 710 with 8).  bf16, 4 query heads per kv head, 8192 blocks, us per
-// launch with 4 / 8 / 16 wavefronts: 128 rows 293 / 169 / 131, 256 rows
-// 321 / 201 / 176, 512 rows 379 / 344 / 345, 1024 rows 668 / 667 / 674; 512
-// blocks: 256 rows 24 / 18 / 17, 512 rows 30 / 27 / 34, 1024 rows 47 / 50 / 65.
-int select_waves(int dtype, unsigned rows, int cus) {
-  if (rows <= (unsigned)cus) return 16;
-  return dtype != FERRY_F32 && rows <= 2u * (unsigned)cus ? 8 : 4;
+// Wavefronts of a Quest selection workgroup (one row each; `heads` per kv head,
+// contexts of up to `mb` blocks).  A wavefront's pass takes 16 blocks, so
+// contexts of up to 64 give no more than four of them something to score, and
+// the others only lengthen the top k (64 rows of 64 blocks, bf16, 4 heads: 7.4
+// us with 4, 8.0 with 8, 10.4 with 16).  A launch of no more rows than CUs has
+// one workgroup per CU whatever its size, so a row's records are scored by 16
+// wavefronts, or 8 where 16 have less than two passes (64 rows of 256 blocks
+// 13.2 / 10.4 / 10.9, of 384 18.2 / 13.0 / 14.1, 8 rows of 768 - / 17.9 / 16.2)
+// or where fp32 rows of a whole layer wait for memory (128 rows of 1024 blocks,
+// 8 kv heads of 8 heads 382 / 273 / 293, of 4 266 / 270 / 276).  Up to two rows
+// per CU, 8; more rows fill the CUs with workgroups of 4, whose top-k phases
+// overlap the others' loads better.  So do the rows past one per CU that are
+// bound by memory: fp32 (384 rows of 8192 blocks, 2 heads: 652 with 4, 710 with
+// 8) and 16-bit layers of one head per kv head (300 rows of 1024 blocks, 32 kv
+// heads: 800 / 990 / 968; with 2 heads and 8 kv heads 267 / 233 / 244).  bf16, 4
+// heads, 8192 blocks: 256 rows 321 / 201 / 176, 512 rows 379 / 344 / 345, 1024
+// rows 668 / 667 / 674; 512 blocks: 256 rows 24 / 18 / 17, 512 rows 30 / 27 / 34.
+int select_waves(int dtype, bool layer, int heads, int mb, unsigned rows, int cus) {
+  if (mb <= 64) return 4;
+  const bool f32 = dtype == FERRY_F32;
+  if (rows <= (unsigned)cus) return mb < 512 || (layer && f32) ? 8 : 16;
+  const bool memory = f32 || (layer && heads == 1 && dtype != FERRY_FP8_E4M3);
+  return !memory && rows <= 2u * (unsigned)cus ? 8 : 4;
 }
 
 template <int DT, int G, bool LAYER>
@@ -1474,7 +1485,7 @@ void launch_sel(const dim3& grid, size_t lds, hipStream_t s, const SelArgs& a) {
     FERRY_SEL_LAUNCH(16, true);
     return;
   }
-  switch (select_waves(DT, grid.x, a.cus)) {
+  switch (select_waves(DT, LAYER, G, a.max_n, grid.x, a.cus)) {
     case 16: FERRY_SEL_LAUNCH(16, false); return;
     case 8: FERRY_SEL_LAUNCH(8, false); return;
     default: FERRY_SEL_LAUNCH(4, false); return;

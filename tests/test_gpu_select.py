@@ -67,21 +67,30 @@ def test_select_topk_bit_exact(dtype, Hkv, Hq, host_blocks, mode):
     assert p.ex.stats()["device_error"] == 0
 
 
-@pytest.mark.parametrize("dtype,Hkv,Hq,mode,n_req", [
-    (F.BF16, 2, 8, F.TOPK_PER_HEAD, 100),
-    (F.FP8, 2, 16, F.TOPK_PER_HEAD, 100),
-    (F.F32, 2, 2, F.TOPK_PER_HEAD, 100),
-    (F.F16, 2, 4, F.TOPK_LAYER_MAX, 200),
+@pytest.mark.parametrize("dtype,Hkv,Hq,mode,n_req,mb", [
+    (F.BF16, 2, 8, F.TOPK_PER_HEAD, 100, 600),
+    (F.FP8, 2, 16, F.TOPK_PER_HEAD, 100, 600),
+    (F.F32, 2, 2, F.TOPK_PER_HEAD, 100, 600),
+    (F.F16, 2, 16, F.TOPK_LAYER_MAX, 200, 600),  # 8 heads per kv head
+    (F.F32, 2, 16, F.TOPK_LAYER_MAX, 200, 600),  # fp32 layers: 8 wavefronts, then 4
+    (F.BF16, 3, 3, F.TOPK_LAYER_MAX, 200, 600),  # one head per kv head: 16, then 4
+    (F.BF16, 2, 8, F.TOPK_PER_HEAD, 100, 270),   # up to 511 blocks: 8, 8, 4
+    (F.F32, 2, 2, F.TOPK_PER_HEAD, 100, 270),
+    (F.F16, 2, 4, F.TOPK_LAYER_MAX, 200, 270),
+    (F.BF16, 2, 8, F.TOPK_PER_HEAD, 100, 64),    # up to 64: always 4
+    (F.BF16, 2, 8, F.TOPK_PER_HEAD, 100, 65),
 ])
-def test_select_workgroup_sizes_bit_exact(dtype, Hkv, Hq, mode, n_req):
+def test_select_workgroup_sizes_bit_exact(dtype, Hkv, Hq, mode, n_req, mb):
     """A workgroup has 16, 8 or 4 wavefronts by the rows of the launch (up to
-    256, 512, more on 256 CUs): 200, 400 and 600 rows of one context set, with
-    context lengths around a wavefront's and a workgroup's span of blocks."""
-    L, k, mb = 3, 12, 270
+    256, 512, more on 256 CUs), the longest context, the type and the mode: 200,
+    400 and 600 rows of one context set, with context lengths around a
+    wavefront's and a workgroup's span of blocks."""
+    L, k = 3, 12
     p = Pair(n_req, L, Hkv, Hq, k, 16, mb, dtype, host_blocks=1031)
     p.ex.summaries_build()
     rng = np.random.default_rng(dtype + 3)
-    ctx = rng.choice([0, 12, 13, 15, 16, 17, 63, 64, 65, 255, 256, 257, 270], n_req).astype(np.int32)
+    ctx = rng.choice([0, 12, 13, 15, 16, 17, 63, 64, 65, 255, 256, 257, 270, 511, 513, 600],
+                     n_req).clip(0, mb).astype(np.int32)
     q = rng.standard_normal((n_req, L, Hq, 128)).astype(np.float32)
     dq, dctx = torch.from_numpy(q).cuda(), torch.from_numpy(ctx).cuda()
     want = O.select_topk(p.g, q, ctx, mode)
@@ -99,6 +108,8 @@ def test_select_workgroup_sizes_bit_exact(dtype, Hkv, Hq, mode, n_req):
     (F.FP8, 1, 8, F.TOPK_PER_HEAD, 9),      # 9 rows, 6
     (F.F32, 2, 8, F.TOPK_PER_HEAD, 64),     # 128 rows, 2
     (F.F16, 2, 8, F.TOPK_LAYER_MAX, 13),    # 13 rows of all heads, 3
+    (F.F32, 2, 16, F.TOPK_LAYER_MAX, 13),   # 8 heads per kv head
+    (F.FP8, 2, 16, F.TOPK_LAYER_MAX, 13),
 ])
 def test_select_split_rows_bit_exact(dtype, Hkv, Hq, mode, n_req):
     """A launch of few rows shares each row's blocks between workgroups; the
