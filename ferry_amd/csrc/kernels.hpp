@@ -89,7 +89,8 @@ template <bool SERIAL>
 __global__ void k_lru_step(Geo g, const uint32_t* sel, uint32_t* slots_out, uint32_t* miss_count,
                            ferry_miss* misses, uint8_t* miss_flag, SetState st, Ring ring, int l0,
                            int nl, unsigned long long* sel_counts, int* err);
-// One workgroup per set, for sets of at least kLruGroupSel selections a step.
+// One workgroup per set, for sets of at least kLruGroupSel selections a step
+// (lru_grouped).
 constexpr int kLruGroupWaves = 4;
 constexpr int kLruGroupSel = 256;
 constexpr int kLruGroupLds = 256;  // its own LDS words beside the set's, at most

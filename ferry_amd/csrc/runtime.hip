@@ -1112,6 +1112,19 @@ int ferry_missq_drain(ferry_ctx* ctx, void* stream) {
 
 namespace {
 
+// A workgroup per set (k_lru_group): for sets of at least kLruGroupSel
+// selections, where a wavefront's share is one round of lanes; of fewer than
+// twice as many while the launch has up to four sets per CU, past which a
+// wavefront per set fills the GPU with fewer barriers.  us per launch, a
+// wavefront / a workgroup per set: 256 selections 64 sets 11.7 / 9.2, 512 sets
+// 12.3 / 10.2, 1024 sets 13.1 / 13.0, 2048 sets 15.8 / 21.3; 512 selections 64
+// sets 18.7 / 11.3, 1024 sets 23.5 / 16.7, 2048 sets 32.4 / 30.5; 1024 selections
+// 1024 sets 47.8 / 39.2.
+bool lru_grouped(const Geo& g, long nsets, int cus) {
+  return g.max_sel >= kLruGroupSel && (g.max_sel >= 2 * kLruGroupSel || nsets <= 4l * cus) &&
+         lru_stages_sel(g) && lru_lds_wave_words(g) * 4 + kLruGroupLds <= 65536;
+}
+
 int bookkeep_ring(ferry_ctx* ctx, int32_t l0, int32_t nl, const uint32_t* sel, uint32_t* slots,
                   uint32_t* miss_count, ferry_miss* misses, uint8_t* miss_flag, void* stream,
                   int which) {
@@ -1126,8 +1139,7 @@ int bookkeep_ring(ferry_ctx* ctx, int32_t l0, int32_t nl, const uint32_t* sel, u
     hipLaunchKernelGGL(k_lru_step<true>, grid, block, ctx->lru_lds, (hipStream_t)stream, g, sel, slots,
                        miss_count, misses, miss_flag, ctx->st, ctx->ring(which), l0, nl,
                        ctx->sel_counts, ctx->err);
-  else if (g.max_sel >= kLruGroupSel && lru_stages_sel(g) &&
-           lru_lds_wave_words(g) * 4 + kLruGroupLds <= 65536)
+  else if (lru_grouped(g, nsets, ctx->cus))
     hipLaunchKernelGGL(k_lru_group<kLruGroupWaves>, dim3((unsigned)nsets), dim3(64 * kLruGroupWaves),
                        lru_lds_wave_words(g) * 4, (hipStream_t)stream, g, sel, slots, miss_count, misses,
                        miss_flag, ctx->st, ctx->ring(which), l0, nl, ctx->sel_counts, ctx->err);

@@ -1,5 +1,5 @@
-"""Bookkeeping of sets with many selections a step (a workgroup per set from
-256 selections): misses, slots, flags and LRU state bit-exact against the
+"""Bookkeeping of sets with many selections a step (a workgroup per set from 256
+selections, in launches of many sets from 512): misses, slots, flags and LRU state bit-exact against the
 oracle at run lengths around a wavefront's share, and the same errors."""
 import numpy as np
 import pytest
@@ -16,6 +16,8 @@ pytestmark = pytest.mark.gpu
     (1, 255, 3, 300),    # the largest set of the one-wavefront kernel
     (1, 256, 3, 257),    # one wavefront's run each; almost every block evicted
     (1, 257, 2, 300),    # a run of one position
+    (1, 256, 257, 270),  # 1028 sets: past four per CU, a wavefront per set again (256 CUs)
+    (1, 512, 257, 520),  # ... and sets of 512 selections, which keep the workgroup
     (5, 57, 13, 320),    # 285 positions, the last group has 3 members
     (32, 40, 40, 1400),  # 1280 positions, the last group has 8 members
     (16, 64, 32, 1536),  # the shared-prefix shape
