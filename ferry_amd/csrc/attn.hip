@@ -114,7 +114,7 @@ __global__ __launch_bounds__(W * 64) void k_attn(Geo g, const float* __restrict_
   __shared__ int id_cnt[kMaxTopK / 64];
 
   // (request, layer in [l0, l0 + nl), kv head) of this workgroup
-  const int wrow = MODE == kSplitRow ? blockIdx.x / rs.parts : blockIdx.x;  // row of the launch
+  const uint32_t wrow = MODE == kSplitRow ? blockIdx.x / rs.parts : blockIdx.x;  // row of the launch
   const int part0 = MODE == kSplitRow ? blockIdx.x % rs.parts : 0;
   const int h = wrow % g.Hkv;
   const int rl = (wrow / (nl * g.Hkv)) * g.L + l0 + (wrow / g.Hkv) % nl;
@@ -135,7 +135,7 @@ __global__ __launch_bounds__(W * 64) void k_attn(Geo g, const float* __restrict_
   const int k = stage_row_ids<W>(slots + (size_t)row * g.k, g.k, ids, id_cnt);
 
   // one pass, or with kRowAlone one for each part
-  for (int part = part0; part < (MODE == kRowAlone ? rs.parts : part0 + 1); ++part) {
+  for (int part = part0;;) {
     // this wavefront takes blocks w0, w0 + WS, ... of the row
     const int WS = MODE == kWholeRow ? W : W * rs.parts;
     const int w0 = MODE == kWholeRow ? wave : part * W + wave;
@@ -304,6 +304,7 @@ __global__ __launch_bounds__(W * 64) void k_attn(Geo g, const float* __restrict_
       }
     }
     if constexpr (MODE == kRowAlone) __syncthreads();  // `red` is read, the part's state written
+    if (MODE != kRowAlone || ++part == rs.parts) break;
   }
   if constexpr (MODE != kWholeRow) {
     __shared__ uint32_t seen;

@@ -103,11 +103,12 @@ __device__ inline void wait_blocks(int later) {
 // same XCD (workgroups go round the 8 XCDs), close in time, so a block that
 // several of them read is found in that XCD's L2.
 struct GroupPart {
-  int set, part;
+  uint32_t set;
+  int part;
 };
 __device__ inline GroupPart group_part(uint32_t i, int parts) {
   const uint32_t r = i % (8u * (uint32_t)parts);
-  return {(int)(i / (8u * (uint32_t)parts) * 8u + r % 8u), (int)(r / 8u)};
+  return {i / (8u * (uint32_t)parts) * 8u + r % 8u, (int)(r / 8u)};
 }
 
 // Exclusive prefix sum of v over the workgroup's threads (thread order);
@@ -188,7 +189,7 @@ __global__ __launch_bounds__(W * 64) void k_attn_group(
   // `all` requests from o0, and the member rows it attends, `mem` from m0:
   // the set's, or those of this workgroup's part
   const GroupPart gp = SPLIT ? group_part(blockIdx.x, (g.group + mpw - 1) / mpw)
-                             : GroupPart{(int)blockIdx.x, 0};
+                             : GroupPart{blockIdx.x, 0};
   const int h = gp.set % g.Hkv;
   const int l = l0 + (gp.set / g.Hkv) % nl;
   const int o = gp.set / (nl * g.Hkv);

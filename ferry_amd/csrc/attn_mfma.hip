@@ -45,7 +45,7 @@ __global__ __launch_bounds__(W * 64) void k_attn_mfma(Geo g, const float* __rest
   __shared__ uint32_t ids[kMaxTopK];
   __shared__ int id_cnt[kMaxTopK / 64];
 
-  const int wrow = MODE == kSplitRow ? blockIdx.x / rs.parts : blockIdx.x;  // row of the launch
+  const uint32_t wrow = MODE == kSplitRow ? blockIdx.x / rs.parts : blockIdx.x;  // row of the launch
   const int part0 = MODE == kSplitRow ? blockIdx.x % rs.parts : 0;
   const int h = wrow % g.Hkv;
   const int rl = (wrow / (nl * g.Hkv)) * g.L + l0 + (wrow / g.Hkv) % nl;
@@ -64,7 +64,7 @@ __global__ __launch_bounds__(W * 64) void k_attn_mfma(Geo g, const float* __rest
   const int k = stage_row_ids<W>(slots + (size_t)row * g.k, g.k, ids, id_cnt);
 
   // one pass, or with kRowAlone one for each part
-  for (int part = part0; part < (MODE == kRowAlone ? rs.parts : part0 + 1); ++part) {
+  for (int part = part0;;) {
     // this wavefront takes blocks w0, w0 + WS, ... of the row
     const int WS = MODE == kWholeRow ? W : W * rs.parts;
     const int w0 = MODE == kWholeRow ? wave : part * W + wave;
@@ -197,6 +197,7 @@ __global__ __launch_bounds__(W * 64) void k_attn_mfma(Geo g, const float* __rest
         out[((size_t)rl * g.Hq + (size_t)h * G + hq) * D + d] = l > 0.0f ? o / l : 0.0f;
       }
     }
+    if (MODE != kRowAlone || ++part == rs.parts) break;
   }
   if constexpr (MODE != kWholeRow) {
     __shared__ uint32_t seen;

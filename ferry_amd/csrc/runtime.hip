@@ -530,11 +530,15 @@ int check_bufs(std::initializer_list<std::pair<const void*, const char*>> bufs) 
 // one on every CU, and between three where that is one but three put two on
 // most (rows in (CUs / 2, 2 CUs / 3]).  More, or more rows, only add to the
 // merge.  A part's wavefronts have two blocks each, and a row at most kMaxParts
-// parts, past which the merge takes what the shorter parts give.  us per launch, whole
-// rows / split, bf16, 4 query heads, k 128: 8 rows 31.2 / 10.9 (8 parts), 64 rows
+// parts, past which the merge takes what the shorter parts give.  A row of few
+// blocks is sooner done whole: parts begin at six blocks a wavefront, four for
+// fp32 (a block is twice as long), thirds at twelve.  us per launch, whole rows /
+// split, bf16, 4 query heads, k 128: 8 rows 31.2 / 10.9 (8 parts), 64 rows
 // 34.0 / 18.4 (4), 128 rows 40.8 / 28.2 (2), 160 rows 41.6 / 35.5 (3), 192 rows
-// 41.8 (44.1 in 2); fp32, 1 head, k 32: 8 rows 12.7 / 8.1 (4), 128 rows
-// 17.2 / 15.3 (2).
+// 41.8 (44.1 in 2); k 24: 8 rows 8.5 / 8.4, 64 rows 10.5 / 9.9; k 16: 8 rows
+// 7.1 / 8.1, 64 rows 9.0 / 9.4; k 32: 160 rows 13.7 / 14.6; fp32, 1 head, k 32:
+// 8 rows 12.7 / 8.1 (4), 128 rows 17.2 / 15.3 (2); k 16: 8 rows 7.3 / 7.2, 160 rows
+// 10.9 / 13.8; 8 heads, k 16: 8 rows 15.4 / 12.8.
 // The parts change the order of a row's sums, so they are for the kernels whose
 // sums and weights keep what 32-bit sums show (fp32 weights; two bf16 terms).
 // fp8 and grouped fp16 KV round each weight to fp16 against the running maximum
@@ -543,7 +547,8 @@ int check_bufs(std::initializer_list<std::pair<const void*, const char*>> bufs) 
 // parts, 12.4 whole).
 int row_parts(const AttnPlan& p, long rows, int k) {
   if (p.grouped || (p.mfma && p.dtype != FERRY_BF16)) return 1;
-  const long n = rows * 2 <= p.cus ? p.cus / rows : rows * 3 <= 2l * p.cus ? 3 : 1;
+  if (k < (p.dtype == FERRY_F32 ? 4 : 6) * p.waves) return 1;
+  const long n = rows * 2 <= p.cus ? p.cus / rows : rows * 3 <= 2l * p.cus && k >= 12 * p.waves ? 3 : 1;
   return (int)std::max<long>(1, std::min<long>(std::min<long>(n, kMaxParts), k / (2 * p.waves)));
 }
 
