@@ -1689,17 +1689,26 @@ uint64_t mass_ws_bytes(ferry_ctx* ctx, int nl, uint64_t wgs) {
 // two for fp8).  Fewer units leave slots idle and every unit's records to one
 // workgroup's loads in flight, so each unit is split: about two parts per slot
 // while a part has 256 blocks (the second hides the first's start), at least
-// one part per slot while a part has 32.  us per one-layer launch, 8192 / 512
-// blocks, whole and split by this rule: bf16 128 units 859 / 76 and 750 / 66, 32
-// units 827 / 67 and 214 / 36, 8 units 813 / 66 and 83 / 27; fp8 128 units
-// 814 / 67 and 438 / 48.  256 bf16 units in 2 parts each scored in no less time
-// than whole.  The lists are the same either way.
+// one part per slot while a part has 32.  The merge of a split launch takes 3 us
+// with 1 query head per kv head, 8 with 4 and 12 with 8, so contexts have to be
+// longer with more heads and with fewer idle CUs; with a unit on every CU only
+// fp8, whose units are bound by their arithmetic, gains.  us per one-layer
+// launch, whole / split: bf16, 4 heads, 8192 blocks: 8 units 813 / 83, 32 units
+// 827 / 214, 128 units 859 / 750; 64 units 140 blocks 30.9 / 29.1, 512 68 / 48; 128
+// units 140 blocks 33.9 / 36.0, 256 46.0 / 44.3, 512 76 / 66; 8 heads: 64 units 140
+// blocks 32.5 / 36.4, 256 43.4 / 39.2, 128 units 256 blocks 48.4 / 51.0, 512
+// 77.8 / 73.6; 256 units: fp8 1 head 512 blocks 72 / 64, 4 heads 1024 127 / 130, 2048
+// 234 / 233, 8192 849 / 814, 8 heads 2048 240 / 256, 4096 492 / 440; fp16 4 heads 512
+// 101 / 107, 8192 1362 / 1452.  The lists are the same either way.
 int mass_parts(ferry_ctx* ctx, int nl) {
   const Geo& g = ctx->g;
   const uint64_t units = (uint64_t)g.n_req * nl * g.Hkv, mb = (uint64_t)g.max_blocks;
   if (g.dtype == FERRY_F32) return 1;
-  const uint64_t slots = (uint64_t)mass_split_resident(ctx);
+  const uint64_t slots = (uint64_t)mass_split_resident(ctx), cus = (uint64_t)ctx->cus;
   if (2 * units > slots) return 1;
+  if (2 * units > cus && g.dtype != FERRY_FP8_E4M3) return 1;
+  const uint64_t least = 4 * units <= cus ? 32 : 2 * units <= cus ? 64 : 512;  // blocks per head of the group
+  if (mb < least * (uint64_t)(g.Hq / g.Hkv)) return 1;
   const uint64_t large = std::min((2 * slots + units - 1) / units, mb / 256);
   return (int)std::max<uint64_t>(1, std::max(large, std::min(slots / units, mb / 32)));
 }
@@ -1898,7 +1907,10 @@ int launch_select_mass(ferry_ctx* ctx, int32_t l0, int32_t nl, const float* q,
     mass = score;
   }
   const int rows = parts > 1 ? 1 : g.Hkv;  // mass rows of an item
-  if (items <= (unsigned)ctx->cus)
+  // 16 wavefronts shorten a long top k and lengthen a short one: 16 items
+  // of 140 blocks 33.9 -> 34.9 us a launch, of 300 49.8 -> 49.2, of 1200 133 -> 130;
+  // 64 items 67.3 -> 67.9, 119 -> 117, 407 -> 399
+  if (items <= (unsigned)ctx->cus && g.max_blocks > 256)
     hipLaunchKernelGGL((k_mass_topk<kMassTopkWideWaves>), dim3(items), dim3(64 * kMassTopkWideWaves), lds,
                        s, g, ctx_blocks, mass, rows, sel, l0, nl, g.max_blocks);
   else
