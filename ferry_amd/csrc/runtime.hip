@@ -1296,15 +1296,8 @@ int ferry_decode_step(ferry_ctx* ctx, const uint32_t* sel, const float* q, uint3
   // (attention time) / (fetch time) of a layer at typical MI355X rates
   // (6.5 TB/s HBM reads, 55 GB/s host link; 2 for the slowdown of sharing the
   // GPU with the fetch).  At the 7B shape r = 0.08: the last range is one layer.
-  // A last range that still has layers to hide gives its last one a range of
-  // its own (two streams): the others attend while that one is fetched, for one
-  // more bookkeeping, drain and hand-over between the streams, some 30 us (the
-  // shared-prefix step of 8 layers: 997 us in two ranges, 978 in three).
-  hipStream_t ms = (hipStream_t)stream, ss = (hipStream_t)side_stream;
-  const bool overlap = ss != nullptr && ss != ms;
   std::vector<int> first(chunks + 1, L);
   {
-    bool cut_tail = false;
     int tail = (L + chunks - 1) / chunks;
     if (adaptive && chunks >= 2 && last > 0) {
       const Geo& g = ctx->g;
@@ -1317,18 +1310,15 @@ int ferry_decode_step(ferry_ctx* ctx, const uint32_t* sel, const float* q, uint3
       const int rest = (L - 1 + chunks - 2) / (chunks - 1);  // layers of the other ranges
       const double want = std::ceil(2.0 * attn_s / fetch_s * rest);
       if (want < (double)tail) tail = std::max(1, (int)want);
-      cut_tail = overlap && attn_s / L * (tail - 1) > 30e-6;
     }
     // the other chunks - 1 ranges split L - tail layers as evenly as possible
     const int head = L - tail, nh = chunks - 1;
     for (int c = 0; c < nh; ++c) first[c] = c * head / nh;
     first[nh] = head;
     first[chunks] = L;
-    if (cut_tail) {
-      first.insert(first.end() - 1, L - 1);
-      ++chunks;
-    }
   }
+  hipStream_t ms = (hipStream_t)stream, ss = (hipStream_t)side_stream;
+  const bool overlap = ss != nullptr && ss != ms;
   HIPC(hipSetDevice(ctx->device));
   if (!sel || !slots || !miss_count || !misses) return fail(FERRY_EINVAL, "null buffer");
   if (!overlap) {  // one stream: bookkeeping, fetch and attention range by range
