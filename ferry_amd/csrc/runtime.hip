@@ -170,6 +170,7 @@ struct ferry_ctx {
   uint32_t* trim_gen = nullptr;    // [n_owners] last ferry_members_leave that shrank the owner
   float* split_state = nullptr;    // [kSplitStreams][2 CUs][G][kPartFloats] softmax states of split rows
   uint32_t* split_count = nullptr;  // [kSplitStreams][CUs] finished parts of each row, 0 between launches
+  bool split = true;               // several workgroups may share a row or unit (FERRY_SPLIT=0, or no memory: none do)
   std::mutex split_mu;             // guards the slots past the first, from choice to record
   SplitSlot split_slot[kSplitStreams];
   uint32_t member_calls = 0;       // ferry_members_leave calls so far (trim generations)
@@ -553,7 +554,7 @@ int row_parts(const AttnPlan& p, long rows, int k) {
 }
 
 // The split state of a launch on stream `s`: `slot`, or -1 where there is none
-// (a workgroup then takes a whole row): for a stream being captured (a graph may
+// (a workgroup then takes a whole row): without memory for it, for a stream being captured (a graph may
 // be replayed on any stream), for the per-thread default stream (one handle, a
 // stream per thread), and while other streams use all slots.  The default
 // stream has slot 0: it is never destroyed and runs its launches in order.  Any
@@ -566,7 +567,7 @@ int row_parts(const AttnPlan& p, long rows, int k) {
 class SplitLease {
  public:
   SplitLease(ferry_ctx* ctx, hipStream_t s) : ctx_(ctx), s_(s) {
-    if (s == hipStreamPerThread) return;
+    if (!ctx->split || s == hipStreamPerThread) return;
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(s, &cap) != hipSuccess) {
       (void)hipGetLastError();
@@ -740,6 +741,7 @@ int ferry_ctx_create(const ferry_config* cfg, int device, ferry_ctx** out) {
   if (const char* e = std::getenv("FERRY_THIEF_WAVES")) c->thief_waves = std::max(1, std::atoi(e));
   if (const char* e = std::getenv("FERRY_STEAL_INFLIGHT")) c->steal_inflight = std::max(1, std::atoi(e));
   if (const char* e = std::getenv("FERRY_ATTN_GROUPED")) c->attn_grouped = std::atoi(e) != 0;
+  if (const char* e = std::getenv("FERRY_SPLIT")) c->split = std::atoi(e) != 0;
   if (const char* e = std::getenv("FERRY_ATTN_LOADS"))
     c->attn_loads = std::string(e) == "nt" ? 1 : (std::string(e) == "temporal" ? 2 : 0);
   c->device = device;
@@ -853,8 +855,11 @@ int ferry_ctx_create(const ferry_config* cfg, int device, ferry_ctx** out) {
   TRY(dalloc(&c->step_acc, 3));
   TRY(dalloc(&c->done, 1));
   TRY(dalloc(&c->err, 1));
-  TRY(dalloc(&c->split_state, kSplitStreams * split_state_floats(c)));
-  TRY(dalloc(&c->split_count, (size_t)kSplitStreams * c->cus));
+  if (c->split && (hipMalloc(&c->split_state, kSplitStreams * split_state_floats(c) * sizeof(float)) != hipSuccess ||
+                   hipMalloc(&c->split_count, (size_t)kSplitStreams * c->cus * sizeof(uint32_t)) != hipSuccess)) {
+    (void)hipGetLastError();
+    c->split = false;  // rows then have one workgroup each
+  }
 #define HIPT(x)                                                                        \
   do {                                                                                 \
     hipError_t e_ = (x);                                                               \
@@ -880,7 +885,7 @@ int ferry_ctx_create(const ferry_config* cfg, int device, ferry_ctx** out) {
   HIPT(hipHostGetDevicePointer((void**)&c->pend_dev, c->pend_host, 0));
   HIPT(hipMemset(c->done, 0, 4));
   HIPT(hipMemset(c->err, 0, 4));
-  HIPT(hipMemset(c->split_count, 0, (size_t)kSplitStreams * c->cus * 4));
+  if (c->split) HIPT(hipMemset(c->split_count, 0, (size_t)kSplitStreams * c->cus * 4));
   HIPT(hipMemset(c->pool, 0, nslots * g.bb));
   // pinned host tier, mapped into the device address space
   const size_t hbytes = (size_t)g.host_blocks * g.bb;
@@ -1394,7 +1399,7 @@ int ferry_summaries_build(ferry_ctx* ctx, uint64_t n_records, void* stream) {
       return rc;
     ctx->sum_blocks = S;
   }
-  if (!ctx->sel_keys && g.group == 1 && (uint64_t)g.max_blocks * 4 <= 65536) {  // what select_topk takes
+  if (ctx->split && !ctx->sel_keys && g.group == 1 && (uint64_t)g.max_blocks * 4 <= 65536) {  // what select_topk takes
     const uint64_t words = kSplitStreams * select_split_rows(ctx) * (uint64_t)g.max_blocks;
     if (hipMalloc(&ctx->sel_keys, words * 4) != hipSuccess) {  // selections then run unsplit
       (void)hipGetLastError();
@@ -1693,7 +1698,7 @@ uint64_t mass_ws_bytes(ferry_ctx* ctx, int nl, uint64_t wgs) {
 int mass_parts(ferry_ctx* ctx, int nl) {
   const Geo& g = ctx->g;
   const uint64_t units = (uint64_t)g.n_req * nl * g.Hkv, mb = (uint64_t)g.max_blocks;
-  if (g.dtype == FERRY_F32) return 1;
+  if (g.dtype == FERRY_F32 || !ctx->split) return 1;
   const uint64_t slots = (uint64_t)mass_split_resident(ctx), cus = (uint64_t)ctx->cus;
   if (2 * units > slots) return 1;
   if (2 * units > cus && g.dtype != FERRY_FP8_E4M3) return 1;

@@ -92,15 +92,16 @@ def _check_twins(gp, rp, sel, dtype, Hq, n_req, seed):
     assert np.array_equal(got, _decode(gp, q, gp.bufs["slots"]))
 
 
-@pytest.mark.parametrize("L", [10, 20, 40])
+@pytest.mark.parametrize("L", [10, 12, 20, 40])
 @pytest.mark.parametrize("dtype,Hkv,Hq,group,n_req", [
     (F.FP8, 4, 16, 16, 32),  # G 4, 4 tiles
     (F.BF16, 4, 16, 12, 23),  # G 4, 3 tiles; the last group has 11 members
 ])
 def test_group_kernel_member_splits(dtype, Hkv, Hq, group, n_req, L):
-    """A launch of few group sets splits a set's query tiles between workgroups:
-    80 sets run two tiles per workgroup (the CASES above one), 160 whole sets
-    with eight wavefronts, 320 whole sets with four."""
+    """A launch of few group sets splits a set's query tiles between workgroups
+    (on 256 CUs): 80 sets of 4 tiles run two per workgroup, of 3 tiles one (the
+    CASES above one); 96 sets two, the last workgroup of 3 tiles one; 160 run
+    whole sets with eight wavefronts, 320 whole sets with four."""
     sets = 2 * L * Hkv
     gp, rp, sel = _twins(dtype, Hkv, Hq, group, n_req, L=L, steps=1, waves=8 if sets <= 256 else 4)
     _check_twins(gp, rp, sel, dtype, Hq, n_req, seed=L)

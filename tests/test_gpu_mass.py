@@ -110,7 +110,9 @@ def test_ktiles_bit_exact(dtype):
     (F.F32, 1, 2),    # GQA-2, f32
     (F.BF16, 1, 8),   # GQA-8
 ])
-def test_select_mass_parity(dtype, Hkv, Hq):
+@pytest.mark.parametrize("split", [1, 0])  # units shared between workgroups, or whole
+def test_select_mass_parity(dtype, Hkv, Hq, split, monkeypatch):
+    monkeypatch.setenv("FERRY_SPLIT", str(split))
     n_req, L, k, mb = 6, 2, 16, 300
     p = Pair(n_req, L, Hkv, Hq, k, 64, mb, dtype, host_blocks=4099)
     p.ex.ktiles_build()
@@ -126,11 +128,14 @@ def test_select_mass_parity(dtype, Hkv, Hq):
     assert p.ex.stats()["device_error"] == 0
 
 
-@pytest.mark.parametrize("dtype,Hkv,Hq", [(F.F16, 2, 2), (F.BF16, 2, 8)])
-def test_select_mass_hbm_workspace_parity(dtype, Hkv, Hq, monkeypatch):
+@pytest.mark.parametrize("dtype,Hkv,Hq", [(F.F16, 2, 2), (F.BF16, 2, 8), (F.F16, 1, 8)])
+@pytest.mark.parametrize("split", [1, 0])
+def test_select_mass_hbm_workspace_parity(dtype, Hkv, Hq, split, monkeypatch):
     # 16-bit K keeps each block's log-sum in LDS; FERRY_MASS_WS=hbm (read when the
     # K table is built) keeps the (max, sum) pairs in the context's HBM workspace
+    # and forms the masses from them, in whole units and in split ones
     monkeypatch.setenv("FERRY_MASS_WS", "hbm")
+    monkeypatch.setenv("FERRY_SPLIT", str(split))
     n_req, L, k, mb = 6, 2, 16, 300
     print(f"[mass] HBM workspace dtype={dtype} Hkv={Hkv} Hq={Hq}", flush=True)
     p = Pair(n_req, L, Hkv, Hq, k, 64, mb, dtype, host_blocks=4099)
@@ -145,7 +150,8 @@ def test_select_mass_hbm_workspace_parity(dtype, Hkv, Hq, monkeypatch):
 
 
 @pytest.mark.parametrize("dtype,Hkv,Hq,ws", [
-    (F.BF16, 8, 16, ""), (F.F16, 8, 8, ""), (F.FP8, 8, 16, ""), (F.BF16, 8, 8, "hbm")])
+    (F.BF16, 8, 16, ""), (F.F16, 8, 8, ""), (F.FP8, 8, 16, ""), (F.BF16, 8, 8, "hbm"),
+    (F.BF16, 8, 64, ""), (F.FP8, 8, 32, "")])
 def test_select_mass_split_and_whole_units(dtype, Hkv, Hq, ws, monkeypatch):
     """A launch of few (request, layer, kv head) units splits each one's blocks
     between workgroups, a launch of many gives a unit to one workgroup: 64 and

@@ -32,8 +32,10 @@ def _rel(a, b):
     (F.F16, 2, 2, 43, 24),     # 86 rows, 2 (vector ALUs)
     (F.BF16, 2, 4, 64, 40),    # 128 rows, 2
     (F.F16, 2, 4, 64, 40),     # 128 rows, 1 (fp16 weights)
-    (F.F32, 2, 4, 65, 25),     # 130 rows, 3
-    (F.BF16, 2, 16, 85, 24),   # 170 rows, 3
+    (F.F32, 2, 4, 65, 50),     # 130 rows, 3
+    (F.BF16, 2, 16, 85, 49),   # 170 rows, 3
+    (F.F32, 2, 4, 65, 25),     # 130 rows, 1: thirds begin at 48 blocks
+    (F.BF16, 2, 16, 8, 23),    # 16 rows, 1: parts begin at 24 blocks
     (F.BF16, 3, 6, 57, 30),    # 171 rows, 1
     (F.FP8, 3, 3, 57, 30),
 ])
@@ -63,6 +65,31 @@ def test_row_split_parity(dtype, Hkv, Hq, n_req, k):
         assert _rel(got[~none], ref[~none]) < TOL[dtype]
     assert torch.equal(out, again)  # parts are merged in part order
     assert p.ex.stats()["device_error"] == 0
+
+
+@pytest.mark.parametrize("dtype,Hkv,Hq,k", [(F.F32, 2, 16, 64), (F.F16, 2, 2, 48), (F.BF16, 2, 8, 67),
+                                             (F.BF16, 1, 8, 33)])
+def test_rows_without_split_memory_give_the_same_bits(dtype, Hkv, Hq, k, monkeypatch):
+    """A context without memory for split rows attends them in one workgroup and
+    selects from whole rows."""
+    n_req = 9
+    mb, sels = _zipf_stream(n_req, 1, Hkv, k, 800, 900, 1, seed=k)
+    q = torch.randn((n_req, 1, Hq, 128), device="cuda")
+    ctx = torch.full((n_req,), mb, dtype=torch.int32, device="cuda")
+    outs, picks = [], []
+    for split in (1, 0):
+        monkeypatch.setenv("FERRY_SPLIT", str(split))
+        p = Pair(n_req, 1, Hkv, Hq, k, 2 * k, mb, dtype)
+        p.step(sels[0])
+        p.ex.summaries_build()
+        outs.append(torch.full_like(q, 7.0))
+        picks.append(torch.full((n_req, 1, Hkv, k), -7, dtype=torch.int32, device="cuda"))
+        p.ex.sparse_decode(q, p.bufs["slots"], outs[-1])
+        p.ex.select_topk(q, ctx, picks[-1])
+        torch.cuda.synchronize()
+        assert p.ex.stats()["device_error"] == 0
+    assert torch.equal(outs[0], outs[1])
+    assert torch.equal(picks[0], picks[1])
 
 
 class _Pool:

@@ -41,11 +41,14 @@ def _both(ex, q, ctx, shape):
 
 @pytest.mark.parametrize("dtype,Hkv,Hq,ws", [(F.BF16, 4, 16, ""), (F.F16, 2, 4, ""), (F.FP8, 2, 8, ""),
                                              (F.BF16, 2, 8, "hbm"), (F.F32, 2, 4, "")])
-def test_noalloc_select_mass_equals_select_mass(dtype, Hkv, Hq, ws, monkeypatch):
-    # 16-bit K keeps the blocks' log-sums in LDS (or, with FERRY_MASS_WS=hbm,
+@pytest.mark.parametrize("split", [1, 0])
+def test_noalloc_select_mass_equals_select_mass(dtype, Hkv, Hq, ws, split, monkeypatch):
+    # These launches have few units, which several workgroups share; without
+    # that (FERRY_SPLIT=0) 16-bit K keeps the blocks' log-sums in LDS (or, with FERRY_MASS_WS=hbm,
     # their max and sum in workspace slices, as fp8 K does); fp32 K runs the
     # one-launch kernel with slices.  The context reads the variable when it
     # first plans a mass selection.
+    monkeypatch.setenv("FERRY_SPLIT", str(split))
     if ws:
         monkeypatch.setenv("FERRY_MASS_WS", ws)
     else:
