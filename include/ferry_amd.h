@@ -356,8 +356,8 @@ int ferry_decode_chunks(const ferry_ctx* ctx, uint64_t pending_blocks, int32_t* 
  * (device, context length of each request in blocks, <= max_blocks), sel
  * [B][L][Hkv][k] u32 out (device) -- the input of ferry_fetch_step.  A launch
  * of few rows shares each row between workgroups, which meet in memory that
- * ferry_summaries_build allocates for the stream (as ferry_sparse_decode_layers
- * does).  Needs group == 1 and (query heads per row * D + max_blocks) * 4 <= 64 KiB. */
+ * ferry_summaries_build allocates and streams use as in
+ * ferry_sparse_decode_layers; the selection is the same without.  Needs group == 1 and (query heads per row * D + max_blocks) * 4 <= 64 KiB. */
 #define FERRY_TOPK_PER_HEAD 0
 #define FERRY_TOPK_LAYER_MAX 1
 int ferry_summaries_build(ferry_ctx* ctx, uint64_t n_records, void* stream);

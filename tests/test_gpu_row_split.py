@@ -67,11 +67,13 @@ def test_row_split_parity(dtype, Hkv, Hq, n_req, k):
     assert p.ex.stats()["device_error"] == 0
 
 
-@pytest.mark.parametrize("dtype,Hkv,Hq,k", [(F.F32, 2, 16, 64), (F.F16, 2, 2, 48), (F.BF16, 2, 8, 67),
-                                             (F.BF16, 1, 8, 33)])
-def test_rows_without_split_memory_give_the_same_bits(dtype, Hkv, Hq, k, monkeypatch):
-    """A context without memory for split rows attends them in one workgroup and
-    selects from whole rows."""
+@pytest.mark.parametrize("waves", [4, 8])
+@pytest.mark.parametrize("dtype,Hkv,Hq,k", [(F.F32, 2, 16, 160), (F.F16, 2, 2, 48), (F.BF16, 2, 8, 67),
+                                             (F.BF16, 1, 8, 160)])
+def test_rows_without_split_memory_give_the_same_bits(dtype, Hkv, Hq, k, waves, monkeypatch):
+    """A context without memory for split rows attends them in one workgroup (the
+    states of up to 8 parts of 8 heads in LDS) and selects from whole rows."""
+    monkeypatch.setenv("FERRY_ATTN_WAVES", str(waves))
     n_req = 9
     mb, sels = _zipf_stream(n_req, 1, Hkv, k, 800, 900, 1, seed=k)
     q = torch.randn((n_req, 1, Hq, 128), device="cuda")
