@@ -399,7 +399,7 @@ __global__ __launch_bounds__(W * 64) void k_select_topk(Geo g, const float* __re
   float* qs = reinterpret_cast<float*>(lds);
   uint32_t* keys = lds + Gq * D;
 
-  const uint32_t wrow = SPLIT ? blockIdx.x / parts : blockIdx.x;  // row of the launch
+  const int wrow = SPLIT ? blockIdx.x / parts : blockIdx.x;  // row of the launch
   const int part = SPLIT ? blockIdx.x % parts : 0;
   const int hrow = LAYER ? 0 : wrow % g.Hkv;
   const int rl_idx = LAYER ? wrow : wrow / g.Hkv;  // (request, layer in range)
