@@ -540,8 +540,10 @@ int check_bufs(std::initializer_list<std::pair<const void*, const char*>> bufs) 
 // 7.1 / 8.1, 64 rows 9.0 / 9.4; k 32: 160 rows 13.7 / 14.6; fp32, 1 head, k 32:
 // 8 rows 12.7 / 8.1 (4), 128 rows 17.2 / 15.3 (2); k 16: 8 rows 7.3 / 7.2, 160 rows
 // 10.9 / 13.8; 8 heads, k 16: 8 rows 15.4 / 12.8.
-// The parts change the order of a row's sums, so they are for the kernels whose
-// sums and weights keep what 32-bit sums show (fp32 weights; two bf16 terms).
+// The parts change the order of a row's sums and the running maxima that its
+// weights are held against, so they are for the kernels with fp32 weights
+// (outputs move by 2e-7) and with weights of two bf16 terms (by 8e-6, less than
+// the 1e-5 they are off the 64-bit result).
 // fp8 and grouped fp16 KV round each weight to fp16 against the running maximum
 // of the wavefront, which other parts would change: their outputs would move by
 // 3e-4 with the number of rows (8 rows of 64 fp8 blocks, 4 heads: 8.0 us in

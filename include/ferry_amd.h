@@ -282,7 +282,8 @@ int ferry_attn_kernel(const ferry_ctx* ctx, int32_t* kind, int32_t* waves);
  * kv head) rows of fp32, bf16 or ungrouped fp16 KV attends each row in parts,
  * whose number follows from the rows of the launch, k and the GPU's CUs: such a
  * row's sums run in another order than in a launch of many rows and differ from
- * it in their last bits.  Several workgroups share a row's parts; they meet in
+ * it in their last bits (2e-7 relative; 8e-6 for grouped bf16, which is that far
+ * from the exact result).  Several workgroups share a row's parts; they meet in
  * memory that the context keeps for the default stream and for three created
  * streams at a time (a stream that comes later takes it over once the launches
  * of another are done).  With more in use, and while a stream is being captured,
