@@ -657,9 +657,10 @@ int select_parts(const ferry_ctx* ctx, unsigned rows, int heads) {
 
 // Attention of layers [l0, l0 + nl).  attn_blocks (decode steps only): the
 // prefix-group kernel adds the distinct blocks it reads there, which the next
-// step's layer chunking takes as the attention's bytes.
+// step's layer chunking takes as the attention's bytes.  whole_rows: for layer
+// ranges that follow from timing, which rows in parts would show in their bits.
 int decode_layers(ferry_ctx* ctx, int32_t l0, int32_t nl, const float* q, const uint32_t* slots,
-                  float* out, void* stream, unsigned long long* attn_blocks) {
+                  float* out, void* stream, unsigned long long* attn_blocks, bool whole_rows) {
   if (int rc = check_bufs({{q, "q"}, {slots, "slots"}, {out, "out"}})) return rc;
   const Geo& g = ctx->g;
   if (l0 < 0 || nl < 1 || l0 + nl > g.L) return fail(FERRY_EINVAL, "bad layer range");
@@ -669,7 +670,7 @@ int decode_layers(ferry_ctx* ctx, int32_t l0, int32_t nl, const float* q, const 
   AttnArgs a{g, q, slots, ctx->pool, ctx->pool_scales, out, qscale, l0, nl, ctx->err,
              attn_blocks, RowSplit{nullptr, nullptr, 1}};
   const AttnPlan p = attn_plan(ctx);
-  a.rs.parts = row_parts(p, (long)grid.x, g.k);
+  a.rs.parts = whole_rows ? 1 : row_parts(p, (long)grid.x, g.k);
   std::optional<SplitLease> lease;
   if (a.rs.parts > 1) {
     lease.emplace(ctx, (hipStream_t)stream);
@@ -1226,7 +1227,7 @@ int ferry_fetch_step(ferry_ctx* ctx, const uint32_t* sel, uint32_t* slots, uint3
 int ferry_sparse_decode_layers(ferry_ctx* ctx, int32_t l0, int32_t nl, const float* q,
                                const uint32_t* slots, float* out, void* stream) {
   if (int rc = check_ctx(ctx)) return rc;
-  return decode_layers(ctx, l0, nl, q, slots, out, stream, nullptr);
+  return decode_layers(ctx, l0, nl, q, slots, out, stream, nullptr, false);
 }
 
 int ferry_attn_kernel(const ferry_ctx* ctx, int32_t* kind, int32_t* waves) {
@@ -1296,6 +1297,9 @@ int ferry_decode_step(ferry_ctx* ctx, const uint32_t* sel, const float* q, uint3
     if (int rc = ferry_decode_chunks(ctx, last, &chunks)) return rc;
   }
   chunks = std::min(chunks, L);
+  // the adaptive ranges follow from a step that the GPU had closed by now, so
+  // the same step may run in other ranges when it is repeated
+  const bool whole_rows = adaptive && L > 1;
   // Layer ranges: `chunks` even ranges, except that the adaptive count also
   // shortens the last one.  Its attention is the one the fetch cannot hide;
   // the range before it attends while the last range is fetched, which takes
@@ -1334,7 +1338,7 @@ int ferry_decode_step(ferry_ctx* ctx, const uint32_t* sel, const float* q, uint3
       if (nl <= 0) continue;
       int rc = bookkeep_ring(ctx, l0, nl, sel, slots, miss_count, misses, nullptr, ms, 0);
       if (!rc) rc = drain_ring(ctx, ms, 0);
-      if (!rc) rc = decode_layers(ctx, l0, nl, q, slots, out, ms, ctx->step_acc + 1);
+      if (!rc) rc = decode_layers(ctx, l0, nl, q, slots, out, ms, ctx->step_acc + 1, whole_rows);
       if (rc) return rc;
     }
   } else {
@@ -1370,7 +1374,7 @@ int ferry_decode_step(ferry_ctx* ctx, const uint32_t* sel, const float* q, uint3
       if (i + 2 < n)  // ring i mod 2 is drained
         if (int rc = book_fetch(i + 2)) return rc;
       if (int rc = decode_layers(ctx, first[c], first[c + 1] - first[c], q, slots, out, ms,
-                                 ctx->step_acc + 1))
+                                 ctx->step_acc + 1, whole_rows))
         return rc;
     }
   }

@@ -213,6 +213,30 @@ def test_row_split_streams_and_graphs():
     assert p.ex.stats()["device_error"] == 0
 
 
+@pytest.mark.parametrize("dtype,Hq", [(F.F32, 2), (F.BF16, 8), (F.FP8, 8)])
+def test_adaptive_steps_do_not_depend_on_their_ranges(dtype, Hq):
+    """The same steps in one layer range and in eight: the same bits, though a
+    range of few rows is a launch of few rows."""
+    n_req, L, Hkv, k = 4, 8, 2, 48
+    mb, sels = _zipf_stream(n_req, L, Hkv, k, 200, 300, 4, seed=9)
+    pairs = [Pair(n_req, L, Hkv, Hq, k, 2 * k, mb, dtype) for _ in range(2)]
+    pairs[0].ex.set_batch_policy(512.0, 512.0, 1.0)
+    pairs[1].ex.set_batch_policy(1e-3, 1e-3, 1.0)
+    assert pairs[0].ex.decode_chunks(100) == 1 and pairs[1].ex.decode_chunks(100) == L
+    side = torch.cuda.Stream()
+    for sel in sels:
+        ds = torch.from_numpy(np.array(sel, np.uint32).view(np.int32)).cuda().view(n_req, L, Hkv, k)
+        q = torch.randn((n_req, L, Hq, 128), device="cuda")
+        outs = []
+        for p in pairs:
+            out = torch.full_like(q, 7.0)
+            p.ex.decode_step(ds, q, p.bufs, out, side_stream=side)
+            torch.cuda.synchronize()  # the next step knows what this one fetched
+            assert p.ex.stats()["device_error"] == 0
+            outs.append(out)
+        assert torch.equal(outs[0], outs[1])
+
+
 class _Streams:
     """Streams created and destroyed through the HIP runtime (torch keeps its own)."""
 
